@@ -224,11 +224,12 @@ int hmc_ray_weight_factors(hmc_ctx *ctx, int64_t n, const float *energy, const f
  * reference counterpart: the measurement hook for the per-kernel roofline). */
 int hmc_set_profiling(hmc_ctx *ctx, int enabled);
 /* Launch shape of the transport rounds: lanes per CU of each round's grid (multiple
- * of 256 in [256, 8192]; default 2048), queue indices a wave claims at a time and
- * output slots it reserves at a time (each a multiple of 64 in [64, 1024]; default
- * 64), and whether each group of four rounds is replayed from a captured HIP graph
- * (default 1; profiled transports launch one by one, so that every kernel is
- * timed). None of them changes a result. No reference counterpart beyond the
+ * of 256 in [256, 8192]), queue indices a wave claims at a time and output slots it
+ * reserves at a time (each a multiple of 64 in [64, 1024]), and whether each group of
+ * four rounds is replayed from a captured HIP graph (default 1; profiled transports
+ * launch one by one, so that every kernel is timed). A context on which this was never
+ * called sizes the first three itself, each round by its queue's length. None of them
+ * changes a result. No reference counterpart beyond the
  * chunk_size / queue_factor knobs of WarpEngine (engine.py:369-407): these are the
  * autotuner's knobs. */
 int hmc_set_launch(hmc_ctx *ctx, int round_lanes_per_cu, int refill_block, int push_chunk,

@@ -59,7 +59,7 @@ struct Queue {
   Particle* data;
   unsigned int* count;
   unsigned int capacity;
-  unsigned int push_chunk = 64;  // slots a wave reserves per atomic (multiple of 64)
+  unsigned int push_chunk = 64;  // slots a wave reserves per atomic (multiple of 64; 0: sized_push_chunk)
   int lds = -1;                  // which of the wave's two output-chunk states (LDS) is this queue's
 };
 
@@ -106,7 +106,7 @@ __device__ inline long long wave_sum(long long v) {
 }
 
 // Queue indices handed to the idle lanes of a wave, in blocks of R (the refill block,
-// a multiple of 64 set per transport call) given to the idle lanes in lane order. A
+// a multiple of 64) given to the idle lanes in lane order. A
 // wave's first block is its own by position (wave w of the grid takes [R w, R w + R)),
 // with no atomic; later blocks come from one atomic per block on the queue head,
 // offset past those static blocks. So the single
@@ -114,21 +114,41 @@ __device__ inline long long wave_sum(long long v) {
 // starts beyond an exhausted queue exits without touching it: a round can launch at
 // full width whatever its queue holds. (Reading the head before claiming, instead,
 // queues that read behind the head's atomics in L2 and costs far more than it saves.)
+// R is the caller's (hmc_set_launch), or sized by what the queue still holds: a quarter
+// of a wave's even share at first, then half of an even share of the rest, in
+// [64, 512]. Atomics on the one head serialise at about 5 ns each, so a long queue wants
+// long blocks (1e7 photons: 3.1 ms for the first photon round at R = 64, 1.1 ms at 256);
+// a short queue, or the end of a long one, wants short blocks that spread over the waves.
 // Called by every lane still in the round loop, at the loop head (converged); the
 // pool state is therefore identical in all of them. Which lane transports which
 // particle does not change any result: each particle carries its own random stream
 // and the tallies are integer sums.
 struct RefillPool {
   unsigned int next, end;
-  unsigned int block;     // R
+  unsigned int block;     // R of the next claim
   unsigned int n_static;  // indices below this are the waves' static first blocks
+  unsigned int n_in;      // queue length (0: R is the caller's and stays)
   // Every wave of the grid owns one static block.
-  __device__ explicit RefillPool(unsigned int r)
-      : next((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * r),
-        end((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * r + r),
-        block(r),
-        n_static(gridDim.x * (blockDim.x >> 6) * r) {}
+  __device__ RefillPool(unsigned int r, unsigned int queue_length)
+      : block(r ? r : sized(queue_length, 4u)), n_in(r ? 0u : queue_length) {
+    const unsigned int wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    next = wave * block;
+    end = next + block;
+    n_static = gridDim.x * (blockDim.x >> 6) * block;
+  }
+  __device__ static unsigned int sized(unsigned int left, unsigned int parts) {
+    return min(max((left / (gridDim.x * (blockDim.x >> 6) * parts)) & ~63u, 64u), 512u);
+  }
 };
+
+// Output slots a wave reserves per atomic (chunk_reserve) where the caller set none: 256
+// for a round long enough that each wave fills several such chunks and whose queues
+// hold 16 times what the unfilled tails can take, else 64, so that the padding of a
+// short round or a tight queue stays small.
+__device__ inline unsigned int sized_push_chunk(unsigned int n_in, unsigned int capacity) {
+  const unsigned int slots = gridDim.x * (blockDim.x >> 6) * 256u;
+  return n_in >= slots && capacity / 16u >= slots ? 256u : 64u;
+}
 
 __device__ inline unsigned int refill_index(RefillPool& pool, unsigned int* head, bool idle) {
   const unsigned long long mask = __ballot(idle ? 1 : 0);
@@ -151,6 +171,7 @@ __device__ inline unsigned int refill_index(RefillPool& pool, unsigned int* head
     idx = rank < avail ? pool.next + rank : base + (rank - avail);
     pool.next = base + (want - avail);
     pool.end = base + pool.block;
+    if (pool.n_in) pool.block = RefillPool::sized(pool.n_in - min(base, pool.n_in), 2u);
   }
   return idx;
 }
@@ -192,7 +213,7 @@ struct TransportParams {
   float pcut, ecut, step_fraction, resolution;
   float log_pcut;  // logf(pcut), for the bremsstrahlung spectrum
   int transport_electrons, msc_gs, dose_to_water, max_steps;
-  unsigned int refill_block;  // queue indices a wave claims at a time (multiple of 64)
+  unsigned int refill_block;  // queue indices a wave claims at a time (multiple of 64; 0: by the queue's length)
 };
 
 // Per-lane books kept in registers and flushed once per lane at the end of a round;
@@ -489,7 +510,8 @@ k_photon_round(TransportParams P, Queue qin,
   if (__lane_id() < 2) g_books[(6 + __lane_id()) * 4 + wave_in_block] = 0;
   qe.lds = 0;
   qp.lds = 1;
-  RefillPool pool(P.refill_block);
+  if (qe.push_chunk == 0u) qe.push_chunk = qp.push_chunk = sized_push_chunk(n_in, qe.capacity);
+  RefillPool pool(P.refill_block, n_in);
   while (true) {
     const unsigned int i = refill_index(pool, head, !active);
     if (!active) {
@@ -659,7 +681,8 @@ k_electron_round(TransportParams P, Queue qin,
   if (__lane_id() < 2) g_books[(6 + __lane_id()) * 4 + wave_in_block] = 0;
   qp.lds = 0;
   qe.lds = 1;
-  RefillPool pool(P.refill_block);
+  if (qe.push_chunk == 0u) qe.push_chunk = qp.push_chunk = sized_push_chunk(n_in, qe.capacity);
+  RefillPool pool(P.refill_block, n_in);
   while (true) {
     // Idle lanes take new particles together, once kRefillIdleLanes of the wave's
     // looping lanes are idle (or all of them): the refill block then runs for more
@@ -1507,10 +1530,10 @@ struct hmc_ctx {
   bool profile = false;
   std::vector<hipEvent_t> ev_pool;  // per-launch timing events (profiling)
 
-  // launch shape of the transport rounds (hmc_set_launch)
-  int round_lanes_per_cu = 2048;
-  int refill_block = 64;
-  int push_chunk = 64;
+  // launch shape of the transport rounds (hmc_set_launch); 0: sized by the work
+  int round_lanes_per_cu = 0;
+  int refill_block = 0;
+  int push_chunk = 0;
   bool use_graphs = true;
   // the captured group of rounds and what it was captured with
   hipGraphExec_t round_graph = nullptr;
@@ -2613,6 +2636,14 @@ int hmc_set_launch(hmc_ctx* ctx, int round_lanes_per_cu, int refill_block, int p
 // launches. With events (profiling), each round's two kernels are bracketed.
 constexpr int kRoundsPerSync = 4;
 
+// Lanes per CU of a round's grid where the caller set none: three waves per SIMD. A
+// wave's steps are gathers of 64 scattered addresses, and the CU's one L1 serves about
+// one line per cycle: more waves thrash it sooner than they hide its latency. Slab
+// phantom, 1e7 histories, whole run: 6.54 ms at 768, 6.61 at 1024, 6.84 at 1280 (9.2 at
+// 2048 with refill blocks and push chunks of 64); 100-beamlet Dij 30.8, 30.9, 31.7 ms
+// (38.3).
+constexpr int kAutoLanesPerCu = 768;
+
 // ------------------------------------------------------------- electron energy sort
 //
 // Before the first electron round of a group, its queue is reordered by energy into
@@ -2945,8 +2976,13 @@ int hmc_transport(hmc_ctx* ctx, uint64_t seed, const hmc_work_item* items, int n
   // Rounds launch at full width: lanes of an exhausted queue exit at once, so the host
   // never needs a queue's size to launch it, and it enqueues kRoundsPerSync photon /
   // electron rounds between count reads.
-  const unsigned int round_blocks = static_cast<unsigned int>(
-      blocks_for(static_cast<long long>(std::max(ctx->cu_count, 1)) * ctx->round_lanes_per_cu));
+  // Where the caller set no width: kAutoLanesPerCu, or fewer lanes when a chunk's
+  // histories need fewer (at least one workgroup per CU).
+  const long long cus = std::max(ctx->cu_count, 1);
+  const long long lanes = ctx->round_lanes_per_cu
+                              ? cus * ctx->round_lanes_per_cu
+                              : std::min(cus * kAutoLanesPerCu, std::max(cus * 256, chunk_n));
+  const unsigned int round_blocks = static_cast<unsigned int>(blocks_for(lanes));
   if (static_cast<long long>(round_blocks) * 4 * ctx->refill_block > (1ll << 30))
     return fail(ctx, HMC_EINVAL, "round width times refill block too large");
   long long overflow = 0, rounds = 0, launches[2] = {0, 0}, graph_launches = 0;

@@ -281,6 +281,7 @@ class HipEngine:
         self._index = _device_index(self.device)
         self._ctx = nat.Context(self._index)
         self._info = nat.device_info(self._index)
+        # set_launch's defaults; until it is called the library sizes the rounds by their queues
         self.launch = {"round_lanes_per_cu": 2048, "refill_block": 64, "push_chunk": 64, "use_graphs": True}
         self._population_token = None
         self._ray_model = None

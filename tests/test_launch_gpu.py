@@ -47,6 +47,16 @@ def test_launch_shape_and_graphs_change_no_bit(slab):
         assert (got.counters["graph_launches"] > 0) == launch.get("use_graphs", True), launch
 
 
+@pytest.mark.parametrize("histories", (63, 65, 12_345, 700_001, 3_000_000))
+def test_rounds_sized_by_their_queue_match_a_fixed_shape(slab, histories):
+    """An engine without set_launch sizes refill blocks, push chunks and the grid by the
+    queue: less than a wave's worth, around one wave, and long enough for long blocks."""
+    grid, xs, src = slab
+    sized = _engine(grid, xs).run(src, histories, 1, seed=5)
+    _same(_engine(grid, xs, round_lanes_per_cu=2048, refill_block=64, push_chunk=64).run(src, histories, 1, seed=5),
+          sized)
+
+
 def test_graph_replays_match_eager_runs(slab):
     grid, xs, src = slab
     eng = _engine(grid, xs)
