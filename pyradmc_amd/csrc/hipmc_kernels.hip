@@ -68,8 +68,9 @@ struct Queue {
 // would become a generic address): the two output queues' current chunks
 // [wave][queue][next, end], and the block's ledger reduction slots [book][wave]
 // (books 6 and 7: the wave's pops and pushes).
-__shared__ unsigned int g_chunk[4][2][2];
-__shared__ long long g_books[8 * 4];
+constexpr int kMaxBlockWaves = 16;  // of any round kernel
+__shared__ unsigned int g_chunk[kMaxBlockWaves][2][2];
+__shared__ long long g_books[8 * kMaxBlockWaves];
 
 // Accesses to that state: relaxed atomics at wave scope, so that every access is a real
 // LDS access (lanes of divergent branches see one another's updates) and the compiler
@@ -131,7 +132,8 @@ struct RefillPool {
   // Every wave of the grid owns one static block.
   __device__ RefillPool(unsigned int r, unsigned int queue_length)
       : block(r ? r : sized(queue_length, 4u)), n_in(r ? 0u : queue_length) {
-    const unsigned int wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    // Consecutive blocks first: a short queue spreads over all CUs.
+    const unsigned int wave = (threadIdx.x >> 6) * gridDim.x + blockIdx.x;
     next = wave * block;
     end = next + block;
     n_static = gridDim.x * (blockDim.x >> 6) * block;
@@ -240,8 +242,8 @@ struct LaneTally {
 
   // base = L_P_VOX for the photon round, L_E_VOX for the electron round. Every thread
   // of the block must call this after its lane loop (it synchronises the block): the
-  // books are summed over the wave, then over the block in LDS (red: 8 x 4 slots; the
-  // wave's pop and push counts are already in red[6*4 + wave] and red[7*4 + wave]),
+  // books are summed over the wave, then over the block in LDS (red: 8 rows
+  // of kMaxBlockWaves; the wave's pop and push counts are already in rows 6 and 7),
   // and written with one atomic per book per block.
   __device__ void flush(unsigned long long* ledger, int base, long long* red) const {
     const long long books[6] = {escaped, unscored, deposited, static_cast<long long>(vox),
@@ -250,14 +252,14 @@ struct LaneTally {
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
       const long long total = wave_sum(books[k]);
-      if (__lane_id() == 0) red[k * 4 + wave] = total;
+      if (__lane_id() == 0) red[k * kMaxBlockWaves + wave] = total;
     }
     __syncthreads();
     if (threadIdx.x < 8) {
       const int slot[8] = {L_ESCAPED, L_UNSCORED, L_DEPOSITED, base,
                            base + 1,  base + 2,   base + 3,    base + 4};
       long long total = 0;
-      for (int wv = 0; wv < static_cast<int>(blockDim.x >> 6); ++wv) total += red[threadIdx.x * 4 + wv];
+      for (int wv = 0; wv < static_cast<int>(blockDim.x >> 6); ++wv) total += red[threadIdx.x * kMaxBlockWaves + wv];
       if (total != 0)
         atomicAdd(ledger + slot[threadIdx.x], static_cast<unsigned long long>(total));
     }
@@ -282,7 +284,7 @@ __device__ inline unsigned int chunk_reserve(const Queue& q) {
   if (lane == leader) {
     const int wave = static_cast<int>(threadIdx.x >> 6);
     unsigned int* chunk = g_chunk[wave][q.lds];
-    lds_add(&g_books[7 * 4 + wave], cnt);
+    lds_add(&g_books[7 * kMaxBlockWaves + wave], cnt);
     next = lds_load(chunk);
     avail = lds_load(chunk + 1) - next;
     if (cnt <= avail) {
@@ -314,7 +316,7 @@ __device__ inline void count_pops(bool real) {
   const unsigned long long mask = __ballot(real ? 1 : 0);
   const unsigned long long active = __ballot(1);
   if (static_cast<int>(__lane_id()) == __ffsll(static_cast<long long>(active)) - 1) {
-    lds_add(&g_books[6 * 4 + (threadIdx.x >> 6)], __popcll(mask));
+    lds_add(&g_books[6 * kMaxBlockWaves + (threadIdx.x >> 6)], __popcll(mask));
   }
 }
 
@@ -357,10 +359,11 @@ __device__ inline float spr(const TransportParams& P, float e, int mat) {
 // scoring grid or the unscored book (pyradmc/backends/warp/kernels.py:535-584). As there,
 // quanta are x + 1/2 truncated toward zero (an amount a rounding step left slightly
 // negative rounds toward zero, unlike an escape's floor).
-template <bool kFast>
+template <bool kFast, bool kOne>
 __device__ inline void deposit(const TransportParams& P, LaneTally& tal, long long base, float x,
                                float y, float z, float amount, float factor) {
-  const long long idx = kFast ? grid_index(P.s, x, y, z) : scoring_index(P.s, x, y, z);
+  // Fast build: the scoring grid is the transport grid, whose numbers are at hand.
+  const long long idx = kFast ? grid_index<kOne>(P.g, x, y, z) : scoring_index<kOne>(P.s, x, y, z);
   if (idx >= 0) {
     const long long q = whole_to_ll(trunc(static_cast<double>(amount) * static_cast<double>(factor) *
                                           kInvQuantum + 0.5));
@@ -382,23 +385,23 @@ __device__ inline void escape(LaneTally& tal, float amount) {
 }
 
 // Deposit if inside the transport grid, else escaped (kernels.py:600-633).
-template <bool kFast>
+template <bool kFast, bool kOne>
 __device__ inline void deposit_or_escape(const TransportParams& P, LaneTally& tal, long long base,
                                          float x, float y, float z, float amount, float factor) {
   if (amount <= 0.0f) return;
-  if (inside_grid(P.g, x, y, z)) deposit<kFast>(P, tal, base, x, y, z, amount, factor);
+  if (inside_grid(P.g, x, y, z)) deposit<kFast, kOne>(P, tal, base, x, y, z, amount, factor);
   else escape(tal, amount);
 }
 
 // One half-substep's continuous loss, in equal pieces no longer than the
 // resolution (pyradmc/transport/electron.py:169-191, 361-380).
-template <bool kFast>
+template <bool kFast, bool kOne>
 __device__ inline void deposit_spread(const TransportParams& P, LaneTally& tal, long long base,
                                       float x, float y, float z, float ux, float uy, float uz,
                                       float length, float amount, float factor) {
   if constexpr (kFast) {  // one piece: the midpoint takes the whole amount
     const float t = 0.5f * length;
-    deposit_or_escape<kFast>(P, tal, base, x + ux * t, y + uy * t, z + uz * t, amount, factor);
+    deposit_or_escape<kFast, kOne>(P, tal, base, x + ux * t, y + uy * t, z + uz * t, amount, factor);
     return;
   }
   int n = 1;
@@ -410,18 +413,18 @@ __device__ inline void deposit_spread(const TransportParams& P, LaneTally& tal, 
   const float piece = length / static_cast<float>(n);
   for (int k = 0; k < n; ++k) {
     const float t = (static_cast<float>(k) + 0.5f) * piece;
-    deposit_or_escape<kFast>(P, tal, base, x + ux * t, y + uy * t, z + uz * t, share, factor);
+    deposit_or_escape<kFast, kOne>(P, tal, base, x + ux * t, y + uy * t, z + uz * t, share, factor);
   }
 }
 
 // Positron annihilation at rest: two back-to-back 511 keV photons, isotropic
 // (pyradmc/transport/particles.py:75-102).
-template <bool kFast>
+template <bool kFast, bool kOne>
 __device__ inline void annihilate(const TransportParams& P, LaneTally& tal, const Queue& qp,
                                   long long base, uint32_t column, float x, float y, float z,
                                   float w, float factor, uint64_t& rng) {
   if (P.pcut >= kElectronMass) {
-    deposit<kFast>(P, tal, base, x, y, z, w * 2.0f * kElectronMass, factor);
+    deposit<kFast, kOne>(P, tal, base, x, y, z, w * 2.0f * kElectronMass, factor);
     return;
   }
   float ax, ay, az;
@@ -507,7 +510,7 @@ k_photon_round(TransportParams P, Queue qin,
   // ledger reduction slots.
   const int wave_in_block = static_cast<int>(threadIdx.x >> 6);
   if (__lane_id() < 4) g_chunk[wave_in_block][__lane_id() >> 1][__lane_id() & 1] = 0u;
-  if (__lane_id() < 2) g_books[(6 + __lane_id()) * 4 + wave_in_block] = 0;
+  if (__lane_id() < 2) g_books[(6 + __lane_id()) * kMaxBlockWaves + wave_in_block] = 0;
   qe.lds = 0;
   qp.lds = 1;
   if (qe.push_chunk == 0u) qe.push_chunk = qp.push_chunk = sized_push_chunk(n_in, qe.capacity);
@@ -587,14 +590,14 @@ k_photon_round(TransportParams P, Queue qin,
         const uint64_t child = spawn_stream(rng);
         push(qe, ELECTRON, column, recoil, w, x, y, z, ex, ey, ez, child);
       } else {
-        deposit<kFast>(P, tal, base, x, y, z, w * recoil,
+        deposit<kFast, false>(P, tal, base, x, y, z, w * recoil,
                 spr<kFast>(P, recoil, mat));
       }
       const float cg = compton_cos(e, ratio);
       rotate(ux, uy, uz, cg, phi);
       e *= ratio;
       if (e <= P.pcut) {
-        deposit<kFast>(P, tal, base, x, y, z, w * e, spr<kFast>(P, e, mat));
+        deposit<kFast, false>(P, tal, base, x, y, z, w * e, spr<kFast>(P, e, mat));
         active = false;
         continue;
       }
@@ -614,7 +617,7 @@ k_photon_round(TransportParams P, Queue qin,
         const uint64_t child = spawn_stream(rng);
         push(qe, ELECTRON, column, e, w, x, y, z, ux, uy, uz, child);
       } else {
-        deposit<kFast>(P, tal, base, x, y, z, w * e, spr<kFast>(P, e, mat));
+        deposit<kFast, false>(P, tal, base, x, y, z, w * e, spr<kFast>(P, e, mat));
       }
       active = false;
     } else {  // pair production
@@ -628,21 +631,21 @@ k_photon_round(TransportParams P, Queue qin,
           const uint64_t child = spawn_stream(rng);
           push(qe, ELECTRON, column, share_e, w, x, y, z, ux, uy, uz, child);
         } else {
-          deposit<kFast>(P, tal, base, x, y, z, w * share_e,
+          deposit<kFast, false>(P, tal, base, x, y, z, w * share_e,
                   spr<kFast>(P, share_e, mat));
         }
         if (share_p > P.ecut) {
           const uint64_t child = spawn_stream(rng);
           push(qe, POSITRON, column, share_p, w, x, y, z, ux, uy, uz, child);
         } else {
-          deposit<kFast>(P, tal, base, x, y, z, w * share_p,
+          deposit<kFast, false>(P, tal, base, x, y, z, w * share_p,
                   spr<kFast>(P, share_p, mat));
-          annihilate<kFast>(P, tal, qp, base, column, x, y, z, w, f_ann, rng);
+          annihilate<kFast, false>(P, tal, qp, base, column, x, y, z, w, f_ann, rng);
         }
       } else {
-        deposit<kFast>(P, tal, base, x, y, z, w * kinetic,
+        deposit<kFast, false>(P, tal, base, x, y, z, w * kinetic,
                 spr<kFast>(P, kinetic, mat));
-        annihilate<kFast>(P, tal, qp, base, column, x, y, z, w, f_ann, rng);
+        annihilate<kFast, false>(P, tal, qp, base, column, x, y, z, w, f_ann, rng);
       }
       active = false;
     }
@@ -659,10 +662,45 @@ k_photon_round(TransportParams P, Queue qin,
 // CSDA loss through the restricted range and its inverse, Bernoulli brems, random
 // hinge with GS (or Gaussian) deflection, two half-step deposits, Moller delta
 // (pyradmc/transport/electron.py:292-481, kernels.py:1532-1885).
-template <bool kFast>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HMC_ROUND_WAVES, 8)))
-k_electron_round(TransportParams P, Queue qin,
-                                                        unsigned int* head, Queue qp, Queue qe) {
+//
+// What bounds it: a wave's step gathers from 64 scattered addresses at a time, and a
+// CU's L1 serves about one cache line per cycle, so each gather costs the CU some 64
+// cycles whatever its width; and the rare blocks of a step run for a lane or two of 64.
+// kOne, the build for one material whose tables fit (every analytic water run): the
+// electron tables sit in LDS (56 KB a block of 12 waves) and the material map is not
+// read, which leaves the density, the GS nodes and the tallies as gathers.
+// Moller interactions (1 % of the steps, but in 40 % of a wave's passes) wait in a
+// stack in LDS: the lane that meets one writes its particle there and is free for
+// another, and once kMollerBatch wait, idle lanes take them back and run the block
+// together. Lanes that wait in place for the others (no stack) cost more than they save.
+// Slab phantom, 1e7 histories, whole run: 6.54 ms with tables in L2 and Moller
+// interactions in place, 5.46 with both changes, 5.28 with 24-bit voxel indices and
+// unscaled quotients, 4.98 with the GS nodes of a cell in one 16-byte gather. Blocks of
+// 12 waves, one to a CU: 5.0 ms; two to a CU 5.3 (the L1 holds fewer waves' lines).
+// More materials or longer tables than fit take the general build.
+constexpr int kTablePoints = 2048;   // largest table of the kOne build
+constexpr int kMollerSlots = 32;     // stack slots of a wave
+constexpr int kMollerBatch = 16;     // waiting particles that make a batch
+constexpr int kParticleWords = 12;   // x y z e | ux uy uz w | rng | column and kind | steps
+template <bool kOne>
+constexpr int kElectronThreads = kOne ? 768 : 256;
+
+template <bool kOne>
+struct ElectronShared {
+  uint32_t stack[kElectronThreads<kOne> / 64][kParticleWords][kMollerSlots];
+};
+template <>
+struct ElectronShared<true> {
+  float4 a[kTablePoints];  // DevTables::elec_a of the one material
+  float2 b[kTablePoints];  // scattering power, log eta
+  float inv_range[kTablePoints];
+  uint32_t stack[kElectronThreads<true> / 64][kParticleWords][kMollerSlots];
+};
+
+template <bool kFast, bool kOne>
+__global__ void __launch_bounds__(kElectronThreads<kOne>) __attribute__((amdgpu_waves_per_eu(kOne ? 3 : HMC_ROUND_WAVES, 8)))
+k_electron_round(TransportParams P, Queue qin, unsigned int* head, Queue qp, Queue qe) {
+  __shared__ ElectronShared<kOne> sh;
   const unsigned int n_in = min(*qin.count, qin.capacity);
   LaneTally tal;
   bool active = false;
@@ -678,208 +716,298 @@ k_electron_round(TransportParams P, Queue qin,
   // ledger reduction slots.
   const int wave_in_block = static_cast<int>(threadIdx.x >> 6);
   if (__lane_id() < 4) g_chunk[wave_in_block][__lane_id() >> 1][__lane_id() & 1] = 0u;
-  if (__lane_id() < 2) g_books[(6 + __lane_id()) * 4 + wave_in_block] = 0;
+  if (__lane_id() < 2) g_books[(6 + __lane_id()) * kMaxBlockWaves + wave_in_block] = 0;
   qp.lds = 0;
   qe.lds = 1;
   if (qe.push_chunk == 0u) qe.push_chunk = qp.push_chunk = sized_push_chunk(n_in, qe.capacity);
   RefillPool pool(P.refill_block, n_in);
+  if constexpr (kOne) {
+    // A block whose first wave has no static block has no work at all (its other waves'
+    // blocks lie further on).
+    if (blockIdx.x * pool.block < n_in) {
+      for (int k = static_cast<int>(threadIdx.x); k < n; k += kElectronThreads<kOne>) {
+        sh.a[k] = P.t.elec_a[k];
+        const float4 b = P.t.elec_b[k];
+        sh.b[k] = make_float2(b.x, b.y);
+        sh.inv_range[k] = P.t.inv_range[k];
+      }
+    }
+    __syncthreads();
+  }
+  auto spr_of = [&](float energy, int mat) {
+    return kOne ? 1.0f : spr<kFast>(P, energy, mat);  // the first material is water
+  };
+  auto& stack = sh.stack[wave_in_block];
+  unsigned int waiting = 0;  // stack entries of this wave
+  bool parked = false;       // this lane's Moller interaction found the stack full
+  bool exhausted = false;    // this wave's claims lie beyond the queue
+  // All lanes stay in the loop until the wave has nothing left.
   while (true) {
-    // Idle lanes take new particles together, once kRefillIdleLanes of the wave's
-    // looping lanes are idle (or all of them): the refill block then runs for more
-    // lanes at a time and in fewer passes. Each particle's history is its own, so
-    // the results do not depend on when a lane takes it.
-    const int n_idle = __popcll(__ballot(!active));
-    const bool refill_now = !active && (n_idle >= kRefillIdleLanes || n_idle == __popcll(__ballot(1)));
-    const unsigned int i = refill_index(pool, head, refill_now);
-    if (!active) {
-      if (!refill_now) continue;
-      if (i >= n_in) break;
-      uint32_t meta;
-      load_particle(qin.data, i, x, y, z, e, ux, uy, uz, w, rng, meta);
-      const bool real = (meta & 3u) != kEmptyKind;  // else padding left by a producer wave
-      count_pops(real);
-      if (!real) continue;
-      column = meta >> 3;
-      positron = (meta & 3u) == POSITRON;
-      base = static_cast<long long>(column) * P.s.n_voxels;
-      const float latent = positron ? 2.0f * kElectronMass : 0.0f;
-      if (!enter_grid(P.g, x, y, z, ux, uy, uz)) {
-        escape(tal, w * (e + latent));
-        continue;
+    // Idle lanes take new particles together, once kRefillIdleLanes of the wave are idle:
+    // the refill block then runs for more lanes at a time and in fewer passes. Each
+    // particle's history is its own, so the results do not depend on when a lane takes it.
+    const unsigned long long idle_mask = __ballot(active ? 0 : 1);
+    const unsigned int n_idle = static_cast<unsigned int>(__popcll(idle_mask));
+    const bool refill_now = n_idle >= static_cast<unsigned int>(kRefillIdleLanes);
+    if (__ballot(parked ? 1 : 0) != 0ull ||
+        (refill_now && (waiting >= static_cast<unsigned int>(kMollerBatch) || (exhausted && waiting != 0u)))) {
+      const unsigned int take = min(waiting, n_idle);
+      waiting -= take;
+      const unsigned int rank =
+          static_cast<unsigned int>(__popcll(idle_mask & ((1ull << __lane_id()) - 1ull)));
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const bool popped = !active && rank < take;
+      if (popped) {
+        const unsigned int slot = waiting + rank;
+        x = __uint_as_float(stack[0][slot]);
+        y = __uint_as_float(stack[1][slot]);
+        z = __uint_as_float(stack[2][slot]);
+        e = __uint_as_float(stack[3][slot]);
+        ux = __uint_as_float(stack[4][slot]);
+        uy = __uint_as_float(stack[5][slot]);
+        uz = __uint_as_float(stack[6][slot]);
+        w = __uint_as_float(stack[7][slot]);
+        rng = static_cast<uint64_t>(stack[8][slot]) | (static_cast<uint64_t>(stack[9][slot]) << 32);
+        const uint32_t word = stack[10][slot];
+        column = word >> 1;
+        positron = (word & 1u) != 0u;
+        steps = static_cast<int>(stack[11][slot]);
+        base = static_cast<long long>(column) * P.s.n_voxels;
+        active = true;
       }
-      active = true;
-      steps = 0;
-    }
-    tal.steps++;
-    const float latent = positron ? 2.0f * kElectronMass : 0.0f;
-    if (++steps > P.max_steps) {
-      atomicAdd(P.ledger + L_TRAPPED, 1ull);
-      escape(tal, w * (e + latent));
-      active = false;
-      continue;
-    }
-
-    const int ix = axis_index(x, P.g.x_lo, P.g.inv_sx, P.g.nx);
-    const int iy = axis_index(y, P.g.y_lo, P.g.inv_sy, P.g.ny);
-    const int iz = axis_index(z, P.g.z_lo, P.g.inv_sz, P.g.nz);
-    const long long vox = (static_cast<long long>(ix) * P.g.ny + iy) * P.g.nz + iz;
-    const int mat = P.g.material[vox];
-    tal.vox++;
-
-    if (e <= P.ecut) {
-      // Terminal: local deposit, annihilation for a positron.
-      deposit<kFast>(P, tal, base, x, y, z, w * e, spr<kFast>(P, e, mat));
-      if (positron)
-        annihilate<kFast>(P, tal, qp, base, column, x, y, z, w,
-                   spr<kFast>(P, kElectronMass, mat), rng);
-      active = false;
-      continue;
-    }
-    const float rho = P.g.density[vox];
-    const long long row = static_cast<long long>(mat) * n;
-
-    int ei;
-    float ew;
-    const float log_e = __logf(e);
-    grid_locate(log_e, P.t.e_log_min, P.t.e_inv_dlog, n, ei, ew);
-    const float4 ea = lerp4(P.t.elec_a + row, ei, ew);  // csda, moller, r_range, radiative
-
-    const float range_cm = ea.x / rho;
-    float s_max = P.step_fraction * range_cm;
-    if (!P.msc_gs) {
-      const float tp = lerp4(P.t.elec_b + row, ei, ew).x;
-      s_max = fminf(s_max, kHingeTheta2Max / (tp * rho));
-    }
-    const float s_boundary = boundary_distance(P.g, x, y, z, ux, uy, uz) + kBoundaryNudge;
-    const float s_geometry = fminf(s_max, s_boundary);
-    const float sigma_moller = rho * ea.y;
-    float s = s_geometry;
-    bool moller_pending = false;
-    if (sigma_moller > 0.0f) {
-      const float s_int = sample_path(sigma_moller, rng);
-      if (s_int <= s_geometry) {
-        s = s_int;
-        moller_pending = true;
+      if (popped || parked) {
+        parked = false;
+        const float delta = sample_moller(e, P.ecut, rng);
+        float cd, cp;
+        moller_cosines(e, delta, cd, cp);
+        const float mphi = kTwoPi * uniform(rng);
+        float dx = ux, dy = uy, dz = uz;
+        rotate(dx, dy, dz, cd, mphi);
+        const uint64_t child = spawn_stream(rng);
+        push(qe, ELECTRON, column, delta, w, x, y, z, dx, dy, dz, child);
+        rotate(ux, uy, uz, cp, mphi + kPi);
+        e -= delta;
       }
-    }
-
-    const float available = ea.z;
-    float de;
-    if (rho * s >= available) {
-      s = available / rho;
-      de = e - P.ecut;
-      moller_pending = false;
-    } else {
-      int ri;
-      float rw;
-      grid_locate(__logf(available - rho * s), P.t.r_log_min, P.t.r_inv_dlog, n, ri, rw);
-      float e_end = lerp1(P.t.inv_range + row, ri, rw);
-      e_end = fminf(fmaxf(e_end, P.ecut), e);
-      de = e - e_end;
-    }
-    // Bernoulli bremsstrahlung matched to the radiative stopping power
-    // (pyradmc/physics/brems.py:30-66).
-    const float radiative_loss = ea.w * rho * s;
-    float emit_probability, local_brems;
-    brems_step(e, radiative_loss, P.pcut, log_e, P.log_pcut, emit_probability, local_brems);
-    const float continuous = de + local_brems;
-    const bool emit_brems = uniform(rng) < emit_probability;
-    const float factor = spr<kFast>(P, e, mat);
-
-    const float s1 = uniform(rng) * s;
-    const float s2 = s - s1;
-    const float d1 = s > 0.0f ? continuous * (s1 / s) : 0.0f;
-    const float d2 = continuous - d1;
-
-    deposit_spread<kFast>(P, tal, base, x, y, z, ux, uy, uz, s1, w * d1, factor);
-    e -= d1;
-    x += ux * s1;
-    y += uy * s1;
-    z += uz * s1;
-    if (!inside_grid(P.g, x, y, z)) {
-      escape(tal, w * (e + latent));
-      active = false;
-      continue;
-    }
-
-    const float log_e_mid = __logf(e);
-    grid_locate(log_e_mid, P.t.e_log_min, P.t.e_inv_dlog, n, ei, ew);
-    const float4 eb = lerp4(P.t.elec_b + row, ei, ew);  // scattering power, log eta
-    const float mean_square = eb.x * rho * s;
-    float cos_hinge;
-    if (P.msc_gs) {
-      const float fx = eb.y * kGsBinsPerLog;
-      const float fy = __logf(fmaxf(mean_square, kGsTheta2Min)) * kGsBinsPerLog;
-      cos_hinge = sample_gs(P.t, fx, fy, mean_square, rng);
-    } else {
-      cos_hinge = sample_gaussian_hinge(mean_square, rng);
-    }
-    const float phi = kTwoPi * uniform(rng);
-    rotate(ux, uy, uz, cos_hinge, phi);
-
-    if (emit_brems && e > P.pcut) {
-      float k = sample_brems_energy(P.pcut, log_e_mid, P.log_pcut, rng);
-      k = fminf(k, e - d2);
-      if (k > P.pcut) {
-        float photon_w = w;
-        if (k < kRouletteMeV && w < kRouletteWeightCap) {
-          photon_w = uniform(rng) < kRouletteSurvival ? w / kRouletteSurvival : 0.0f;
-          escape(tal, (w - photon_w) * k);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    } else if (refill_now) {
+      if (!exhausted) {
+        const unsigned int i = refill_index(pool, head, !active);
+        exhausted = __ballot(!active && i >= n_in ? 1 : 0) != 0ull;
+        if (!active && i < n_in) {
+          uint32_t meta;
+          load_particle(qin.data, i, x, y, z, e, ux, uy, uz, w, rng, meta);
+          const bool real = (meta & 3u) != kEmptyKind;  // else padding left by a producer wave
+          count_pops(real);
+          if (real) {
+            column = meta >> 3;
+            positron = (meta & 3u) == POSITRON;
+            base = static_cast<long long>(column) * P.s.n_voxels;
+            if (!enter_grid(P.g, x, y, z, ux, uy, uz)) {
+              escape(tal, w * (e + (positron ? 2.0f * kElectronMass : 0.0f)));
+            } else {
+              active = true;
+              steps = 0;
+            }
+          }
         }
-        if (photon_w > 0.0f) {
-          const uint64_t child = spawn_stream(rng);
-          push(qp, PHOTON, column, k, photon_w, x, y, z, ux, uy, uz, child);
-        }
-      } else {
-        deposit_or_escape<kFast>(P, tal, base, x, y, z, w * k,
-                          spr<kFast>(P, k, mat));
+      } else if (n_idle == 64u) {
+        break;
       }
-      e -= k;
     }
-
-    deposit_spread<kFast>(P, tal, base, x, y, z, ux, uy, uz, s2, w * d2, factor);
-    e -= d2;
-    x += ux * s2;
-    y += uy * s2;
-    z += uz * s2;
-    if (!inside_grid(P.g, x, y, z)) {
-      escape(tal, w * (e + latent));
-      active = false;
-      continue;
-    }
-
-    if (moller_pending && e > 2.0f * P.ecut) {
-      const float delta = sample_moller(e, P.ecut, rng);
-      float cd, cp;
-      moller_cosines(e, delta, cd, cp);
-      const float mphi = kTwoPi * uniform(rng);
-      float dx = ux, dy = uy, dz = uz;
-      rotate(dx, dy, dz, cd, mphi);
-      const uint64_t child = spawn_stream(rng);
-      push(qe, ELECTRON, column, delta, w, x, y, z, dx, dy, dz, child);
-      rotate(ux, uy, uz, cp, mphi + kPi);
-      e -= delta;
-    }
-
-    // Ended at or below the cutoff (a range-limited step ends exactly there): the
-    // terminal deposit the next pass would make, made now with the same position,
-    // energy, random state and books, so that the lane is idle from the next pass on
-    // instead of spending it on the deposit alone. A particle the next pass would
-    // count as trapped is left to it.
-    if (e <= P.ecut && steps < P.max_steps) {
+    bool moller = false;  // this lane's step ended in a Moller interaction
+    if (active && !parked) do {
       tal.steps++;
-      tal.vox++;
-      int mat_end = 0;
-      if constexpr (!kFast) {
-        const int jx = axis_index(x, P.g.x_lo, P.g.inv_sx, P.g.nx);
-        const int jy = axis_index(y, P.g.y_lo, P.g.inv_sy, P.g.ny);
-        const int jz = axis_index(z, P.g.z_lo, P.g.inv_sz, P.g.nz);
-        mat_end = P.g.material[(static_cast<long long>(jx) * P.g.ny + jy) * P.g.nz + jz];
+      const float latent = positron ? 2.0f * kElectronMass : 0.0f;
+      if (++steps > P.max_steps) {
+        atomicAdd(P.ledger + L_TRAPPED, 1ull);
+        escape(tal, w * (e + latent));
+        active = false;
+        break;
       }
-      deposit<kFast>(P, tal, base, x, y, z, w * e, spr<kFast>(P, e, mat_end));
-      if (positron)
-        annihilate<kFast>(P, tal, qp, base, column, x, y, z, w, spr<kFast>(P, kElectronMass, mat_end), rng);
-      active = false;
+
+      const long long vox = grid_index<kOne>(P.g, x, y, z);
+      const int mat = kOne ? 0 : P.g.material[vox];
+      tal.vox++;
+
+      if (e <= P.ecut) {
+        // Terminal: local deposit, annihilation for a positron.
+        deposit<kFast, kOne>(P, tal, base, x, y, z, w * e, spr_of(e, mat));
+        if (positron)
+          annihilate<kFast, kOne>(P, tal, qp, base, column, x, y, z, w, spr_of(kElectronMass, mat), rng);
+        active = false;
+        break;
+      }
+      const float rho = P.g.density[vox];
+      const long long row = static_cast<long long>(mat) * n;
+
+      int ei;
+      float ew;
+      const float log_e = __logf(e);
+      grid_locate(log_e, P.t.e_log_min, P.t.e_inv_dlog, n, ei, ew);
+      float4 ea;  // csda, moller, r_range, radiative
+      if constexpr (kOne) ea = lerp4(sh.a, ei, ew);
+      else ea = lerp4(P.t.elec_a + row, ei, ew);
+      auto scattering = [&]() {  // scattering power, log eta at (ei, ew)
+        if constexpr (kOne) {
+          const float2 lo = sh.b[ei], hi = sh.b[ei + 1];
+          const float wa = 1.0f - ew;
+          return make_float2(lo.x * wa + hi.x * ew, lo.y * wa + hi.y * ew);
+        } else {
+          const float4 b = lerp4(P.t.elec_b + row, ei, ew);
+          return make_float2(b.x, b.y);
+        }
+      };
+
+      const float range_cm = quotient(ea.x, rho);
+      float s_max = P.step_fraction * range_cm;
+      if (!P.msc_gs) {
+        const float tp = scattering().x;
+        s_max = fminf(s_max, quotient(kHingeTheta2Max, tp * rho));
+      }
+      const float s_boundary = boundary_distance(P.g, x, y, z, ux, uy, uz) + kBoundaryNudge;
+      const float s_geometry = fminf(s_max, s_boundary);
+      const float sigma_moller = rho * ea.y;
+      float s = s_geometry;
+      bool moller_pending = false;
+      if (sigma_moller > 0.0f) {
+        const float s_int = sample_path(sigma_moller, rng);
+        if (s_int <= s_geometry) {
+          s = s_int;
+          moller_pending = true;
+        }
+      }
+
+      const float available = ea.z;
+      float de;
+      if (rho * s >= available) {
+        s = quotient(available, rho);
+        de = e - P.ecut;
+        moller_pending = false;
+      } else {
+        int ri;
+        float rw;
+        grid_locate(__logf(available - rho * s), P.t.r_log_min, P.t.r_inv_dlog, n, ri, rw);
+        float e_end;
+        if constexpr (kOne) e_end = lerp1(sh.inv_range, ri, rw);
+        else e_end = lerp1(P.t.inv_range + row, ri, rw);
+        e_end = fminf(fmaxf(e_end, P.ecut), e);
+        de = e - e_end;
+      }
+      // Bernoulli bremsstrahlung matched to the radiative stopping power
+      // (pyradmc/physics/brems.py:30-66).
+      const float radiative_loss = ea.w * rho * s;
+      float emit_probability, local_brems;
+      brems_step(e, radiative_loss, P.pcut, log_e, P.log_pcut, emit_probability, local_brems);
+      const float continuous = de + local_brems;
+      const bool emit_brems = uniform(rng) < emit_probability;
+      const float factor = spr_of(e, mat);
+
+      const float s1 = uniform(rng) * s;
+      const float s2 = s - s1;
+      const float d1 = s > 0.0f ? continuous * quotient(s1, s) : 0.0f;
+      const float d2 = continuous - d1;
+
+      deposit_spread<kFast, kOne>(P, tal, base, x, y, z, ux, uy, uz, s1, w * d1, factor);
+      e -= d1;
+      x += ux * s1;
+      y += uy * s1;
+      z += uz * s1;
+      if (!inside_grid(P.g, x, y, z)) {
+        escape(tal, w * (e + latent));
+        active = false;
+        break;
+      }
+
+      const float log_e_mid = __logf(e);
+      grid_locate(log_e_mid, P.t.e_log_min, P.t.e_inv_dlog, n, ei, ew);
+      const float2 eb = scattering();
+      const float mean_square = eb.x * rho * s;
+      float cos_hinge;
+      if (P.msc_gs) {
+        const float fx = eb.y * kGsBinsPerLog;
+        const float fy = __logf(fmaxf(mean_square, kGsTheta2Min)) * kGsBinsPerLog;
+        cos_hinge = sample_gs(P.t, fx, fy, mean_square, rng);
+      } else {
+        cos_hinge = sample_gaussian_hinge(mean_square, rng);
+      }
+      const float phi = kTwoPi * uniform(rng);
+      rotate(ux, uy, uz, cos_hinge, phi);
+
+      if (emit_brems && e > P.pcut) {
+        float k = sample_brems_energy(P.pcut, log_e_mid, P.log_pcut, rng);
+        k = fminf(k, e - d2);
+        if (k > P.pcut) {
+          float photon_w = w;
+          if (k < kRouletteMeV && w < kRouletteWeightCap) {
+            photon_w = uniform(rng) < kRouletteSurvival ? w / kRouletteSurvival : 0.0f;
+            escape(tal, (w - photon_w) * k);
+          }
+          if (photon_w > 0.0f) {
+            const uint64_t child = spawn_stream(rng);
+            push(qp, PHOTON, column, k, photon_w, x, y, z, ux, uy, uz, child);
+          }
+        } else {
+          deposit_or_escape<kFast, kOne>(P, tal, base, x, y, z, w * k, spr_of(k, mat));
+        }
+        e -= k;
+      }
+
+      deposit_spread<kFast, kOne>(P, tal, base, x, y, z, ux, uy, uz, s2, w * d2, factor);
+      e -= d2;
+      x += ux * s2;
+      y += uy * s2;
+      z += uz * s2;
+      if (!inside_grid(P.g, x, y, z)) {
+        escape(tal, w * (e + latent));
+        active = false;
+        break;
+      }
+
+      moller = moller_pending && e > 2.0f * P.ecut;
+
+      // Ended at or below the cutoff (a range-limited step ends exactly there): the
+      // terminal deposit the next pass would make, made now with the same position,
+      // energy, random state and books, so that the lane is idle from the next pass on
+      // instead of spending it on the deposit alone. A particle the next pass would
+      // count as trapped is left to it.
+      if (e <= P.ecut && steps < P.max_steps) {
+        tal.steps++;
+        tal.vox++;
+        int mat_end = 0;
+        if constexpr (!kFast && !kOne) {
+          mat_end = P.g.material[grid_index<kOne>(P.g, x, y, z)];
+        }
+        deposit<kFast, kOne>(P, tal, base, x, y, z, w * e, spr_of(e, mat_end));
+        if (positron)
+          annihilate<kFast, kOne>(P, tal, qp, base, column, x, y, z, w, spr_of(kElectronMass, mat_end), rng);
+        active = false;
+      }
+    } while (false);
+    const unsigned long long met = __ballot(moller ? 1 : 0);
+    if (met != 0ull) {
+      const unsigned int slot =
+          waiting + static_cast<unsigned int>(__popcll(met & ((1ull << __lane_id()) - 1ull)));
+      if (moller) {
+        if (slot < static_cast<unsigned int>(kMollerSlots)) {
+          stack[0][slot] = __float_as_uint(x);
+          stack[1][slot] = __float_as_uint(y);
+          stack[2][slot] = __float_as_uint(z);
+          stack[3][slot] = __float_as_uint(e);
+          stack[4][slot] = __float_as_uint(ux);
+          stack[5][slot] = __float_as_uint(uy);
+          stack[6][slot] = __float_as_uint(uz);
+          stack[7][slot] = __float_as_uint(w);
+          stack[8][slot] = static_cast<uint32_t>(rng);
+          stack[9][slot] = static_cast<uint32_t>(rng >> 32);
+          stack[10][slot] = (column << 1) | (positron ? 1u : 0u);
+          stack[11][slot] = static_cast<uint32_t>(steps);
+          active = false;
+        } else {
+          parked = true;
+        }
+      }
+      waiting = min(waiting + static_cast<unsigned int>(__popcll(met)), static_cast<unsigned int>(kMollerSlots));
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     }
   }
   seal_chunk(qp);
@@ -1245,6 +1373,20 @@ __global__ void k_set_entries(double* __restrict__ mean, double* __restrict__ si
   }
 }
 
+// The GS grid's nodes [n_eta][n_theta2][n_u] as cells (DevTables::gs): a sample then takes
+// its four values in one 16-byte gather instead of four, for four times the memory.
+__global__ void __launch_bounds__(256) k_gs_cells(const float* __restrict__ nodes, int n_theta2, int n_u,
+                                                  long long cells, float4* __restrict__ out) {
+  for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < cells;
+       i += static_cast<long long>(gridDim.x) * blockDim.x) {
+    const long long u = i % n_u, at = i / n_u;
+    const long long iy = at % (n_theta2 - 1), ix = at / (n_theta2 - 1);
+    const float* lo = nodes + (ix * n_theta2 + iy) * n_u + u;
+    const float* hi = lo + static_cast<long long>(n_theta2) * n_u;
+    out[i] = make_float4(lo[0], hi[0], lo[n_u], hi[n_u]);
+  }
+}
+
 __global__ void k_fill_u64(unsigned long long* a, long long n, unsigned long long v) {
   for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
        i += static_cast<long long>(gridDim.x) * blockDim.x)
@@ -1490,7 +1632,8 @@ struct hmc_ctx {
   DevTables t{};
   std::vector<void*> table_buffers;
   bool has_tables = false;
-  float* d_gs = nullptr;
+  float* d_gs = nullptr;         // nodes as given
+  float4* d_gs_cells = nullptr;  // DevTables::gs
   bool has_gs = false;
 
   // source
@@ -1727,6 +1870,7 @@ void hmc_destroy(hmc_ctx* ctx) {
   (void)hipStreamSynchronize(ctx->stream);
   void* ptrs[] = {ctx->d_density,      ctx->d_material,    ctx->d_mass,       ctx->d_edep,
                   ctx->d_s1,           ctx->d_s2,          ctx->d_nhist,      ctx->d_gs,
+                  ctx->d_gs_cells,
                   ctx->d_edges,        ctx->d_cdf,         ctx->d_beamlet,    ctx->d_up_particle,
                   ctx->d_up,           ctx->d_q[0],        ctx->d_q[1],       ctx->d_q[2],
                   ctx->d_q[3],         ctx->d_counts,      ctx->d_ledger,     ctx->d_items,
@@ -1948,9 +2092,14 @@ int hmc_set_gs(hmc_ctx* ctx, const float* values, int n_eta, int n_theta2, int n
     return fail(ctx, HMC_EINVAL, "GS grid needs at least 2x2 nodes");
   HMC_HIP(ctx, hipSetDevice(ctx->device));
   const size_t count = static_cast<size_t>(n_eta) * n_theta2 * n_u;
+  const long long cells = static_cast<long long>(n_eta - 1) * (n_theta2 - 1) * n_u;
   int rc = upload(ctx, &ctx->d_gs, values, count);
+  if (rc == HMC_OK) rc = dev_alloc(ctx, &ctx->d_gs_cells, static_cast<size_t>(cells));
   if (rc) return rc;
-  ctx->t.gs = ctx->d_gs;
+  hipLaunchKernelGGL(k_gs_cells, dim3(blocks_for(cells, 256, 8192)), dim3(256), 0, ctx->stream, ctx->d_gs, n_theta2,
+                     n_u, cells, ctx->d_gs_cells);
+  HMC_HIP(ctx, hipGetLastError());
+  ctx->t.gs = ctx->d_gs_cells;
   ctx->t.gs_ix0 = ix0;
   ctx->t.gs_iy0 = iy0;
   ctx->t.gs_n_eta = n_eta;
@@ -2794,6 +2943,9 @@ static bool fast_rounds(const TransportParams& P) {
 static int enqueue_round_group(hmc_ctx* ctx, const TransportParams& P, unsigned int round_blocks,
                                unsigned int cap, hipEvent_t* events) {
   const bool fast = fast_rounds(P);
+  const bool one = P.t.n_mat == 1 && P.t.n_points <= kTablePoints && small_grid(P.g.nx, P.g.ny, P.g.nz) &&
+                   small_grid(P.s.nx, P.s.ny, P.s.nz);
+  const unsigned int one_blocks = std::max(1u, round_blocks * 256u / kElectronThreads<true>);
   unsigned int* counts = ctx->d_counts;
   unsigned int* heads = ctx->d_counts + 4;
   int pa = 0, ea = 1, pb = 2, eb = 3;
@@ -2833,12 +2985,18 @@ static int enqueue_round_group(hmc_ctx* ctx, const TransportParams& P, unsigned 
       head_e = heads + pa;
     }
     if (ev) HMC_HIP(ctx, hipEventRecord(ev[2], ctx->stream));
-    if (fast)
-      hipLaunchKernelGGL((k_electron_round<true>), dim3(round_blocks), dim3(256), 0, ctx->stream, P, qin_e,
-                         head_e, qb_p, qb_e);
+    if (one && fast)
+      hipLaunchKernelGGL((k_electron_round<true, true>), dim3(one_blocks), dim3(kElectronThreads<true>), 0,
+                         ctx->stream, P, qin_e, head_e, qb_p, qb_e);
+    else if (one)
+      hipLaunchKernelGGL((k_electron_round<false, true>), dim3(one_blocks), dim3(kElectronThreads<true>), 0,
+                         ctx->stream, P, qin_e, head_e, qb_p, qb_e);
+    else if (fast)
+      hipLaunchKernelGGL((k_electron_round<true, false>), dim3(round_blocks), dim3(kElectronThreads<false>), 0,
+                         ctx->stream, P, qin_e, head_e, qb_p, qb_e);
     else
-      hipLaunchKernelGGL((k_electron_round<false>), dim3(round_blocks), dim3(256), 0, ctx->stream, P, qin_e,
-                         head_e, qb_p, qb_e);
+      hipLaunchKernelGGL((k_electron_round<false, false>), dim3(round_blocks), dim3(kElectronThreads<false>), 0,
+                         ctx->stream, P, qin_e, head_e, qb_p, qb_e);
     HMC_HIP(ctx, hipGetLastError());
     if (ev) HMC_HIP(ctx, hipEventRecord(ev[3], ctx->stream));
     hipLaunchKernelGGL(k_reset_consumed, dim3(1), dim3(64), 0, ctx->stream, counts, heads, pa, ea, cap,
