@@ -65,7 +65,7 @@ int hdn_conv3d_wgrad(const void* x_cm, const void* dz_cm, float* part, int split
 int hdn_conv3d_wgrad_noalloc(const void* x_cm, const void* dz_cm, float* grad, int splits, int n,
                              int d, int h, int w_, int cin, int cout, void* stream);
 
-/* out[i] = sum over s of part[s][i], in split order (deterministic). */
+/* out[i] = sum over s of part[s][i], in a fixed order (deterministic). */
 int hdn_reduce_splits(const float* part, float* out, long long len, int splits, void* stream);
 
 /* Per-channel sums of a channel-major tensor over its P positions: part[splits][C]. */

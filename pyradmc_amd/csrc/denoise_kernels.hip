@@ -166,6 +166,135 @@ __global__ void __launch_bounds__(256) k_conv_fwd(const __bf16* __restrict__ x,
   }
 }
 
+// The same convolution where 64-position waves are too few to fill the chip (the deep
+// levels of a small batch): the kNW waves of a workgroup take the k-steps of one 64-position
+// block in turn, each loading its next step's operands before this step's MFMAs, and
+// their sums add in a fixed tree through LDS. Four 8^3 volumes of 128 -> 128 channels:
+// 130 us as one wave per block (108 k-steps, each waiting for its loads), 22 us split;
+// 16^3, 64 -> 64: 67 and 28 us.
+constexpr int kSplitWaves = 8;
+
+template <int TM, int SRC>
+__global__ void __launch_bounds__(64 * kSplitWaves) k_conv_fwd_split(
+    const __bf16* __restrict__ x, const __bf16* __restrict__ x2, const __bf16* __restrict__ wt,
+    const float* __restrict__ bias, __bf16* __restrict__ y_nd, __bf16* __restrict__ y_cm, int n, int d, int h, int w,
+    int cin, int cout, float slope) {
+  __shared__ f32x4 sums[kSplitWaves / 2][TM * 4][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const long long P = static_cast<long long>(n) * d * h * w;
+  const long long p0 = static_cast<long long>(blockIdx.x) * 64;
+  const int co0 = blockIdx.y * 16 * TM;
+  const int col = lane & 15;
+  const int kg = lane >> 4;
+
+  int pn[4], pz[4], py[4], px[4];
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb) {
+    long long t = p0 + 16 * nb + col;
+    px[nb] = static_cast<int>(t % w);
+    t /= w;
+    py[nb] = static_cast<int>(t % h);
+    t /= h;
+    pz[nb] = static_cast<int>(t % d);
+    pn[nb] = static_cast<int>(t / d);
+  }
+
+  f32x4 acc[TM][4];
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) acc[m][nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  const int kc = SRC == kSrcLow8 ? 8 : cin;  // channels read per tap
+  const int K = 27 * kc;
+  // Operands of k-step k0 (zero past K). A position outside the volume reads the tensor's
+  // first element, always valid, and is replaced by zero.
+  auto load = [&](int k0, bf16x8 (&a)[TM], bf16x8 (&b)[4]) {
+    const int k = k0 + 8 * kg;
+    const bool in = k < K;
+    const int tap = in ? k / kc : 0;
+    const int c = in ? k - tap * kc : 0;
+    const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
+#pragma unroll
+    for (int m = 0; m < TM; ++m) {
+      a[m] = load8(wt + (static_cast<long long>(tap) * cout + co0 + 16 * m + col) * cin + c);
+      if (!in) a[m] = zero8();
+    }
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) {
+      const int zz = pz[nb] + dz, yy = py[nb] + dy, xx = px[nb] + dx;
+      const bool ok = in && zz >= 0 && zz < d && yy >= 0 && yy < h && xx >= 0 && xx < w;
+      long long q;
+      if constexpr (SRC == kSrcUp)
+        q = ((static_cast<long long>(pn[nb]) * (d >> 1) + (zz >> 1)) * (h >> 1) + (yy >> 1)) * (w >> 1) + (xx >> 1);
+      else
+        q = ((static_cast<long long>(pn[nb]) * d + zz) * h + yy) * w + xx;
+      q = ok ? q * cin + c : 0;
+      b[nb] = load8(x + q);
+      if constexpr (SRC == kSrcAdd) b[nb] = add8(b[nb], load8(x2 + q));
+      if (!ok) b[nb] = zero8();
+    }
+  };
+  auto mfmas = [&](const bf16x8 (&a)[TM], const bf16x8 (&b)[4]) {
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) acc[m][nb] = mfma16(a[m], b[nb], acc[m][nb]);
+  };
+  constexpr int kStep = 32 * kSplitWaves;
+  bf16x8 a0[TM], a1[TM], b0[4], b1[4];
+  int k0 = 32 * wave;
+  load(k0, a0, b0);
+  for (; k0 < K; k0 += 2 * kStep) {
+    load(k0 + kStep, a1, b1);
+    mfmas(a0, b0);
+    if (k0 + kStep >= K) break;
+    load(k0 + 2 * kStep, a0, b0);
+    mfmas(a1, b1);
+  }
+
+  for (int half = kSplitWaves / 2; half >= 1; half >>= 1) {
+    if (wave >= half && wave < 2 * half) {
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) sums[wave - half][4 * m + nb][lane] = acc[m][nb];
+    }
+    __syncthreads();
+    if (wave < half) {
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) acc[m][nb] += sums[wave][4 * m + nb][lane];
+    }
+    __syncthreads();
+  }
+  if (wave != 0) return;
+
+#pragma unroll
+  for (int m = 0; m < TM; ++m) {
+    const int cb = co0 + 16 * m + 4 * kg;
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) {
+      const long long p = p0 + 16 * nb + col;
+      __bf16 out[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float v = acc[m][nb][r] + (bias ? bias[cb + r] : 0.0f);
+        out[r] = static_cast<__bf16>(act(v, slope));
+      }
+      uint2 packed;
+      std::memcpy(&packed, out, 8);
+      *reinterpret_cast<uint2*>(y_nd + p * cout + cb) = packed;
+      if (y_cm) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y_cm[static_cast<long long>(cb + r) * P + p] = out[r];
+      }
+    }
+  }
+}
+
 // The same convolution for rows of KW = 64 or 32 voxels (w == KW, h % (256 / KW) == 0,
 // cout 16 x TM): a workgroup computes 256 / KW consecutive h-rows of one z-slice (256
 // positions; each wave 64 of them) and first stages the input those rows read - 3 z x
@@ -356,14 +485,53 @@ __device__ inline bf16x8 load_row8(const __bf16* row, int x0, int w, int dx) {
   return r;
 }
 
+// A workgroup's weight-gradient block: the four waves' accumulators added in wave order,
+// nine taps at a time through LDS, and written by the first wave.
+// D[i = ci][j = co]: a lane holds ci = ci0 + 4 kg + r, co = co0 + col.
+__device__ inline void store_wgrad(const f32x4 (&acc)[27], float4 (*sums)[9][64], float* out, int ci0, int co0,
+                                   int cin, int cout) {
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int t0 = 0; t0 < 27; t0 += 9) {
+    __syncthreads();
+    if (wave > 0) {
+#pragma unroll
+      for (int t = 0; t < 9; ++t)
+        sums[wave - 1][t][lane] = make_float4(acc[t0 + t][0], acc[t0 + t][1], acc[t0 + t][2], acc[t0 + t][3]);
+    }
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll
+      for (int t = 0; t < 9; ++t) {
+        float4 v = make_float4(acc[t0 + t][0], acc[t0 + t][1], acc[t0 + t][2], acc[t0 + t][3]);
+#pragma unroll
+        for (int w = 0; w < 3; ++w) {
+          const float4 o = sums[w][t][lane];
+          v.x += o.x;
+          v.y += o.y;
+          v.z += o.z;
+          v.w += o.w;
+        }
+        *reinterpret_cast<float4*>(out + (static_cast<long long>(t0 + t) * cout + co0 + (lane & 15)) * cin + ci0 +
+                                   4 * (lane >> 4)) = v;
+      }
+    }
+  }
+}
+
 // Weight-gradient partials: part[s][tap][co][ci] = sum over split s's positions of
-// dz[p][co] x[p + off(tap)][ci]. One wave owns one 16x16 (ci, co) block for all 27
-// taps (108 accumulators) and a contiguous range of positions, in chunks of 32.
-__global__ void __launch_bounds__(64) k_conv_wgrad(const __bf16* __restrict__ x_cm,
+// dz[p][co] x[p + off(tap)][ci]. A workgroup owns one 16x16 (ci, co) block for all 27
+// taps (108 accumulators a lane) and a contiguous range of positions, which its four waves
+// take in chunks of 32; their sums add in wave order (add_waves). For rows that
+// k_conv_wgrad_tile does not take.
+__global__ void __launch_bounds__(256) k_conv_wgrad(const __bf16* __restrict__ x_cm,
                                                    const __bf16* __restrict__ dz_cm,
                                                    float* __restrict__ part, int n, int d, int h,
                                                    int w, int cin, int cout, long long per_split) {
-  const int lane = threadIdx.x;
+  __shared__ float4 sums[3][9][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
   const int col = lane & 15;
   const int kg = lane >> 4;
   const int ci0 = 16 * blockIdx.x;
@@ -379,7 +547,7 @@ __global__ void __launch_bounds__(64) k_conv_wgrad(const __bf16* __restrict__ x_
 
   const __bf16* xrow_c = x_cm + static_cast<long long>(ci0 + col) * P;
   const __bf16* dz_c = dz_cm + static_cast<long long>(co0 + col) * P;
-  for (long long pb = pbeg; pb < pend; pb += 32) {
+  for (long long pb = pbeg + 32 * wave; pb < pend; pb += 128) {
     const long long p = pb + 8 * kg;  // this lane's 8 positions: one aligned W-row segment
     const bf16x8 b = load8(dz_c + p);
     long long t = p;
@@ -405,24 +573,149 @@ __global__ void __launch_bounds__(64) k_conv_wgrad(const __bf16* __restrict__ x_
       }
     }
   }
-  // D[i = ci][j = co]: lane holds ci = ci0 + 4 kg + r, co = co0 + col.
-  float* out = part + static_cast<long long>(split) * 27 * cout * cin;
-#pragma unroll
-  for (int tap = 0; tap < 27; ++tap) {
-    float4 v = make_float4(acc[tap][0], acc[tap][1], acc[tap][2], acc[tap][3]);
-    *reinterpret_cast<float4*>(out + (static_cast<long long>(tap) * cout + co0 + col) * cin + ci0 +
-                               4 * kg) = v;
-  }
+  store_wgrad(acc, sums, part + static_cast<long long>(split) * 27 * cout * cin, ci0, co0, cin, cout);
 }
 
-// out[i] = sum_s part[s][i], in split order (deterministic).
-__global__ void k_reduce_splits(const float* __restrict__ part, float* __restrict__ out,
-                                long long len, int splits) {
-  for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < len;
-       i += static_cast<long long>(gridDim.x) * blockDim.x) {
+// The same partials for rows of W = 64, 32 or 16 voxels (w == W, h % (256 / W) == 0): a
+// workgroup takes tiles of 256 positions (256 / W rows of one z-slice; each wave 64 of
+// them) and stages the 16 input channels' rows of a tile - 3 z x (rows + 2) h, zero
+// outside the volume - in LDS, so an element is loaded 4.5 times (W = 64) instead of 27,
+// in runs of whole rows. The rows of one channel-major tensor lie the channel stride
+// apart (2 MiB at 128^3 voxels), so gathering a tap's 16 channels straight from memory sent
+// every load of a wave to one L2 channel. Rows are 8 elements longer than W: the zeros
+// beyond both row ends, read by the +-1 shifts. The channel stride is an odd number of
+// 16-byte units, so that 16 channels' reads spread over the banks. The next tile's loads
+// are issued before this tile's products and stored to LDS after them.
+// Four 64^3 volumes of 16 -> 16 channels: 172 us gathered, 57 us staged; 32^3, 64 -> 32:
+// 158 and 50 us.
+template <int W>
+__global__ void __launch_bounds__(256, 2) k_conv_wgrad_tile(const __bf16* __restrict__ x_cm,
+                                                         const __bf16* __restrict__ dz_cm,
+                                                         float* __restrict__ part, int n, int d, int h, int cin,
+                                                         int cout, int splits) {
+  constexpr int kRows = 256 / W, kTH = kRows + 2, kStride = W + 8, kChannel = 3 * kTH * kStride + 8;
+  constexpr int kUnits = 16 * 3 * kTH * (W / 8);  // 16-byte units of a tile
+  constexpr int kPer = (kUnits + 255) / 256;
+  static_assert(kChannel % 16 == 8, "the channel stride is an odd number of 16-byte units");
+  constexpr int kSumBytes = 3 * 9 * 64 * static_cast<int>(sizeof(float4));
+  constexpr int kBytes = 16 * kChannel * 2 > kSumBytes ? 16 * kChannel * 2 : kSumBytes;
+  __shared__ __align__(16) unsigned char lds[kBytes];
+  __bf16* tile = reinterpret_cast<__bf16*>(lds);
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int col = lane & 15;
+  const int kg = lane >> 4;
+  const int ci0 = 16 * blockIdx.x;
+  const int co0 = 16 * blockIdx.y;
+  const int split = blockIdx.z;
+  const int rows = h / kRows;
+  const long long P = static_cast<long long>(n) * d * h * W;
+  const long long tiles = P / 256;
+  const long long t_beg = tiles * split / splits, t_end = tiles * (split + 1) / splits;
+
+  for (int i = threadIdx.x; i < kBytes / 16; i += 256)  // row ends (and all else) start as zeros
+    reinterpret_cast<u32x4*>(lds)[i] = u32x4{0u, 0u, 0u, 0u};
+
+  u32x4 next[kPer];
+  bf16x8 dz_next[2];
+  auto load_tile = [&](long long t) {
+    const int hb = static_cast<int>(t % rows);
+    const long long zt = t / rows;
+    const int z = static_cast<int>(zt % d);
+    const long long nn = zt / d;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const int i = static_cast<int>(threadIdx.x) + 256 * j;
+      const int x8 = i % (W / 8), row = (i / (W / 8)) % (3 * kTH), ch = i / (W / 8 * 3 * kTH);
+      const int gz = z + row / kTH - 1, gy = hb * kRows + row % kTH - 1;
+      const bool ok = i < kUnits && gz >= 0 && gz < d && gy >= 0 && gy < h;
+      // An element outside the volume reads the tensor's first one, always valid.
+      const long long at = ok ? static_cast<long long>(ci0 + ch) * P + ((nn * d + gz) * h + gy) * W + 8 * x8 : 0;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(x_cm + at);
+      next[j] = ok ? v : u32x4{0u, 0u, 0u, 0u};
+    }
+    const __bf16* dz = dz_cm + static_cast<long long>(co0 + col) * P + t * 256 + 64 * wave + 8 * kg;
+    dz_next[0] = load8(dz);
+    dz_next[1] = load8(dz + 32);
+  };
+  auto store_tile = [&]() {
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const int i = static_cast<int>(threadIdx.x) + 256 * j;
+      const int x8 = i % (W / 8), row = (i / (W / 8)) % (3 * kTH), ch = i / (W / 8 * 3 * kTH);
+      if (i < kUnits) *reinterpret_cast<u32x4*>(tile + ch * kChannel + row * kStride + 8 + 8 * x8) = next[j];
+    }
+  };
+
+  f32x4 acc[27];
+#pragma unroll
+  for (int t = 0; t < 27; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  if (t_beg < t_end) load_tile(t_beg);
+  for (long long t = t_beg; t < t_end; ++t) {
+    __syncthreads();  // the previous tile's reads (or the clearing) are done
+    store_tile();
+    const bf16x8 dz[2] = {dz_next[0], dz_next[1]};
+    __syncthreads();
+    if (t + 1 < t_end) load_tile(t + 1);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int p = 64 * wave + 32 * c + 8 * kg;  // this lane's 8 positions of the tile
+      const __bf16* base = tile + col * kChannel + (p / W) * kStride + 8 + p % W;
+#pragma unroll
+      for (int zy = 0; zy < 9; ++zy) {
+        const __bf16* q = base + ((zy / 3) * kTH + zy % 3) * kStride;
+        const u32x4 cur = *reinterpret_cast<const u32x4*>(q);
+        const unsigned int before = *reinterpret_cast<const unsigned int*>(q - 2);
+        const unsigned int after = *reinterpret_cast<const unsigned int*>(q + 8);
+        u32x4 lo, hi;
+        lo[0] = __builtin_amdgcn_alignbit(cur[0], before, 16);
+        hi[3] = __builtin_amdgcn_alignbit(after, cur[3], 16);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          lo[k + 1] = __builtin_amdgcn_alignbit(cur[k + 1], cur[k], 16);
+          hi[k] = lo[k + 1];
+        }
+        bf16x8 a;
+        std::memcpy(&a, &lo, 16);
+        acc[3 * zy] = mfma16(a, dz[c], acc[3 * zy]);
+        std::memcpy(&a, &cur, 16);
+        acc[3 * zy + 1] = mfma16(a, dz[c], acc[3 * zy + 1]);
+        std::memcpy(&a, &hi, 16);
+        acc[3 * zy + 2] = mfma16(a, dz[c], acc[3 * zy + 2]);
+      }
+    }
+  }
+  store_wgrad(acc, reinterpret_cast<float4(*)[9][64]>(lds), part + static_cast<long long>(split) * 27 * cout * cin,
+              ci0, co0, cin, cout);
+}
+
+// out[i] = sum_s part[s][i] in a fixed order: wave g of a workgroup adds splits g,
+// g + 16, ... of 64 outputs, eight loads in flight, and the 16 waves' sums add in wave
+// order. One thread per output, as before, left 27 waves to walk 2048 splits one load at a
+// time: 470 us for 56 MB; 9 us now for the 21 MB that k_conv_wgrad_tile's splits leave.
+constexpr int kReduceWaves = 16;
+
+__global__ void __launch_bounds__(64 * kReduceWaves) k_reduce_splits(const float* __restrict__ part,
+                                                                     float* __restrict__ out, long long len,
+                                                                     int splits) {
+  __shared__ float sums[kReduceWaves][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  for (long long i0 = static_cast<long long>(blockIdx.x) * 64; i0 < len; i0 += static_cast<long long>(gridDim.x) * 64) {
+    const long long i = i0 + lane;
     float s = 0.0f;
-    for (int k = 0; k < splits; ++k) s += part[static_cast<long long>(k) * len + i];
-    out[i] = s;
+    if (i < len) {
+#pragma unroll 8
+      for (int k = wave; k < splits; k += kReduceWaves) s += part[static_cast<long long>(k) * len + i];
+    }
+    sums[wave][lane] = s;
+    __syncthreads();
+    if (wave == 0 && i < len) {
+      for (int g = 1; g < kReduceWaves; ++g) s += sums[g][lane];
+      out[i] = s;
+    }
+    __syncthreads();
   }
 }
 
@@ -702,6 +995,12 @@ extern "C" {
 
 namespace {
 
+// Below this many 64-position waves the k-steps are split over workgroups
+// (k_conv_fwd_split). Whole and split, us: 64 waves 125 and 22 (8^3 x 4, 128 -> 128),
+// 256 waves 66 and 27 (16^3 x 4, 64 -> 64), 768 waves 67 and 68 (12 x 8 x 8 x 32,
+// 64 -> 128), 1024 waves 37 and 52 (32^3 x 2, 32 -> 64).
+constexpr long long kFillWaves = 768;
+
 template <int SRC>
 int conv_fwd(const __bf16* xb, const __bf16* x2b, const __bf16* wb, const float* bias, __bf16* yb, __bf16* cb,
              int n, int d, int h, int w, int cin, int cout, float slope, hipStream_t stream) {
@@ -735,6 +1034,18 @@ int conv_fwd(const __bf16* xb, const __bf16* x2b, const __bf16* wb, const float*
   }
   const long long P = static_cast<long long>(n) * d * h * w;
   const int tm = cout % 64 == 0 ? 4 : (cout % 32 == 0 ? 2 : 1);
+  // Fewer waves than kFillWaves leave SIMDs idle or waiting for loads: split the k-steps.
+  if (P / 64 * (cout / (16 * tm)) < kFillWaves) {
+    const int ts = cout % 32 == 0 ? 2 : 1;
+    const dim3 blocks(static_cast<unsigned int>(P / 64), static_cast<unsigned int>(cout / (16 * ts)));
+    if (ts == 2)
+      hipLaunchKernelGGL((k_conv_fwd_split<2, SRC>), blocks, dim3(64 * kSplitWaves), 0, stream, xb, x2b, wb, bias, yb,
+                         cb, n, d, h, w, cin, cout, slope);
+    else
+      hipLaunchKernelGGL((k_conv_fwd_split<1, SRC>), blocks, dim3(64 * kSplitWaves), 0, stream, xb, x2b, wb, bias, yb,
+                         cb, n, d, h, w, cin, cout, slope);
+    return launch_status();
+  }
   const dim3 grid(static_cast<unsigned int>((P + 255) / 256), static_cast<unsigned int>(cout / (16 * tm)));
   if (tm == 4)
     hipLaunchKernelGGL((k_conv_fwd<4, SRC>), grid, dim3(256), 0, stream, xb, x2b, wb, bias, yb, cb, n, d, h, w,
@@ -772,13 +1083,21 @@ void launch_wgrad(const void* x_cm, const void* dz_cm, float* part, int splits, 
                   int w, int cin, int cout, long long per_split, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned int>(cin / 16), static_cast<unsigned int>(cout / 16),
                   static_cast<unsigned int>(splits));
-  hipLaunchKernelGGL(k_conv_wgrad, grid, dim3(64), 0, stream, static_cast<const __bf16*>(x_cm),
-                     static_cast<const __bf16*>(dz_cm), part, n, d, h, w, cin, cout, per_split);
+  const __bf16* xb = static_cast<const __bf16*>(x_cm);
+  const __bf16* db = static_cast<const __bf16*>(dz_cm);
+  if (w == 64 && h % 4 == 0)
+    hipLaunchKernelGGL(k_conv_wgrad_tile<64>, grid, dim3(256), 0, stream, xb, db, part, n, d, h, cin, cout, splits);
+  else if (w == 32 && h % 8 == 0)
+    hipLaunchKernelGGL(k_conv_wgrad_tile<32>, grid, dim3(256), 0, stream, xb, db, part, n, d, h, cin, cout, splits);
+  else if (w == 16 && h % 16 == 0)
+    hipLaunchKernelGGL(k_conv_wgrad_tile<16>, grid, dim3(256), 0, stream, xb, db, part, n, d, h, cin, cout, splits);
+  else
+    hipLaunchKernelGGL(k_conv_wgrad, grid, dim3(256), 0, stream, xb, db, part, n, d, h, w, cin, cout, per_split);
 }
 
 void launch_reduce(const float* part, float* out, long long len, int splits, hipStream_t stream) {
-  const unsigned int blocks = static_cast<unsigned int>(std::min<long long>(blocks_for(len, 256), 65535));
-  hipLaunchKernelGGL(k_reduce_splits, dim3(blocks), dim3(256), 0, stream, part, out, len, splits);
+  const unsigned int blocks = static_cast<unsigned int>(std::min<long long>(blocks_for(len, 64), 65535));
+  hipLaunchKernelGGL(k_reduce_splits, dim3(blocks), dim3(64 * kReduceWaves), 0, stream, part, out, len, splits);
 }
 
 // Device address of `scratch` on each GPU, looked up once per device with that device

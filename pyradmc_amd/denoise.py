@@ -336,7 +336,11 @@ class Conv3dDenoiser:
             _call("hdn_act_bwd", _ptr(y), _ptr(dy), _ptr(dz_nd), _ptr(dz_cm), P, lay.cout, SLOPE,
                   self._stream())
         # weight and bias gradients (deterministic split reductions)
-        splits = max(1, min(P // 512, 2048 // max(1, (lay.cin // 16) * (lay.cout // 16))))
+        # about three workgroups of four waves per CU over all 16 x 16 channel blocks, each
+        # split owning a whole number of 32-position chunks
+        splits = max(1, min(P // 512, 768 // max(1, (lay.cin // 16) * (lay.cout // 16))))
+        per_split = -(-P // (32 * splits)) * 32
+        splits = -(-P // per_split)
         part = torch.empty((splits, 27, lay.cout, lay.cin), dtype=torch.float32, device=y.device)
         _call("hdn_conv3d_wgrad", _ptr(inp_cm), _ptr(dz_cm), _ptr(part), splits, n, d, h, w,
               lay.cin, lay.cout, self._stream())

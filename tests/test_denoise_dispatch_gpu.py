@@ -1,0 +1,72 @@
+"""The convolutions' and reductions' kernels at the sizes where their dispatch changes,
+against the float64 oracle on bf16-rounded inputs (tolerances as in
+tests/test_denoise_gpu.py: 2^-8 relative for a bf16 output, 1e-4 for float32 sums)."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from oracle import conv_ref as cr
+from tests.test_denoise_gpu import _bf, _close_bf16, _cm, _dev, _np, _rounded, dn  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+# Weight gradients: rows of 64, 32 and 16 in whole tiles (several per split, one, and
+# fewer tiles than splits: some partials are zeros), a tile height that does not divide h
+# and short rows (the general kernel), with position counts off the splits' multiples.
+@pytest.mark.parametrize("shape, cin, cout, splits", [
+    ((1, 2, 4, 64), 16, 16, 1), ((1, 5, 8, 64), 16, 32, 3), ((2, 3, 4, 64), 32, 16, 16),
+    ((1, 1, 8, 32), 16, 16, 1), ((2, 3, 16, 32), 32, 32, 5), ((1, 3, 16, 16), 64, 16, 2),
+    ((2, 2, 32, 16), 16, 48, 7), ((1, 3, 6, 64), 16, 16, 4), ((1, 5, 8, 8), 16, 32, 3),
+])
+def test_weight_gradient_tiles(dn, shape, cin, cout, splits):  # noqa: F811
+    import torch
+
+    rng = np.random.default_rng(cin + cout + splits)
+    n, d, h, w = shape
+    x, dz = _rounded(rng.standard_normal(shape + (cin,))), _rounded(rng.standard_normal(shape + (cout,)))
+    x_cm, dz_cm = _cm(_dev(_bf(x)), cin), _cm(_dev(_bf(dz)), cout)
+    part = torch.full((splits, 27, cout, cin), float("nan"), dtype=torch.float32, device="cuda:0")
+    gw = torch.empty((27, cout, cin), dtype=torch.float32, device="cuda:0")
+    dn._call("hdn_conv3d_wgrad", x_cm.data_ptr(), dz_cm.data_ptr(), part.data_ptr(), splits, n, d, h, w, cin, cout,
+             None)
+    dn._call("hdn_reduce_splits", part.data_ptr(), gw.data_ptr(), gw.numel(), splits, None)
+    ref = cr.conv_wgrad(x, dz)
+    np.testing.assert_allclose(_np(gw), ref, rtol=1e-4, atol=1e-4 * np.abs(ref).max())
+
+
+# Forward convolutions just below and at the wave count from which one wave takes a whole
+# 64-position block: the k-steps split over a workgroup, and not; few and many k-steps.
+@pytest.mark.parametrize("shape, cin, cout", [
+    ((1, 1, 4, 16), 128, 128), ((3, 5, 8, 8), 128, 64), ((1, 8, 8, 8), 16, 48),
+    ((3, 15, 32, 32), 16, 16), ((3, 16, 32, 32), 16, 16),
+])
+def test_forward_split_and_whole(dn, shape, cin, cout):  # noqa: F811
+    import torch
+
+    rng = np.random.default_rng(cin + cout)
+    n, d, h, w = shape
+    x = _rounded(rng.standard_normal(shape + (cin,)))
+    master = rng.standard_normal((27, cout, cin)).astype(np.float32) * 0.1
+    bias = rng.standard_normal(cout).astype(np.float32)
+    wq = _rounded(master)
+    xd, wf, bd = _dev(_bf(x)), _dev(_bf(wq)), _dev(torch.from_numpy(bias))
+    y = torch.empty(shape + (cout,), dtype=torch.bfloat16, device="cuda:0")
+    y_cm = torch.empty((cout, n * d * h * w), dtype=torch.bfloat16, device="cuda:0")
+    dn._call("hdn_conv3d_fwd", xd.data_ptr(), wf.data_ptr(), bd.data_ptr(), y.data_ptr(), y_cm.data_ptr(), n, d, h, w,
+             cin, cout, 0.1, None)
+    _close_bf16(_np(y), cr.leaky(cr.conv_fwd(x, wq, bias.astype(np.float64)), 0.1))
+    np.testing.assert_array_equal(_np(y_cm), _np(y).reshape(-1, cout).T)
+
+
+@pytest.mark.parametrize("splits, length", [(1, 5), (16, 64), (17, 65), (700, 6912)])
+def test_reduce_splits(dn, splits, length):  # noqa: F811
+    import torch
+
+    part = torch.rand((splits, length), device="cuda:0")
+    out = torch.empty(length, device="cuda:0")
+    dn._call("hdn_reduce_splits", part.data_ptr(), out.data_ptr(), length, splits, None)
+    # float32 sums of positive terms: at most one rounding of each partial sum per term
+    np.testing.assert_allclose(_np(out), part.double().sum(dim=0).cpu().numpy(), rtol=(splits + 1) * 2.0 ** -24)
