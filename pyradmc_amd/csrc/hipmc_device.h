@@ -276,13 +276,14 @@ __device__ inline void rotate(float& ux, float& uy, float& uz, float cos_t, floa
   }
 }
 
-// Photon channel from the four attenuation coefficients with one uniform, in the order
-// Compton, photoelectric, pair, Rayleigh (pyradmc/physics/channel.py:17-60).
-__device__ inline int select_process(float mu_c, float mu_p, float mu_pp, float mu_r, uint64_t& rng) {
-  const float threshold = uniform(rng) * (mu_c + mu_p + mu_pp + mu_r);
-  if (threshold < mu_c) return COMPTON;
-  if (threshold < mu_c + mu_p) return PHOTOELECTRIC;
-  if (threshold < mu_c + mu_p + mu_pp) return PAIR;
+// Photon channel with one uniform from the running sums of the four attenuation
+// coefficients in the order Compton, photoelectric, pair, Rayleigh
+// (pyradmc/physics/channel.py:17-60).
+__device__ inline int select_process(float mu1, float mu2, float mu3, float mu_total, uint64_t& rng) {
+  const float threshold = uniform(rng) * mu_total;
+  if (threshold < mu1) return COMPTON;
+  if (threshold < mu2) return PHOTOELECTRIC;
+  if (threshold < mu3) return PAIR;
   return RAYLEIGH;
 }
 

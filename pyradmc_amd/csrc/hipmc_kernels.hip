@@ -484,18 +484,37 @@ __device__ inline bool enter_grid(const DevGrid& g, float& x, float& y, float& z
 // round gained nothing from the same rule).
 constexpr int kRefillIdleLanes = 16;
 
+// Largest table of the kOne builds (tables of one material in LDS).
+constexpr int kTablePoints = 2048;
+
+// Lanes of a wave in the photon round that make a refill, or a pass over the real
+// interactions, worth its instructions.
+constexpr int kPhotonBatch = 24;
+
 // Energy bins of the electron queue's sort (a quarter octave each above the cutoff),
 // and the blocks that sort it, each over one contiguous range of the queue.
 constexpr int kEnergyBins = 32;
 constexpr int kSortBlocks = 1024;
 
-template <bool kFast>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HMC_ROUND_WAVES, 8)))
-k_photon_round(TransportParams P, Queue qin,
-                                                      unsigned int* head, Queue qe, Queue qp) {
+template <bool kOne>
+constexpr int kPhotonThreads = kOne ? 768 : 256;
+
+template <bool kOne>
+struct PhotonShared {};
+template <>
+struct PhotonShared<true> {
+  float4 photon[kTablePoints];  // DevTables::photon of the one material
+  float majorant[kTablePoints];
+};
+
+template <bool kFast, bool kOne>
+__global__ void __launch_bounds__(kPhotonThreads<kOne>) __attribute__((amdgpu_waves_per_eu(kOne ? 3 : HMC_ROUND_WAVES, 8)))
+k_photon_round(TransportParams P, Queue qin, unsigned int* head, Queue qe, Queue qp) {
+  __shared__ PhotonShared<kOne> sh;
   const unsigned int n_in = min(*qin.count, qin.capacity);
   LaneTally tal;
-  bool active = false;
+  bool flying = false;  // on a Woodcock flight
+  bool hit = false;     // at a real interaction, not yet made
   float x = 0, y = 0, z = 0, e = 0, ux = 0, uy = 0, uz = 1, w = 0;
   uint64_t rng = 0;
   uint32_t column = 0;
@@ -503,6 +522,10 @@ k_photon_round(TransportParams P, Queue qin,
   float mu_maj = 0.0f;
   int pi = 0;
   float pw = 0.0f;
+  float4 c = make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // compton, photo, pair, rayleigh of the last voxel's material
+  // Running sums of the channels' attenuation at the last voxel, in channel order.
+  float mu1 = 0.0f, mu2 = 0.0f, mu3 = 0.0f, mu_real = 0.0f;
+  int mat = 0;
   int steps = 0;
   const int n = P.t.n_points;
 
@@ -515,139 +538,162 @@ k_photon_round(TransportParams P, Queue qin,
   qp.lds = 1;
   if (qe.push_chunk == 0u) qe.push_chunk = qp.push_chunk = sized_push_chunk(n_in, qe.capacity);
   RefillPool pool(P.refill_block, n_in);
+  if constexpr (kOne) {
+    if (blockIdx.x * pool.block < n_in) {  // else no wave of the block has work
+      for (int k = static_cast<int>(threadIdx.x); k < n; k += kPhotonThreads<kOne>) {
+        sh.photon[k] = P.t.photon[k];
+        sh.majorant[k] = P.t.majorant[k];
+      }
+    }
+    __syncthreads();
+  }
+  auto spr_of = [&](float energy) { return kOne ? 1.0f : spr<kFast>(P, energy, mat); };
+  // Table position, majorant and (one material) coefficients at the photon's energy.
+  auto at_energy = [&]() {
+    grid_locate(__logf(e), P.t.p_log_min, P.t.p_inv_dlog, n, pi, pw);
+    if constexpr (kOne) {
+      mu_maj = lerp1(sh.majorant, pi, pw);
+      c = lerp4(sh.photon, pi, pw);
+    } else {
+      mu_maj = lerp1(P.t.majorant, pi, pw);
+    }
+  };
+  bool exhausted = false;  // this wave's claims lie beyond the queue
   while (true) {
-    const unsigned int i = refill_index(pool, head, !active);
-    if (!active) {
-      if (i >= n_in) break;
-      uint32_t meta;
-      load_particle(qin.data, i, x, y, z, e, ux, uy, uz, w, rng, meta);
-      const bool real = (meta & 3u) != kEmptyKind;  // else padding left by a producer wave
-      count_pops(real);
-      if (!real) continue;
-      column = meta >> 3;
-      base = static_cast<long long>(column) * P.s.n_voxels;
-      if (!enter_grid(P.g, x, y, z, ux, uy, uz)) {
+    const unsigned int n_idle = static_cast<unsigned int>(__popcll(__ballot(!flying && !hit ? 1 : 0)));
+    if (n_idle >= static_cast<unsigned int>(kPhotonBatch) && !exhausted) {
+      const bool idle = !flying && !hit;
+      const unsigned int i = refill_index(pool, head, idle);
+      exhausted = __ballot(idle && i >= n_in ? 1 : 0) != 0ull;
+      if (idle && i < n_in) {
+        uint32_t meta;
+        load_particle(qin.data, i, x, y, z, e, ux, uy, uz, w, rng, meta);
+        const bool real = (meta & 3u) != kEmptyKind;  // else padding left by a producer wave
+        count_pops(real);
+        if (real) {
+          column = meta >> 3;
+          base = static_cast<long long>(column) * P.s.n_voxels;
+          if (!enter_grid(P.g, x, y, z, ux, uy, uz)) {
+            escape(tal, w * e);
+          } else {
+            flying = true;
+            steps = 0;
+            at_energy();
+          }
+        }
+      }
+    } else if (n_idle == 64u) {
+      break;
+    }
+    if (flying) do {
+      tal.steps++;
+      if (++steps > P.max_steps) {
+        atomicAdd(P.ledger + L_TRAPPED, 1ull);
         escape(tal, w * e);
-        continue;
+        flying = false;
+        break;
       }
-      active = true;
-      steps = 0;
-      grid_locate(__logf(e), P.t.p_log_min, P.t.p_inv_dlog, n, pi, pw);
-      mu_maj = lerp1(P.t.majorant, pi, pw);
-    }
-    tal.steps++;
-    if (++steps > P.max_steps) {
-      atomicAdd(P.ledger + L_TRAPPED, 1ull);
-      escape(tal, w * e);
-      active = false;
-      continue;
-    }
+      const float step = sample_path(mu_maj, rng);
+      x += step * ux;
+      y += step * uy;
+      z += step * uz;
+      if (!inside_grid(P.g, x, y, z)) {
+        escape(tal, w * e);
+        flying = false;
+        break;
+      }
+      const long long vox = grid_index<kOne>(P.g, x, y, z);
+      const float rho = P.g.density[vox];
+      tal.vox++;
+      if constexpr (!kOne) {
+        mat = P.g.material[vox];
+        c = lerp4(P.t.photon + static_cast<long long>(mat) * n, pi, pw);
+      }
+      mu1 = rho * c.x;
+      mu2 = mu1 + rho * c.y;
+      mu3 = mu2 + rho * c.z;
+      mu_real = mu3 + rho * c.w;
+      if (mu_real > mu_maj) {
+        atomicAdd(P.ledger + L_VIOLATIONS, 1ull);
+        escape(tal, w * e);
+        flying = false;
+        break;
+      }
+      hit = uniform(rng) * mu_maj < mu_real;  // else delta scattering
+      flying = !hit;
+    } while (false);
 
-    const float step = sample_path(mu_maj, rng);
-    x += step * ux;
-    y += step * uy;
-    z += step * uz;
-    if (!inside_grid(P.g, x, y, z)) {
-      escape(tal, w * e);
-      active = false;
-      continue;
-    }
-    const int ix = axis_index(x, P.g.x_lo, P.g.inv_sx, P.g.nx);
-    const int iy = axis_index(y, P.g.y_lo, P.g.inv_sy, P.g.ny);
-    const int iz = axis_index(z, P.g.z_lo, P.g.inv_sz, P.g.nz);
-    const long long vox = (static_cast<long long>(ix) * P.g.ny + iy) * P.g.nz + iz;
-    const float rho = P.g.density[vox];
-    const int mat = P.g.material[vox];
-    tal.vox++;
-    const float4 c = lerp4(P.t.photon + static_cast<long long>(mat) * n, pi, pw);
-    const float mu_c = rho * c.x;
-    const float mu_p = rho * c.y;
-    const float mu_pp = rho * c.z;
-    const float mu_r = rho * c.w;
-    const float mu_real = mu_c + mu_p + mu_pp + mu_r;
-    if (mu_real > mu_maj) {
-      atomicAdd(P.ledger + L_VIOLATIONS, 1ull);
-      escape(tal, w * e);
-      active = false;
-      continue;
-    }
-    if (uniform(rng) * mu_maj >= mu_real) continue;  // delta scattering
+    const unsigned int n_hit = static_cast<unsigned int>(__popcll(__ballot(hit ? 1 : 0)));
+    if (n_hit < static_cast<unsigned int>(kPhotonBatch) && __ballot(flying ? 1 : 0) != 0ull) continue;
+    if (hit) {
+      hit = false;
+      const int process = select_process(mu1, mu2, mu3, mu_real, rng);
 
-    const int process = select_process(mu_c, mu_p, mu_pp, mu_r, rng);
-
-    if (process == RAYLEIGH) {
-      const float cos_r = sample_coherent(P.t, mat, e, rng);
-      const float phi = kTwoPi * uniform(rng);
-      rotate(ux, uy, uz, cos_r, phi);
-    } else if (process == COMPTON) {
-      const float ratio = sample_compton_ratio(e, rng);
-      const float recoil = e * (1.0f - ratio);
-      const float phi = kTwoPi * uniform(rng);
-      if (P.transport_electrons && recoil > P.ecut) {
-        const float ce = compton_electron_cos(e, ratio);
-        float ex = ux, ey = uy, ez = uz;
-        rotate(ex, ey, ez, ce, phi + kPi);
-        const uint64_t child = spawn_stream(rng);
-        push(qe, ELECTRON, column, recoil, w, x, y, z, ex, ey, ez, child);
-      } else {
-        deposit<kFast, false>(P, tal, base, x, y, z, w * recoil,
-                spr<kFast>(P, recoil, mat));
-      }
-      const float cg = compton_cos(e, ratio);
-      rotate(ux, uy, uz, cg, phi);
-      e *= ratio;
-      if (e <= P.pcut) {
-        deposit<kFast, false>(P, tal, base, x, y, z, w * e, spr<kFast>(P, e, mat));
-        active = false;
-        continue;
-      }
-      if (e < kRouletteMeV && w < kRouletteWeightCap) {
-        const float new_w = uniform(rng) < kRouletteSurvival ? w / kRouletteSurvival : 0.0f;
-        escape(tal, (w - new_w) * e);
-        if (new_w == 0.0f) {
-          active = false;
-          continue;
-        }
-        w = new_w;
-      }
-      grid_locate(__logf(e), P.t.p_log_min, P.t.p_inv_dlog, n, pi, pw);
-      mu_maj = lerp1(P.t.majorant, pi, pw);
-    } else if (process == PHOTOELECTRIC) {
-      if (P.transport_electrons && e > P.ecut) {
-        const uint64_t child = spawn_stream(rng);
-        push(qe, ELECTRON, column, e, w, x, y, z, ux, uy, uz, child);
-      } else {
-        deposit<kFast, false>(P, tal, base, x, y, z, w * e, spr<kFast>(P, e, mat));
-      }
-      active = false;
-    } else {  // pair production
-      const float kinetic = e - 2.0f * kElectronMass;
-      const float f_ann = spr<kFast>(P, kElectronMass, mat);
-      if (P.transport_electrons) {
-        const float fraction = uniform(rng);
-        const float share_e = fraction * kinetic;
-        const float share_p = (1.0f - fraction) * kinetic;
-        if (share_e > P.ecut) {
+      if (process == RAYLEIGH) {
+        const float cos_r = sample_coherent(P.t, mat, e, rng);
+        const float phi = kTwoPi * uniform(rng);
+        rotate(ux, uy, uz, cos_r, phi);
+        flying = true;
+      } else if (process == COMPTON) {
+        const float ratio = sample_compton_ratio(e, rng);
+        const float recoil = e * (1.0f - ratio);
+        const float phi = kTwoPi * uniform(rng);
+        if (P.transport_electrons && recoil > P.ecut) {
+          const float ce = compton_electron_cos(e, ratio);
+          float ex = ux, ey = uy, ez = uz;
+          rotate(ex, ey, ez, ce, phi + kPi);
           const uint64_t child = spawn_stream(rng);
-          push(qe, ELECTRON, column, share_e, w, x, y, z, ux, uy, uz, child);
+          push(qe, ELECTRON, column, recoil, w, x, y, z, ex, ey, ez, child);
         } else {
-          deposit<kFast, false>(P, tal, base, x, y, z, w * share_e,
-                  spr<kFast>(P, share_e, mat));
+          deposit<kFast, kOne>(P, tal, base, x, y, z, w * recoil, spr_of(recoil));
         }
-        if (share_p > P.ecut) {
+        const float cg = compton_cos(e, ratio);
+        rotate(ux, uy, uz, cg, phi);
+        e *= ratio;
+        if (e <= P.pcut) {
+          deposit<kFast, kOne>(P, tal, base, x, y, z, w * e, spr_of(e));
+        } else {
+          flying = true;
+          if (e < kRouletteMeV && w < kRouletteWeightCap) {
+            const float new_w = uniform(rng) < kRouletteSurvival ? w / kRouletteSurvival : 0.0f;
+            escape(tal, (w - new_w) * e);
+            flying = new_w != 0.0f;
+            w = new_w;
+          }
+          if (flying) at_energy();
+        }
+      } else if (process == PHOTOELECTRIC) {
+        if (P.transport_electrons && e > P.ecut) {
           const uint64_t child = spawn_stream(rng);
-          push(qe, POSITRON, column, share_p, w, x, y, z, ux, uy, uz, child);
+          push(qe, ELECTRON, column, e, w, x, y, z, ux, uy, uz, child);
         } else {
-          deposit<kFast, false>(P, tal, base, x, y, z, w * share_p,
-                  spr<kFast>(P, share_p, mat));
-          annihilate<kFast, false>(P, tal, qp, base, column, x, y, z, w, f_ann, rng);
+          deposit<kFast, kOne>(P, tal, base, x, y, z, w * e, spr_of(e));
         }
-      } else {
-        deposit<kFast, false>(P, tal, base, x, y, z, w * kinetic,
-                spr<kFast>(P, kinetic, mat));
-        annihilate<kFast, false>(P, tal, qp, base, column, x, y, z, w, f_ann, rng);
+      } else {  // pair production
+        const float kinetic = e - 2.0f * kElectronMass;
+        const float f_ann = spr_of(kElectronMass);
+        if (P.transport_electrons) {
+          const float fraction = uniform(rng);
+          const float share_e = fraction * kinetic;
+          const float share_p = (1.0f - fraction) * kinetic;
+          if (share_e > P.ecut) {
+            const uint64_t child = spawn_stream(rng);
+            push(qe, ELECTRON, column, share_e, w, x, y, z, ux, uy, uz, child);
+          } else {
+            deposit<kFast, kOne>(P, tal, base, x, y, z, w * share_e, spr_of(share_e));
+          }
+          if (share_p > P.ecut) {
+            const uint64_t child = spawn_stream(rng);
+            push(qe, POSITRON, column, share_p, w, x, y, z, ux, uy, uz, child);
+          } else {
+            deposit<kFast, kOne>(P, tal, base, x, y, z, w * share_p, spr_of(share_p));
+            annihilate<kFast, kOne>(P, tal, qp, base, column, x, y, z, w, f_ann, rng);
+          }
+        } else {
+          deposit<kFast, kOne>(P, tal, base, x, y, z, w * kinetic, spr_of(kinetic));
+          annihilate<kFast, kOne>(P, tal, qp, base, column, x, y, z, w, f_ann, rng);
+        }
       }
-      active = false;
     }
   }
   seal_chunk(qe);
@@ -678,7 +724,6 @@ k_photon_round(TransportParams P, Queue qin,
 // unscaled quotients, 4.98 with the GS nodes of a cell in one 16-byte gather. Blocks of
 // 12 waves, one to a CU: 5.0 ms; two to a CU 5.3 (the L1 holds fewer waves' lines).
 // More materials or longer tables than fit take the general build.
-constexpr int kTablePoints = 2048;   // largest table of the kOne build
 constexpr int kMollerSlots = 32;     // stack slots of a wave
 constexpr int kMollerBatch = 16;     // waiting particles that make a batch
 constexpr int kParticleWords = 12;   // x y z e | ux uy uz w | rng | column and kind | steps
@@ -1773,9 +1818,9 @@ __global__ void __launch_bounds__(256) k_sample_physics(uint64_t seed, long long
   float* o = out + i * HMC_SAMPLE_COLUMNS;
   const float nan = __int_as_float(0x7fc00000);
   o[0] = sample_path(static_cast<float>(a.path_mu), rng);
-  o[1] = static_cast<float>(select_process(static_cast<float>(a.channel_mu[0]), static_cast<float>(a.channel_mu[1]),
-                                           static_cast<float>(a.channel_mu[2]), static_cast<float>(a.channel_mu[3]),
-                                           rng));
+  const float mu1 = static_cast<float>(a.channel_mu[0]), mu2 = mu1 + static_cast<float>(a.channel_mu[1]),
+              mu3 = mu2 + static_cast<float>(a.channel_mu[2]);
+  o[1] = static_cast<float>(select_process(mu1, mu2, mu3, mu3 + static_cast<float>(a.channel_mu[3]), rng));
   const float e0 = static_cast<float>(a.compton_energy[0]);
   const float r = sample_compton_ratio(e0, rng);
   o[2] = r;
@@ -2946,6 +2991,7 @@ static int enqueue_round_group(hmc_ctx* ctx, const TransportParams& P, unsigned 
   const bool one = P.t.n_mat == 1 && P.t.n_points <= kTablePoints && small_grid(P.g.nx, P.g.ny, P.g.nz) &&
                    small_grid(P.s.nx, P.s.ny, P.s.nz);
   const unsigned int one_blocks = std::max(1u, round_blocks * 256u / kElectronThreads<true>);
+  static_assert(kPhotonThreads<true> == kElectronThreads<true>, "both rounds launch one_blocks");
   unsigned int* counts = ctx->d_counts;
   unsigned int* heads = ctx->d_counts + 4;
   int pa = 0, ea = 1, pb = 2, eb = 3;
@@ -2957,12 +3003,18 @@ static int enqueue_round_group(hmc_ctx* ctx, const TransportParams& P, unsigned 
     hipEvent_t* ev = events ? events + 4 * r : nullptr;
     // Photon round: consume pa; electrons append to ea, photons to pb.
     if (ev) HMC_HIP(ctx, hipEventRecord(ev[0], ctx->stream));
-    if (fast)
-      hipLaunchKernelGGL((k_photon_round<true>), dim3(round_blocks), dim3(256), 0, ctx->stream, P, qa_p,
-                         heads + pa, qa_e, qb_p);
+    if (one && fast)
+      hipLaunchKernelGGL((k_photon_round<true, true>), dim3(one_blocks), dim3(kPhotonThreads<true>), 0, ctx->stream, P,
+                         qa_p, heads + pa, qa_e, qb_p);
+    else if (one)
+      hipLaunchKernelGGL((k_photon_round<false, true>), dim3(one_blocks), dim3(kPhotonThreads<true>), 0, ctx->stream,
+                         P, qa_p, heads + pa, qa_e, qb_p);
+    else if (fast)
+      hipLaunchKernelGGL((k_photon_round<true, false>), dim3(round_blocks), dim3(kPhotonThreads<false>), 0,
+                         ctx->stream, P, qa_p, heads + pa, qa_e, qb_p);
     else
-      hipLaunchKernelGGL((k_photon_round<false>), dim3(round_blocks), dim3(256), 0, ctx->stream, P, qa_p,
-                         heads + pa, qa_e, qb_p);
+      hipLaunchKernelGGL((k_photon_round<false, false>), dim3(round_blocks), dim3(kPhotonThreads<false>), 0,
+                         ctx->stream, P, qa_p, heads + pa, qa_e, qb_p);
     HMC_HIP(ctx, hipGetLastError());
     if (ev) HMC_HIP(ctx, hipEventRecord(ev[1], ctx->stream));
     // Electron round: consume ea (including the photon round's pushes). In the first
