@@ -256,6 +256,10 @@ int hmc_folded_quanta(hmc_ctx *ctx, int64_t *total_quanta);
 /* Mean and sigma per (column, voxel): finalize_run (kernels.py:881-909). With
  * mean/sigma NULL the result stays on the device for hmc_truncate. */
 int hmc_finalize(hmc_ctx *ctx, int n_batches, double *mean, double *sigma);
+/* hmc_fold (without a total) and hmc_finalize in one pass over the maps and sums, for the
+ * last fold of a run: the same means, sigmas and quanta, bit for bit. */
+int hmc_fold_finalize(hmc_ctx *ctx, int n_slots_used, const double *nhist, int n_batches,
+                      double *mean, double *sigma);
 /* Per-column truncation and ordered CSC compaction on the device: column_max,
  * count_kept_per_chunk, compact_column_chunked (kernels.py:1032-1168) and the
  * host prefix (engine.py:1496-1557). counts[n_columns] out; entries fetched next. */

@@ -253,6 +253,7 @@ def lib():
         "hmc_fold": (c_int, [ctx_p, c_int, _f64p, POINTER(c_int64)]),
         "hmc_folded_quanta": (c_int, [ctx_p, POINTER(c_int64)]),
         "hmc_finalize": (c_int, [ctx_p, c_int, _f64p, _f64p]),
+        "hmc_fold_finalize": (c_int, [ctx_p, c_int, _f64p, c_int, _f64p, _f64p]),
         "hmc_truncate": (c_int, [ctx_p, c_double, POINTER(c_int64), POINTER(c_int64)]),
         "hmc_fetch_csc": (c_int, [ctx_p, POINTER(c_int64), _f64p, _f64p]),
         "hmc_fetch_csc_f32": (c_int, [ctx_p, POINTER(c_int64), _f32p, _f32p]),

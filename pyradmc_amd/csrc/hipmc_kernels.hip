@@ -1507,75 +1507,140 @@ __global__ void k_fill_u64(unsigned long long* a, long long n, unsigned long lon
 // pyradmc/scoring/dose.py:169-207).
 #pragma clang fp contract(off)
 
-constexpr int kFoldSlots = 4;
+// Slots loaded together and workgroups of a fold: 5 and 16384 (19.5 ms for the Dij below);
+// 8 and 4096: 20.8, 8 and 8192: 20.1, 10 and 8192: 20.0.
+constexpr int kFoldSlots = 5;
+constexpr int kFoldBlocks = 16384;
 
-__global__ void __launch_bounds__(256) k_fold(long long* edep, const double* mass,
-                                              const double* nhist, long long n_vox,
-                                              long long n_cols, int n_slots, double* s1,
-                                              double* s2, unsigned long long* folded) {
-  const long long total = n_vox * n_cols;
-  const long long slot_stride = total;
+// Mean and batch sigma of a cell's float64 sums a and b over n batches.
+__device__ inline void batch_statistics(double a, double b, int n_batches, double& mean, double& sigma) {
+  mean = 0.0;
+  sigma = 0.0;
+  if (a == 0.0 && b == 0.0) return;  // exact zeros stay
+  const double n = static_cast<double>(n_batches);
+  mean = a / n;
+  if (n_batches > 1) {
+    const double var = fmax(0.0, b / n - mean * mean) * n / (n - 1.0);
+    sigma = sqrt(var / n);
+  }
+}
+
+// Largest of the workgroup's (non-negative) values into *target, by one atomic.
+__device__ inline void block_max(double m, double* red, unsigned long long* target) {
+  for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off));
+  if (__lane_id() == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < static_cast<int>(blockDim.x >> 6); ++w) m = fmax(m, red[w]);
+    // Non-negative doubles order like their bit patterns.
+    if (m > 0.0) atomicMax(target, static_cast<unsigned long long>(__double_as_longlong(m)));
+  }
+  __syncthreads();
+}
+
+// Slots 0 .. n_slots - 1 of the tally maps, in slot order, into the sums; the maps are
+// zeroed as they are read. A workgroup takes 256 cells of one column at a time (grid-stride,
+// so that the workgroups in flight read neighbouring lines: with 32 KB of cells each they
+// met in the same channels and the pass took 10.9 ms); a slot's history count is then
+// uniform. Bound by the maps' bytes: most
+// cells of a beamlet column hold nothing, but every map is read. So no other pass over
+// the columns is left: kFirst, the first fold since a reset, writes every cell's sums
+// (no clearing pass before, no sums read), and kLast, the fold before a finalize, writes
+// mean and sigma in their place and the columns' largest means for the truncation. 36
+// columns of 256 x 256 x 128 voxels in 10 slots: clear, fold, finalize and column maxima
+// 9.9 ms as passes of their own, 6.9 ms as one (24 GB of maps read and 4.8 GB of sums
+// written; the card reads 4.0 TB/s). One atomic per workgroup books the folded quanta: one
+// per wave had put 260 000 on one address.
+template <bool kFirst, bool kLast>
+__global__ void __launch_bounds__(256) k_fold(long long* edep, const double* mass, const double* nhist,
+                                              long long n_vox, long long n_cols, int n_slots, long long chunks_per_col, double* s1, double* s2, int n_batches,
+                                              unsigned long long* col_max, unsigned long long* folded) {
+  __shared__ double red[4];
+  __shared__ long long red_q[4];
+  const long long slot_stride = n_vox * n_cols;
   long long local = 0;
-  for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < total;
-       i += static_cast<long long>(gridDim.x) * blockDim.x) {
-    long long col = 0;
-    double m = 0.0, a = 0.0, b = 0.0;
-    bool touched = false;
-    for (int s0 = 0; s0 < n_slots; s0 += kFoldSlots) {
-      // The next kFoldSlots slots' tallies are loaded together (more bytes in flight
-      // per wave), then taken in batch order.
-      long long qs[kFoldSlots];
+  double largest = 0.0;  // mean of the cells since the last column change
+  long long largest_col = 0;
+  for (long long t = blockIdx.x; t < chunks_per_col * n_cols; t += gridDim.x) {
+    const long long col = t / chunks_per_col;
+    const long long v = (t - col * chunks_per_col) * 256 + threadIdx.x;
+    if (kLast && col != largest_col) {
+      block_max(largest, red, col_max + largest_col);
+      largest = 0.0;
+      largest_col = col;
+    }
+    if (v < n_vox) {
+      const long long i = col * n_vox + v;
+      double m = 0.0, a = 0.0, b = 0.0;
+      bool touched = false;
+      if (kLast && !kFirst) {
+        a = s1[i];
+        b = s2[i];
+      }
+      for (int s0 = 0; s0 < n_slots; s0 += kFoldSlots) {
+        // The next kFoldSlots slots' tallies are loaded together (more bytes in flight
+        // per wave), then taken in batch order.
+        long long qs[kFoldSlots];
 #pragma unroll
-      for (int k = 0; k < kFoldSlots; ++k)
-        qs[k] = s0 + k < n_slots ? edep[(s0 + k) * slot_stride + i] : 0;
+        for (int k = 0; k < kFoldSlots; ++k)
+          qs[k] = s0 + k < n_slots ? edep[(s0 + k) * slot_stride + i] : 0;
 #pragma unroll
-      for (int k = 0; k < kFoldSlots; ++k) {
-        const long long q = qs[k];
-        if (q == 0) continue;
-        const int slot = s0 + k;
-        edep[slot * slot_stride + i] = 0;
-        if (!touched) {
-          // Most cells of a beamlet column see no deposit in a fold: their column,
-          // mass and sums are looked up only once a slot holds one.
-          col = i / n_vox;
-          m = mass[i - col * n_vox];
-          a = s1[i];
-          b = s2[i];
+        for (int k = 0; k < kFoldSlots; ++k) {
+          const long long q = qs[k];
+          if (q == 0) continue;
+          const int slot = s0 + k;
+          edep[slot * slot_stride + i] = 0;
+          if (!touched) {
+            // Most cells of a beamlet column see no deposit in a fold: their mass (and
+            // sums) are looked up only once a slot holds one.
+            m = mass[v];
+            if (!kFirst && !kLast) {
+              a = s1[i];
+              b = s2[i];
+            }
+          }
+          double d = 0.0;
+          if (m > 0.0) {
+            const double energy = static_cast<double>(q) * 1.0e-9;
+            d = energy / (m * nhist[slot * n_cols + col]);
+          }
+          a = a + d;
+          b = b + d * d;
+          touched = true;
+          local += q;
         }
-        double d = 0.0;
-        if (m > 0.0) {
-          const double energy = static_cast<double>(q) * 1.0e-9;
-          d = energy / (m * nhist[slot * n_cols + col]);
-        }
-        a = a + d;
-        b = b + d * d;
-        touched = true;
-        local += q;
+      }
+      if (kLast) {
+        double mean, sigma;
+        batch_statistics(a, b, n_batches, mean, sigma);
+        s1[i] = mean;
+        s2[i] = sigma;
+        largest = fmax(largest, mean);
+      } else if (kFirst || touched) {
+        s1[i] = a;
+        s2[i] = b;
       }
     }
-    if (touched) {
-      s1[i] = a;
-      s2[i] = b;
-    }
   }
+  if (kLast) block_max(largest, red, col_max + largest_col);
   const long long sum = wave_sum(local);
-  if (__lane_id() == 0 && sum != 0) atomicAdd(folded, static_cast<unsigned long long>(sum));
+  if (__lane_id() == 0) red_q[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const long long total = red_q[0] + red_q[1] + red_q[2] + red_q[3];
+    if (total != 0) atomicAdd(folded, static_cast<unsigned long long>(total));
+  }
 }
 
 __global__ void __launch_bounds__(256) k_finalize(double* s1, double* s2, long long total,
                                                   int n_batches) {
-  const double n = static_cast<double>(n_batches);
   for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < total;
        i += static_cast<long long>(gridDim.x) * blockDim.x) {
     const double a = s1[i];
     const double b = s2[i];
     if (a == 0.0 && b == 0.0) continue;  // exact zeros stay
-    const double mean = a / n;
-    double sigma = 0.0;
-    if (n_batches > 1) {
-      const double var = fmax(0.0, b / n - mean * mean) * n / (n - 1.0);
-      sigma = sqrt(var / n);
-    }
+    double mean, sigma;
+    batch_statistics(a, b, n_batches, mean, sigma);
     s1[i] = mean;
     s2[i] = sigma;
   }
@@ -1601,20 +1666,8 @@ __global__ void __launch_bounds__(kTruncBlock) k_column_max(const double* mean, 
   double m = 0.0;
   for (long long v = v0 + threadIdx.x; v < v1; v += kTruncBlock)
     m = fmax(m, mean[col * n_vox + v]);
-  __shared__ double red[kTruncBlock];
-  red[threadIdx.x] = m;
-  __syncthreads();
-  for (int s = kTruncBlock / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + s]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    // Non-negative doubles order like their bit patterns.
-    unsigned long long bits;
-    const double v = red[0];
-    memcpy(&bits, &v, sizeof(bits));
-    atomicMax(col_max + col, bits);
-  }
+  __shared__ double red[kTruncBlock / 64];
+  block_max(m, red, col_max + col);
 }
 
 __device__ inline bool keep_entry(double m, double thr) { return m > 0.0 && m >= thr; }
@@ -1729,6 +1782,8 @@ struct hmc_ctx {
   int* d_origins = nullptr;  // window origins for hmc_gather_windows / hmc_scatter_windows
   bool has_scoring = false;
   bool finalized = false;
+  bool sums_clear = false;    // reset since the last fold: the sums count as zeros, whatever the buffers hold
+  bool colmax_ready = false;  // d_colmax holds the finalized means' column maxima
   // Folds made without a host wait (hmc_fold with total_quanta NULL) add their quanta to
   // the device counter past the ledger; the next hmc_finalize reads it back with the
   // means, and hmc_folded_quanta hands it out.
@@ -2092,6 +2147,7 @@ int hmc_set_scoring(hmc_ctx* ctx, int nx, int ny, int nz, const double* origin,
   ctx->n_columns = n_columns;
   ctx->n_slots = n_slots;
   ctx->has_scoring = true;
+  ctx->colmax_ready = false;
   ctx->dirty_slots = n_slots;  // fresh or reused buffers: clear every slot once
   return hmc_reset_maps(ctx);
 }
@@ -2100,18 +2156,14 @@ int hmc_reset_maps(hmc_ctx* ctx) {
   if (!ctx || !ctx->has_scoring) return fail(ctx, HMC_ESTATE, "scoring grid not set");
   HMC_HIP(ctx, hipSetDevice(ctx->device));
   const long long total = ctx->s.n_voxels * ctx->n_columns;
-  const int blocks = blocks_for(total, 256, 65536);
   if (ctx->dirty_slots > 0)
     hipLaunchKernelGGL(k_fill_u64, dim3(blocks_for(total * ctx->dirty_slots, 256, 65536)), dim3(256), 0,
                        ctx->stream, reinterpret_cast<unsigned long long*>(ctx->d_edep),
                        total * ctx->dirty_slots, 0ull);
-  hipLaunchKernelGGL(k_fill_u64, dim3(blocks), dim3(256), 0, ctx->stream,
-                     reinterpret_cast<unsigned long long*>(ctx->d_s1), total, 0ull);
-  hipLaunchKernelGGL(k_fill_u64, dim3(blocks), dim3(256), 0, ctx->stream,
-                     reinterpret_cast<unsigned long long*>(ctx->d_s2), total, 0ull);
   HMC_HIP(ctx, hipGetLastError());  // stream-ordered before the next transport: no host wait
   ctx->dirty_slots = 0;
   ctx->finalized = false;
+  ctx->sums_clear = true;  // the first fold writes every sum
   ctx->fold_pending = false;
   ctx->folded_quanta = 0;
   return HMC_OK;
@@ -3356,7 +3408,9 @@ int hmc_transport(hmc_ctx* ctx, uint64_t seed, const hmc_work_item* items, int n
   return HMC_OK;
 }
 
-int hmc_fold(hmc_ctx* ctx, int n_slots_used, const double* nhist, int64_t* total_quanta) {
+// Queue the fold of slots 0 .. n_slots_used - 1; with n_batches > 0 as the last fold, which
+// finalizes (unless that is done already).
+static int enqueue_fold(hmc_ctx* ctx, int n_slots_used, const double* nhist, int n_batches) {
   if (!ctx || !nhist) return fail(ctx, HMC_EINVAL, "null");
   if (!ctx->has_scoring) return fail(ctx, HMC_ESTATE, "scoring grid not set");
   if (n_slots_used < 1 || n_slots_used > ctx->n_slots)
@@ -3371,22 +3425,43 @@ int hmc_fold(hmc_ctx* ctx, int n_slots_used, const double* nhist, int64_t* total
   // The counter starts from zero unless earlier folds' quanta are still to be read.
   if (!ctx->fold_pending)
     hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, ctx->stream, folded, 1ll, 0ull);
-  const long long total = ctx->s.n_voxels * ctx->n_columns;
-  hipLaunchKernelGGL(k_fold, dim3(blocks_for(total, 256, 65536)), dim3(256), 0, ctx->stream,
-                     ctx->d_edep, ctx->d_mass, ctx->d_nhist, ctx->s.n_voxels, ctx->n_columns,
-                     n_slots_used, ctx->d_s1, ctx->d_s2, folded);
+  const bool last = n_batches > 0 && !ctx->finalized;
+  if (last)
+    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(256), 0, ctx->stream, ctx->d_colmax, ctx->n_columns, 0ull);
+  const long long nv = ctx->s.n_voxels;
+  const long long per_col = (nv + 255) / 256;
+  const auto kernel = ctx->sums_clear ? (last ? k_fold<true, true> : k_fold<true, false>)
+                                      : (last ? k_fold<false, true> : k_fold<false, false>);
+  hipLaunchKernelGGL(kernel, dim3(blocks_for(per_col * ctx->n_columns, 1, kFoldBlocks)), dim3(256), 0, ctx->stream,
+                     ctx->d_edep, ctx->d_mass, ctx->d_nhist, nv, ctx->n_columns, n_slots_used, per_col, ctx->d_s1,
+                     ctx->d_s2, n_batches, ctx->d_colmax, folded);
   HMC_HIP(ctx, hipGetLastError());
+  ctx->sums_clear = false;
   if (n_slots_used >= ctx->dirty_slots) ctx->dirty_slots = 0;  // the fold zeroes what it reads
+  if (last) ctx->finalized = ctx->colmax_ready = true;
+  return HMC_OK;
+}
+
+int hmc_fold(hmc_ctx* ctx, int n_slots_used, const double* nhist, int64_t* total_quanta) {
+  if (int rc = enqueue_fold(ctx, n_slots_used, nhist, 0)) return rc;
   if (!total_quanta) {  // no wait: the total comes back with the next hmc_finalize
     ctx->fold_pending = true;
     return HMC_OK;
   }
-  HMC_HIP(ctx, hipMemcpyAsync(ctx->h_stage + kStageFolded, folded, sizeof(unsigned long long),
+  HMC_HIP(ctx, hipMemcpyAsync(ctx->h_stage + kStageFolded, ctx->d_ledger + L_COUNT, sizeof(unsigned long long),
                               hipMemcpyDeviceToHost, ctx->stream));
   HMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
   ctx->fold_pending = false;
   *total_quanta = static_cast<int64_t>(ctx->h_stage[kStageFolded]);
   return HMC_OK;
+}
+
+int hmc_fold_finalize(hmc_ctx* ctx, int n_slots_used, const double* nhist, int n_batches, double* mean,
+                      double* sigma) {
+  if (!ctx || n_batches < 1) return fail(ctx, HMC_EINVAL, "bad finalize arguments");
+  if (int rc = enqueue_fold(ctx, n_slots_used, nhist, n_batches)) return rc;
+  ctx->fold_pending = true;
+  return hmc_finalize(ctx, n_batches, mean, sigma);
 }
 
 int hmc_folded_quanta(hmc_ctx* ctx, int64_t* total_quanta) {
@@ -3409,11 +3484,19 @@ int hmc_finalize(hmc_ctx* ctx, int n_batches, double* mean, double* sigma) {
   if (!ctx->has_scoring) return fail(ctx, HMC_ESTATE, "scoring grid not set");
   HMC_HIP(ctx, hipSetDevice(ctx->device));
   const long long total = ctx->s.n_voxels * ctx->n_columns;
+  if (ctx->sums_clear) {  // nothing folded since the reset
+    for (double* sums : {ctx->d_s1, ctx->d_s2})
+      hipLaunchKernelGGL(k_fill_u64, dim3(blocks_for(total, 256, 65536)), dim3(256), 0, ctx->stream,
+                         reinterpret_cast<unsigned long long*>(sums), total, 0ull);
+    HMC_HIP(ctx, hipGetLastError());
+    ctx->sums_clear = false;
+  }
   if (!ctx->finalized) {
     hipLaunchKernelGGL(k_finalize, dim3(blocks_for(total, 256, 65536)), dim3(256), 0,
                        ctx->stream, ctx->d_s1, ctx->d_s2, total, n_batches);
     HMC_HIP(ctx, hipGetLastError());
     ctx->finalized = true;
+    ctx->colmax_ready = false;
   }
   if (mean)
     HMC_HIP(ctx, hipMemcpyAsync(mean, ctx->d_s1, sizeof(double) * total, hipMemcpyDeviceToHost,
@@ -3444,10 +3527,13 @@ int hmc_truncate(hmc_ctx* ctx, double truncation, int64_t* counts, int64_t* tota
   int rc;
   if ((rc = dev_alloc(ctx, &ctx->d_chunk_counts, static_cast<size_t>(n_blocks)))) return rc;
   if ((rc = dev_alloc(ctx, &ctx->d_chunk_offsets, static_cast<size_t>(n_blocks)))) return rc;
-  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(256), 0, ctx->stream, ctx->d_colmax,
-                     ctx->n_columns, 0ull);
-  hipLaunchKernelGGL(k_column_max, dim3(static_cast<unsigned>(n_blocks)), dim3(kTruncBlock), 0,
-                     ctx->stream, ctx->d_s1, nv, chunks, ctx->d_colmax);
+  if (!ctx->colmax_ready) {  // else the last fold left them
+    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(256), 0, ctx->stream, ctx->d_colmax,
+                       ctx->n_columns, 0ull);
+    hipLaunchKernelGGL(k_column_max, dim3(static_cast<unsigned>(n_blocks)), dim3(kTruncBlock), 0,
+                       ctx->stream, ctx->d_s1, nv, chunks, ctx->d_colmax);
+    ctx->colmax_ready = true;
+  }
   hipLaunchKernelGGL(k_count_kept, dim3(static_cast<unsigned>(n_blocks)), dim3(kTruncBlock), 0,
                      ctx->stream, ctx->d_s1, nv, chunks, ctx->d_colmax, truncation,
                      ctx->d_chunk_counts);
@@ -3539,6 +3625,7 @@ int hmc_scatter_windows(hmc_ctx* ctx, const int32_t* origins, int64_t n_cols, in
   HMC_HIP(ctx, hipGetLastError());
   HMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
   ctx->finalized = true;  // s1 / s2 now hold mean / sigma for hmc_truncate
+  ctx->sums_clear = ctx->colmax_ready = false;
   return HMC_OK;
 }
 
@@ -3558,6 +3645,7 @@ int hmc_set_column_entries(hmc_ctx* ctx, int64_t column, int64_t n, const int64_
   if ((rc = dev_alloc(ctx, &ctx->d_entry_val, static_cast<size_t>(2 * n)))) return rc;
   HMC_HIP(ctx, hipMemcpy(ctx->d_entry_val, dose, sizeof(double) * n, hipMemcpyHostToDevice));
   HMC_HIP(ctx, hipMemcpy(ctx->d_entry_val + n, sigma, sizeof(double) * n, hipMemcpyHostToDevice));
+  ctx->colmax_ready = false;
   hipLaunchKernelGGL(k_set_entries, dim3(blocks_for(n, 256, 65536)), dim3(256), 0, ctx->stream, ctx->d_s1, ctx->d_s2,
                      static_cast<long long>(column) * ctx->s.n_voxels, static_cast<long long>(n), ctx->d_entry_idx,
                      ctx->d_entry_val, ctx->d_entry_val + n);

@@ -602,6 +602,14 @@ class HipEngine:
         nh = np.ascontiguousarray(np.asarray(nhist, dtype=np.float64).reshape(-1))
         self._ctx.call("hmc_fold", int(n_slots), nat.ptr(nh, nat.c_double), None)
 
+    def _fold_finalize(self, n_slots: int, nhist: np.ndarray, n_batches: int, mean=None, sigma=None) -> None:
+        """The last fold of a run together with its finalize (mean and sigma host arrays,
+        or None to leave them on the device)."""
+        nh = np.ascontiguousarray(np.asarray(nhist, dtype=np.float64).reshape(-1))
+        self._ctx.call("hmc_fold_finalize", int(n_slots), nat.ptr(nh, nat.c_double), int(n_batches),
+                       None if mean is None else nat.ptr(mean, nat.c_double),
+                       None if sigma is None else nat.ptr(sigma, nat.c_double))
+
     def _folded_quanta(self) -> int:
         """Quanta folded since the last call (read back by the finalize after them)."""
         total = nat.c_int64()
@@ -715,13 +723,15 @@ class HipEngine:
                                            books)
             else:
                 self._merge(books, self._transport(seed, items, chunk))
-            self._fold(len(block), np.full(len(block), float(per_batch)))
+            nhist = np.full(len(block), float(per_batch))
+            if block.stop < n_batches:
+                self._fold(len(block), nhist)
+            else:
+                mean = host_array(scoring.n_voxels, np.float64)
+                sigma = host_array(scoring.n_voxels, np.float64)
+                self._fold_finalize(len(block), nhist, n_batches, mean, sigma)
             for _ in block:
                 emitter.tick(per_batch)
-        n_vox = scoring.n_voxels
-        mean = host_array(n_vox, np.float64)
-        sigma = host_array(n_vox, np.float64)
-        self._ctx.call("hmc_finalize", int(n_batches), nat.ptr(mean, nat.c_double), nat.ptr(sigma, nat.c_double))
         deposited_quanta = self._folded_quanta()
 
         if analytic:
@@ -789,8 +799,10 @@ class HipEngine:
             else:
                 self._merge(books, self._transport(seed, items, chunk))
             nhist = np.tile(per_batch[g0:group.stop].astype(np.float64), len(block))
-            self._fold(len(block), nhist)
-        self._ctx.call("hmc_finalize", int(n_batches), None, None)
+            if block.stop < n_batches:
+                self._fold(len(block), nhist)
+            else:
+                self._fold_finalize(len(block), nhist, n_batches)
         return analytic, mono_energy, self._folded_quanta()
 
     def run_dij(

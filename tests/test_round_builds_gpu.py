@@ -81,3 +81,52 @@ def test_moller_stack_in_use_and_full_equals_one_never_used():
     _same(full, few)
     pushed = full.counters["electron_pushes"]
     assert pushed > 64 * 512 // 16  # delta electrons by the dozen per primary
+
+
+@pytest.mark.parametrize("columns, slots, blocks", [(1, 1, 1), (3, 7, 1), (2, 6, 2), (5, 3, 3), (1, 0, 1)])
+def test_folds_in_one_pass_equal_their_parts(columns, slots, blocks):
+    """Random quanta through hmc_fold_finalize (the first fold, a later one, the only one)
+    and hmc_truncate against numpy's float64, bit for bit; a run with nothing folded."""
+    from pyradmc_amd import _native as nat
+
+    rng = np.random.default_rng(columns + slots)
+    shape = (5, 7, 29)  # 1015 voxels: a remainder in every chunk
+    n_vox = int(np.prod(shape))
+    mass = rng.uniform(0.1, 2.0, n_vox)
+    mass[::97] = 0.0
+    ctx = nat.Context(0)
+    zero, one = np.zeros(3), np.ones(3)
+    ctx.call("hmc_set_scoring", *shape, nat.ptr(zero, nat.c_double), nat.ptr(one, nat.c_double),
+             nat.ptr(mass, nat.c_double), columns, max(slots, 1))
+    mean, sigma = np.empty((columns, n_vox)), np.empty((columns, n_vox))
+    n_batches = max(slots * blocks, 1)
+    s1, s2 = np.zeros((columns, n_vox)), np.zeros((columns, n_vox))
+    total = 0
+    for block in range(blocks if slots else 0):
+        quanta = rng.integers(0, 10**9, (slots, columns, n_vox)) * (rng.random((slots, columns, n_vox)) < 0.2)
+        quanta = np.ascontiguousarray(quanta, dtype=np.int64)
+        nhist = np.ascontiguousarray(rng.integers(1, 1000, (slots, columns)), dtype=np.float64)
+        ctx.call("hmc_set_quanta", nat.ptr(quanta, nat.c_int64))
+        if block + 1 < blocks:
+            ctx.call("hmc_fold", slots, nat.ptr(nhist, nat.c_double), None)
+        else:
+            ctx.call("hmc_fold_finalize", slots, nat.ptr(nhist, nat.c_double), n_batches, nat.ptr(mean, nat.c_double),
+                     nat.ptr(sigma, nat.c_double))
+        total += int(quanta.sum())
+        for q, n in zip(quanta, nhist):
+            with np.errstate(divide="ignore", invalid="ignore"):
+                d = np.where(mass > 0.0, q * 1.0e-9 / (mass * n[:, None]), 0.0)
+            s1, s2 = s1 + d, s2 + d * d
+    if not slots:
+        ctx.call("hmc_finalize", n_batches, nat.ptr(mean, nat.c_double), nat.ptr(sigma, nat.c_double))
+    want = s1 / n_batches
+    var = np.maximum(0.0, s2 / n_batches - want * want) * n_batches / max(n_batches - 1.0, 1.0)
+    np.testing.assert_array_equal(mean, want)
+    np.testing.assert_array_equal(sigma, np.sqrt(var / n_batches) if n_batches > 1 else np.zeros_like(want))
+    folded, kept, entries = nat.c_int64(), np.zeros(columns, np.int64), nat.c_int64()
+    ctx.call("hmc_folded_quanta", nat.ctypes.byref(folded))
+    assert folded.value == total
+    ctx.call("hmc_truncate", 0.3, nat.ptr(kept, nat.c_int64), nat.ctypes.byref(entries))
+    expected = (want > 0.0) & (want >= 0.3 * want.max(axis=1, keepdims=True))
+    np.testing.assert_array_equal(kept, expected.sum(axis=1))
+    ctx.close()
