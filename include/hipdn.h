@@ -47,6 +47,14 @@ int hdn_conv3d_fwd(const void* x, const void* w, const float* bias, void* y_nd, 
 int hdn_conv3d_fwd_src(const void* x, const void* x2, int src, const void* w, const float* bias, void* y_nd,
                        void* y_cm, int n, int d, int h, int w_, int cin, int cout, float slope, void* stream);
 
+/* hdn_conv3d_fwd_src with the element-wise step after the convolution taken in its store.
+ * skip (NULL: none; src 0 or 1): hdn_add(y, skip) is stored instead of y. pred (NULL: none;
+ * src 0): only inp[p][0] + y[p][0] in FP32 is stored (the prediction of hdn_loss; inp has
+ * c_in channels; skip must be NULL and y_nd may be). The values are those of the separate calls. */
+int hdn_conv3d_fwd_fused(const void* x, const void* x2, int src, const void* w, const float* bias, const void* skip,
+                         const void* inp, int c_in, float* pred, void* y_nd, void* y_cm, int n, int d, int h,
+                         int w_, int cin, int cout, float slope, void* stream);
+
 /* Weight-gradient partials part[splits][27][cout][cin] (FP32) from the channel-major
  * layer input and output gradient; W % 8 == 0. Sum them with hdn_reduce_splits. */
 int hdn_conv3d_wgrad(const void* x_cm, const void* dz_cm, float* part, int splits, int n, int d,

@@ -61,6 +61,66 @@ __device__ inline bf16x8 add8(bf16x8 a, bf16x8 b) {
   return r;
 }
 
+// What a convolution does with its sums: y = act(bias + sum), rounded to bf16, into y_nd
+// and (where given) the channel-major y_cm; with skip, y + skip rounded again (the values
+// k_add would store) instead of y; with pred, only inp[p][0] + y[p][0] in float32 (the
+// values k_loss would predict) and no y at all.
+struct Epilogue {
+  const float* bias;
+  float slope;
+  const __bf16* skip;
+  __bf16* y_nd;
+  __bf16* y_cm;
+  float* pred;
+  const __bf16* inp;
+  int c_in;  // channels of inp
+};
+
+// Kinds of epilogue. The tiled kernels are built per kind and load what it needs (conv_other)
+// before their k-steps, so that the loads run under the MFMAs; kEpiAny decides at run time.
+constexpr int kEpiPlain = 0, kEpiSkip = 1, kEpiPred = 2, kEpiAny = 3;
+
+// What a lane's four sums of channels cb .. cb + 3 at position p are combined with.
+template <int EPI>
+__device__ inline uint2 conv_other(const Epilogue& E, int cb, long long p, int cout) {
+  if ((EPI == kEpiSkip || EPI == kEpiAny) && E.skip) return *reinterpret_cast<const uint2*>(E.skip + p * cout + cb);
+  if ((EPI == kEpiPred || EPI == kEpiAny) && E.pred && cb == 0) {
+    unsigned short first;
+    std::memcpy(&first, E.inp + p * E.c_in, 2);
+    return make_uint2(first, 0u);
+  }
+  return make_uint2(0u, 0u);
+}
+
+// One lane's four sums: channels cb .. cb + 3 of position p.
+template <int EPI>
+__device__ inline void conv_store(const Epilogue& E, const f32x4& sum, uint2 other, int cb, long long p, int cout,
+                                  long long P) {
+  __bf16 out[4], with[4];
+  std::memcpy(with, &other, 8);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float v = sum[r] + (E.bias ? E.bias[cb + r] : 0.0f);
+    out[r] = static_cast<__bf16>(act(v, E.slope));
+  }
+  if (EPI == kEpiPred || (EPI == kEpiAny && E.pred)) {
+    if (cb == 0) E.pred[p] = static_cast<float>(with[0]) + static_cast<float>(out[0]);
+    return;
+  }
+  if (EPI == kEpiSkip || (EPI == kEpiAny && E.skip)) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      out[r] = static_cast<__bf16>(static_cast<float>(out[r]) + static_cast<float>(with[r]));
+  }
+  uint2 packed;
+  std::memcpy(&packed, out, 8);
+  *reinterpret_cast<uint2*>(E.y_nd + p * cout + cb) = packed;
+  if (E.y_cm) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) E.y_cm[static_cast<long long>(cb + r) * P + p] = out[r];
+  }
+}
+
 // ------------------------------------------------------------------ convolution
 //
 // y[p][co] = act(bias[co] + sum_{tap, ci} x[p + off(tap)][ci] wt[tap][co][ci]) with
@@ -70,11 +130,8 @@ __device__ inline bf16x8 add8(bf16x8 a, bf16x8 b) {
 template <int TM, int SRC>
 __global__ void __launch_bounds__(256) k_conv_fwd(const __bf16* __restrict__ x,
                                                   const __bf16* __restrict__ x2,
-                                                  const __bf16* __restrict__ wt,
-                                                  const float* __restrict__ bias,
-                                                  __bf16* __restrict__ y_nd,
-                                                  __bf16* __restrict__ y_cm, int n, int d, int h,
-                                                  int w, int cin, int cout, float slope) {
+                                                  const __bf16* __restrict__ wt, Epilogue E, int n, int d, int h,
+                                                  int w, int cin, int cout) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const long long P = static_cast<long long>(n) * d * h * w;
@@ -149,19 +206,7 @@ __global__ void __launch_bounds__(256) k_conv_fwd(const __bf16* __restrict__ x,
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
       const long long p = p0 + 16 * nb + col;
-      __bf16 out[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float v = acc[m][nb][r] + (bias ? bias[cb + r] : 0.0f);
-        out[r] = static_cast<__bf16>(act(v, slope));
-      }
-      uint2 packed;
-      std::memcpy(&packed, out, 8);
-      *reinterpret_cast<uint2*>(y_nd + p * cout + cb) = packed;
-      if (y_cm) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) y_cm[static_cast<long long>(cb + r) * P + p] = out[r];
-      }
+      conv_store<kEpiAny>(E, acc[m][nb], conv_other<kEpiAny>(E, cb, p, cout), cb, p, cout, P);
     }
   }
 }
@@ -177,8 +222,7 @@ constexpr int kSplitWaves = 8;
 template <int TM, int SRC>
 __global__ void __launch_bounds__(64 * kSplitWaves) k_conv_fwd_split(
     const __bf16* __restrict__ x, const __bf16* __restrict__ x2, const __bf16* __restrict__ wt,
-    const float* __restrict__ bias, __bf16* __restrict__ y_nd, __bf16* __restrict__ y_cm, int n, int d, int h, int w,
-    int cin, int cout, float slope) {
+    Epilogue E, int n, int d, int h, int w, int cin, int cout) {
   __shared__ f32x4 sums[kSplitWaves / 2][TM * 4][64];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -278,40 +322,23 @@ __global__ void __launch_bounds__(64 * kSplitWaves) k_conv_fwd_split(
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
       const long long p = p0 + 16 * nb + col;
-      __bf16 out[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float v = acc[m][nb][r] + (bias ? bias[cb + r] : 0.0f);
-        out[r] = static_cast<__bf16>(act(v, slope));
-      }
-      uint2 packed;
-      std::memcpy(&packed, out, 8);
-      *reinterpret_cast<uint2*>(y_nd + p * cout + cb) = packed;
-      if (y_cm) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) y_cm[static_cast<long long>(cb + r) * P + p] = out[r];
-      }
+      conv_store<kEpiAny>(E, acc[m][nb], conv_other<kEpiAny>(E, cb, p, cout), cb, p, cout, P);
     }
   }
 }
 
-// The same convolution for rows of KW = 64 or 32 voxels (w == KW, h % (256 / KW) == 0,
+// The same convolution for rows of KW = 32 voxels (w == KW, h % (256 / KW) == 0,
 // cout 16 x TM): a workgroup computes 256 / KW consecutive h-rows of one z-slice (256
 // positions; each wave 64 of them) and first stages the input those rows read - 3 z x
 // (rows + 2) h x (KW + 2) w positions with their one-voxel halo, zero outside the
-// volume - in LDS (KW 64: 38 KB for cin 16, 76 KB for cin 32; KW 32: 33, 65 or 130 KB
-// for cin 16, 32 or 64). Every tap's operand then comes from LDS instead of a gathered
-// global load: the kernel reads each input element from HBM once per workgroup instead
-// of once per tap. The k-loop, MFMA operands and output are those of k_conv_fwd, so
-// the two kernels give identical sums.
-template <int TM, int CIN, int SRC, int KW = 64>
+// volume - in LDS (33, 65 or 130 KB for cin 16, 32 or 64). Every tap's operand then comes
+// from LDS instead of a gathered global load. The k-loop, MFMA operands and output are
+// those of k_conv_fwd, so the two kernels give identical sums.
+template <int TM, int CIN, int SRC, int EPI, int KW>
 __global__ void __launch_bounds__(256) k_conv_fwd_tile(const __bf16* __restrict__ x,
                                                        const __bf16* __restrict__ x2,
-                                                       const __bf16* __restrict__ wt,
-                                                       const float* __restrict__ bias,
-                                                       __bf16* __restrict__ y_nd,
-                                                       __bf16* __restrict__ y_cm, int n, int d, int h,
-                                                       int cout, float slope) {
+                                                       const __bf16* __restrict__ wt, Epilogue E, int n, int d,
+                                                       int h, int cout) {
   constexpr int kW = KW, kRows = 256 / KW, kTW = kW + 2, kTH = kRows + 2, kTZ = 3, kC8 = CIN / 8;
   __shared__ u32x4 tile[kTZ * kTH * kTW * kC8];
   const int rows = h / kRows;
@@ -373,6 +400,14 @@ __global__ void __launch_bounds__(256) k_conv_fwd_tile(const __bf16* __restrict_
     blk_row[nb] = wave * (64 / kW) + (16 * nb) / kW;
     blk_x[nb] = (16 * nb) % kW;
   }
+  const long long P = static_cast<long long>(n) * d * h * kW;
+  const long long row0 = (static_cast<long long>(nn) * d + z) * h + h0;
+  uint2 other[TM][4];
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb)
+      other[m][nb] = conv_other<EPI>(E, 16 * m + 4 * kg, (row0 + blk_row[nb]) * kW + blk_x[nb] + col, cout);
   f32x4 acc[TM][4];
 #pragma unroll
   for (int m = 0; m < TM; ++m)
@@ -434,28 +469,182 @@ __global__ void __launch_bounds__(256) k_conv_fwd_tile(const __bf16* __restrict_
     mfmas(a1, b1);
   }
 
-  const long long P = static_cast<long long>(n) * d * h * kW;
-  const long long row0 = (static_cast<long long>(nn) * d + z) * h + h0;
 #pragma unroll
   for (int m = 0; m < TM; ++m) {
     const int cb = 16 * m + 4 * kg;
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
       const long long p = (row0 + blk_row[nb]) * kW + blk_x[nb] + col;
-      __bf16 out[4];
+      conv_store<EPI>(E, acc[m][nb], other[m][nb], cb, p, cout, P);
+    }
+  }
+}
+
+// The same convolution for rows of 64 voxels (w == 64, h % 4 == 0, cin 16 or 32, cout
+// 16 x TM): the full-resolution layers, bound by the LDS reads of their input fragments
+// (one 1 KiB fragment per MFMA and 16 output channels). A workgroup takes four h-rows and
+// marches along z over zc slices with the three z-planes of a slice in an LDS ring: a
+// plane is loaded once per workgroup (1.55 times in all, for the h and w halo) instead of
+// once per slice it serves, and the next plane's loads run under this slice's MFMAs. The
+// weight fragments of all k-steps stay in registers. 32-channel planes are kept as two
+// halves of 16 channels, so that a fragment's lanes read 32-byte strides (64-byte strides
+// conflict in the banks). The k-steps and their order are those of k_conv_fwd: identical
+// sums. 32 windows of 96 x 64 x 64, us with a 3-plane tile per slice and now: 16 -> 16
+// channels 445 and 260 (the copy rate's floor is 170), the 2-channel input 382 and 190,
+// 32 -> 16 upsampled 870 and 400 (450 with the skip addition in its store).
+template <int TM, int CIN, int SRC, int EPI>
+__global__ void __launch_bounds__(256, (CIN * TM == 16 ? 3 : 2) - (CIN == 16 && (SRC == kSrcAdd || EPI == kEpiSkip) ? 1 : 0))
+    k_conv_fwd_march(
+    const __bf16* __restrict__ x, const __bf16* __restrict__ x2, const __bf16* __restrict__ wt,
+    Epilogue E, int n, int d, int h, int cout, int zc) {
+  constexpr int kW = 64, kRows = 4, kTW = kW + 2, kTH = kRows + 2, kPos = kTH * kTW;
+  constexpr int kKC = SRC == kSrcLow8 ? 8 : CIN;  // channels read per tap
+  constexpr int kC8 = kKC / 8;
+  constexpr int kPosUnits = kC8 >= 2 ? 2 : 1;      // 16-byte units of a position within a half
+  constexpr int kHalf = kPos * kPosUnits;          // units of a half of a plane
+  constexpr int kPlane = kPos * kC8;               // units of a plane
+  constexpr int kPer = (kPlane + 255) / 256;
+  constexpr int K = 27 * kKC, kSteps = (K + 31) / 32;
+  __shared__ u32x4 ring[3 * kPlane];
+  const int rows = h / kRows;
+  const int zchunks = (d + zc - 1) / zc;
+  const int hb = static_cast<int>(blockIdx.x % rows);
+  const int t = static_cast<int>(blockIdx.x / rows);
+  const int z0 = (t % zchunks) * zc;
+  const int z1 = z0 + zc < d ? z0 + zc : d;
+  const int nn = t / zchunks;
+  const int h0 = kRows * hb;
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int col = lane & 15;
+  const int kg = lane >> 4;
+
+  // This thread's units of a plane: place in the ring's slot, and in the tensor's plane
+  // (the half-resolution one for an upsampled input); outside the rows nothing is loaded.
+  u32x4 v[kPer], v2[kPer];
+  auto load_plane = [&](int gz) {
+    const bool zin = gz >= 0 && gz < d;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float v = acc[m][nb][r] + (bias ? bias[cb + r] : 0.0f);
-        out[r] = static_cast<__bf16>(act(v, slope));
-      }
-      uint2 packed;
-      std::memcpy(&packed, out, 8);
-      *reinterpret_cast<uint2*>(y_nd + p * cout + cb) = packed;
-      if (y_cm) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) y_cm[static_cast<long long>(cb + r) * P + p] = out[r];
+    for (int j = 0; j < kPer; ++j) {
+      const int i = static_cast<int>(threadIdx.x) + 256 * j;
+      const int c8 = i % kC8, pos = i / kC8;
+      const int gy = h0 + pos / kTW - 1, gx = pos % kTW - 1;
+      const bool ok = zin && i < kPlane && gy >= 0 && gy < h && gx >= 0 && gx < kW;
+      long long q;
+      if constexpr (SRC == kSrcUp)
+        q = ((static_cast<long long>(nn) * (d >> 1) + (gz >> 1)) * (h >> 1) + (gy >> 1)) * (kW >> 1) + (gx >> 1);
+      else
+        q = ((static_cast<long long>(nn) * d + gz) * h + gy) * kW + gx;
+      // An element outside the volume reads the tensor's first one, always valid.
+      q = ok ? q * CIN + 8 * c8 : 0;
+      v[j] = *reinterpret_cast<const u32x4*>(x + q);
+      if constexpr (SRC == kSrcAdd) v2[j] = *reinterpret_cast<const u32x4*>(x2 + q);
+      if (!ok) {
+        v[j] = u32x4{0u, 0u, 0u, 0u};
+        if constexpr (SRC == kSrcAdd) v2[j] = u32x4{0u, 0u, 0u, 0u};
       }
     }
+  };
+  auto store_plane = [&](int slot) {
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const int i = static_cast<int>(threadIdx.x) + 256 * j;
+      const int c8 = i % kC8, pos = i / kC8;
+      u32x4 val = v[j];
+      if constexpr (SRC == kSrcAdd)
+        val = __builtin_bit_cast(u32x4, add8(__builtin_bit_cast(bf16x8, v[j]), __builtin_bit_cast(bf16x8, v2[j])));
+      if (i < kPlane) ring[slot * kPlane + (c8 / kPosUnits) * kHalf + pos * kPosUnits + c8 % kPosUnits] = val;
+    }
+  };
+
+  // Weight fragments of every k-step (zero past K).
+  bf16x8 a[kSteps][TM];
+#pragma unroll
+  for (int s = 0; s < kSteps; ++s) {
+    const int k = 32 * s + 8 * kg;
+    const bool in = k < K;
+    const int tap = in ? k / kKC : 0, c = in ? k % kKC : 0;
+#pragma unroll
+    for (int m = 0; m < TM; ++m) {
+      a[s][m] = load8(wt + (static_cast<long long>(tap) * cout + 16 * m + col) * CIN + c);
+      if (!in) a[s][m] = zero8();
+    }
+  }
+  // A lane's part of a fragment's place in the ring: its row and column, and its channels
+  // where the four lane groups share a tap (their tap where they do not is added per step).
+  const int lane_units = (wave * kTW + col) * kPosUnits +
+                         (kC8 == 4 ? (kg >> 1) * kHalf + (kg & 1) : kC8 == 2 ? (kg & 1) : 0);
+
+  load_plane(z0 - 1);
+  store_plane(0);
+  load_plane(z0);
+  store_plane(1);
+  load_plane(z0 + 1);
+  int slot = 2;                              // of the plane in registers
+  int pb[3] = {0, kPlane, 2 * kPlane};       // units of planes z - 1, z, z + 1
+  const long long P = static_cast<long long>(n) * d * h * kW;
+  for (int z = z0; z < z1; ++z) {
+    store_plane(slot);
+    __syncthreads();
+    const long long row = ((static_cast<long long>(nn) * d + z) * h + h0 + wave) * kW;
+    uint2 other[TM][4];
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb)
+        other[m][nb] = conv_other<EPI>(E, 16 * m + 4 * kg, row + 16 * nb + col, cout);
+    if (z + 1 < z1) load_plane(z + 2);
+    // Fragments of k-step s. Taps of the step's lane groups: kC8 groups share one.
+    auto load_b = [&](int s, bf16x8 (&b)[4]) {
+      int at;
+      if constexpr (kC8 == 4) {
+        at = pb[s / 9] + ((s / 3 % 3) * kTW + s % 3) * kPosUnits;
+      } else {
+        constexpr int kTaps = 4 / kC8;  // taps of a step
+        at = 0;
+#pragma unroll
+        for (int g = kTaps - 1; g >= 0; --g) {
+          const int tap = kTaps * s + g < 27 ? kTaps * s + g : 26;  // past K the weights are zero
+          const int u = pb[tap / 9] + ((tap / 3 % 3) * kTW + tap % 3) * kPosUnits;
+          at = kg / kC8 <= g ? u : at;
+        }
+      }
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) {
+        const u32x4 f = ring[lane_units + at + 16 * nb * kPosUnits];
+        std::memcpy(&b[nb], &f, 16);
+      }
+    };
+    f32x4 acc[TM][4];
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) acc[m][nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    bf16x8 b[2][4];
+    load_b(0, b[0]);
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      if (s + 1 < kSteps) load_b(s + 1, b[(s + 1) & 1]);
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) acc[m][nb] = mfma16(a[s][m], b[s & 1][nb], acc[m][nb]);
+    }
+#pragma unroll
+    for (int m = 0; m < TM; ++m) {
+      const int cb = 16 * m + 4 * kg;
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) {
+        const long long p = row + 16 * nb + col;
+        conv_store<EPI>(E, acc[m][nb], other[m][nb], cb, p, cout, P);
+      }
+    }
+    __syncthreads();  // plane z - 1 is read no more: the next plane takes its slot
+    const int first = pb[0];
+    pb[0] = pb[1];
+    pb[1] = pb[2];
+    pb[2] = first;
+    slot = slot == 2 ? 0 : slot + 1;
   }
 }
 
@@ -742,8 +931,18 @@ __global__ void __launch_bounds__(256) k_channel_sum(const __bf16* __restrict__ 
 
 // ------------------------------------------------------------------- elementwise
 //
-// Thread = (position p, 8-channel group g); p runs fastest so the channel-major
-// writes of a wave are contiguous.
+// Thread = (position p, 8-channel group g): a wave has 64 consecutive positions of one
+// group, so its channel-major writes are contiguous, and the next wave the same positions'
+// next group, so a position's line is fetched once (with all positions of a group before
+// the next group it came from memory once per group).
+struct Place {
+  long long p;
+  int g;
+};
+__device__ inline Place place(long long i, int groups) {
+  const long long wave = i >> 6;
+  return {(wave / groups << 6) + (i & 63), static_cast<int>(wave % groups)};
+}
 
 __device__ inline void store_both(__bf16* nd, __bf16* cm, long long P, int C, long long p, int g,
                                   const float* v) {
@@ -764,10 +963,8 @@ __global__ void k_act_bwd(const __bf16* __restrict__ y, const __bf16* __restrict
                           __bf16* __restrict__ dz_nd, __bf16* __restrict__ dz_cm, long long P,
                           int C, float slope) {
   const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int groups = C / 8;
-  if (i >= P * groups) return;
-  const long long p = i % P;
-  const int g = static_cast<int>(i / P);
+  const auto [p, g] = place(i, C / 8);
+  if (p >= P) return;
   const bf16x8 yv = load8(y + p * C + 8 * g);
   const bf16x8 gv = load8(dy + p * C + 8 * g);
   float v[8];
@@ -783,10 +980,8 @@ __global__ void k_act_bwd(const __bf16* __restrict__ y, const __bf16* __restrict
 __global__ void k_add(const __bf16* __restrict__ a, const __bf16* __restrict__ b,
                       __bf16* __restrict__ y_nd, __bf16* __restrict__ y_cm, long long P, int C) {
   const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int groups = C / 8;
-  if (i >= P * groups) return;
-  const long long p = i % P;
-  const int g = static_cast<int>(i / P);
+  const auto [p, g] = place(i, C / 8);
+  if (p >= P) return;
   const bf16x8 av = load8(a + p * C + 8 * g);
   const bf16x8 bv = load8(b + p * C + 8 * g);
   float v[8];
@@ -800,10 +995,8 @@ __global__ void k_pool_fwd(const __bf16* __restrict__ x, __bf16* __restrict__ y_
                            __bf16* __restrict__ y_cm, int n, int d, int h, int w, int C) {
   const long long P = static_cast<long long>(n) * d * h * w;
   const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int groups = C / 8;
-  if (i >= P * groups) return;
-  const long long p = i % P;
-  const int g = static_cast<int>(i / P);
+  const auto [p, g] = place(i, C / 8);
+  if (p >= P) return;
   long long t = p;
   const int xx = static_cast<int>(t % w);
   t /= w;
@@ -831,10 +1024,8 @@ __global__ void k_pool_bwd(const __bf16* __restrict__ dy, __bf16* __restrict__ d
                            int h2, int w2, int C) {
   const long long P = static_cast<long long>(n) * d2 * h2 * w2;
   const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int groups = C / 8;
-  if (i >= P * groups) return;
-  const long long p = i % P;
-  const int g = static_cast<int>(i / P);
+  const auto [p, g] = place(i, C / 8);
+  if (p >= P) return;
   long long t = p;
   const int xx = static_cast<int>(t % w2);
   t /= w2;
@@ -856,10 +1047,8 @@ __global__ void k_up_fwd(const __bf16* __restrict__ x, __bf16* __restrict__ y_nd
                          __bf16* __restrict__ y_cm, int n, int d2, int h2, int w2, int C) {
   const long long P = static_cast<long long>(n) * d2 * h2 * w2;
   const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int groups = C / 8;
-  if (i >= P * groups) return;
-  const long long p = i % P;
-  const int g = static_cast<int>(i / P);
+  const auto [p, g] = place(i, C / 8);
+  if (p >= P) return;
   long long t = p;
   const int xx = static_cast<int>(t % w2);
   t /= w2;
@@ -881,10 +1070,8 @@ __global__ void k_up_bwd(const __bf16* __restrict__ dy, __bf16* __restrict__ dx,
                          int h, int w, int C) {
   const long long P = static_cast<long long>(n) * d * h * w;
   const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int groups = C / 8;
-  if (i >= P * groups) return;
-  const long long p = i % P;
-  const int g = static_cast<int>(i / P);
+  const auto [p, g] = place(i, C / 8);
+  if (p >= P) return;
   long long t = p;
   const int xx = static_cast<int>(t % w);
   t /= w;
@@ -981,6 +1168,9 @@ unsigned int blocks_for(long long n, int threads) {
   return static_cast<unsigned int>((n + threads - 1) / threads);
 }
 
+// 256-thread workgroups of an elementwise kernel (place).
+unsigned int place_blocks(long long P, int C) { return blocks_for((P + 63) / 64 * 64 * (C / 8), 256); }
+
 hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 int launch_status() { return hipGetLastError() == hipSuccess ? HDN_OK : HDN_EHIP; }
@@ -1001,35 +1191,32 @@ namespace {
 // 64 -> 128), 1024 waves 37 and 52 (32^3 x 2, 32 -> 64).
 constexpr long long kFillWaves = 768;
 
-template <int SRC>
-int conv_fwd(const __bf16* xb, const __bf16* x2b, const __bf16* wb, const float* bias, __bf16* yb, __bf16* cb,
-             int n, int d, int h, int w, int cin, int cout, float slope, hipStream_t stream) {
+template <int SRC, int EPI>
+int conv_fwd(const __bf16* xb, const __bf16* x2b, const __bf16* wb, const Epilogue& E, int n, int d, int h, int w,
+             int cin, int cout, hipStream_t stream) {
   if (w == 64 && h % 4 == 0 && (cin == 16 || cin == 32) && (cout == 16 || (cout == 32 && cin == 16))) {
-    // Full-resolution layers: input staged in LDS (k_conv_fwd_tile).
-    const dim3 tiles(static_cast<unsigned int>(static_cast<long long>(n) * d * (h / 4)));
+    // Full-resolution layers: about 2048 workgroups, each over enough slices (6 or more)
+    // to spread the two extra planes it loads.
+    const long long columns = static_cast<long long>(n) * (h / 4);
+    const int zc = static_cast<int>(std::min<long long>(d, std::max<long long>(6, columns * d / 2048)));
+    const dim3 blocks(static_cast<unsigned int>(columns * ((d + zc - 1) / zc)));
     if (cin == 16 && cout == 32)
-      hipLaunchKernelGGL((k_conv_fwd_tile<2, 16, SRC>), tiles, dim3(256), 0, stream, xb, x2b, wb, bias, yb, cb, n,
-                         d, h, cout, slope);
+      hipLaunchKernelGGL((k_conv_fwd_march<2, 16, SRC, EPI>), blocks, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, cout, zc);
     else if (cin == 16)
-      hipLaunchKernelGGL((k_conv_fwd_tile<1, 16, SRC>), tiles, dim3(256), 0, stream, xb, x2b, wb, bias, yb, cb, n,
-                         d, h, cout, slope);
+      hipLaunchKernelGGL((k_conv_fwd_march<1, 16, SRC, EPI>), blocks, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, cout, zc);
     else
-      hipLaunchKernelGGL((k_conv_fwd_tile<1, 32, SRC>), tiles, dim3(256), 0, stream, xb, x2b, wb, bias, yb, cb, n,
-                         d, h, cout, slope);
+      hipLaunchKernelGGL((k_conv_fwd_march<1, 32, SRC, EPI>), blocks, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, cout, zc);
     return launch_status();
   }
   if (w == 32 && h % 8 == 0 && (cin == 16 || cin == 32 || cin == 64) && cout == 32) {
     // Half-resolution layers: the same staging, 8 rows of 32 per workgroup.
     const dim3 tiles(static_cast<unsigned int>(static_cast<long long>(n) * d * (h / 8)));
     if (cin == 16)
-      hipLaunchKernelGGL((k_conv_fwd_tile<2, 16, SRC, 32>), tiles, dim3(256), 0, stream, xb, x2b, wb, bias, yb, cb,
-                         n, d, h, cout, slope);
+      hipLaunchKernelGGL((k_conv_fwd_tile<2, 16, SRC, EPI, 32>), tiles, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, cout);
     else if (cin == 32)
-      hipLaunchKernelGGL((k_conv_fwd_tile<2, 32, SRC, 32>), tiles, dim3(256), 0, stream, xb, x2b, wb, bias, yb, cb,
-                         n, d, h, cout, slope);
+      hipLaunchKernelGGL((k_conv_fwd_tile<2, 32, SRC, EPI, 32>), tiles, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, cout);
     else
-      hipLaunchKernelGGL((k_conv_fwd_tile<2, 64, SRC, 32>), tiles, dim3(256), 0, stream, xb, x2b, wb, bias, yb, cb,
-                         n, d, h, cout, slope);
+      hipLaunchKernelGGL((k_conv_fwd_tile<2, 64, SRC, EPI, 32>), tiles, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, cout);
     return launch_status();
   }
   const long long P = static_cast<long long>(n) * d * h * w;
@@ -1039,23 +1226,18 @@ int conv_fwd(const __bf16* xb, const __bf16* x2b, const __bf16* wb, const float*
     const int ts = cout % 32 == 0 ? 2 : 1;
     const dim3 blocks(static_cast<unsigned int>(P / 64), static_cast<unsigned int>(cout / (16 * ts)));
     if (ts == 2)
-      hipLaunchKernelGGL((k_conv_fwd_split<2, SRC>), blocks, dim3(64 * kSplitWaves), 0, stream, xb, x2b, wb, bias, yb,
-                         cb, n, d, h, w, cin, cout, slope);
+      hipLaunchKernelGGL((k_conv_fwd_split<2, SRC>), blocks, dim3(64 * kSplitWaves), 0, stream, xb, x2b, wb, E, n, d, h, w, cin, cout);
     else
-      hipLaunchKernelGGL((k_conv_fwd_split<1, SRC>), blocks, dim3(64 * kSplitWaves), 0, stream, xb, x2b, wb, bias, yb,
-                         cb, n, d, h, w, cin, cout, slope);
+      hipLaunchKernelGGL((k_conv_fwd_split<1, SRC>), blocks, dim3(64 * kSplitWaves), 0, stream, xb, x2b, wb, E, n, d, h, w, cin, cout);
     return launch_status();
   }
   const dim3 grid(static_cast<unsigned int>((P + 255) / 256), static_cast<unsigned int>(cout / (16 * tm)));
   if (tm == 4)
-    hipLaunchKernelGGL((k_conv_fwd<4, SRC>), grid, dim3(256), 0, stream, xb, x2b, wb, bias, yb, cb, n, d, h, w,
-                       cin, cout, slope);
+    hipLaunchKernelGGL((k_conv_fwd<4, SRC>), grid, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, w, cin, cout);
   else if (tm == 2)
-    hipLaunchKernelGGL((k_conv_fwd<2, SRC>), grid, dim3(256), 0, stream, xb, x2b, wb, bias, yb, cb, n, d, h, w,
-                       cin, cout, slope);
+    hipLaunchKernelGGL((k_conv_fwd<2, SRC>), grid, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, w, cin, cout);
   else
-    hipLaunchKernelGGL((k_conv_fwd<1, SRC>), grid, dim3(256), 0, stream, xb, x2b, wb, bias, yb, cb, n, d, h, w,
-                       cin, cout, slope);
+    hipLaunchKernelGGL((k_conv_fwd<1, SRC>), grid, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, w, cin, cout);
   return launch_status();
 }
 
@@ -1130,9 +1312,12 @@ int scratch_for_current_device(void* stream, float** out) {
 
 extern "C" {
 
-int hdn_conv3d_fwd_src(const void* x, const void* x2, int src, const void* wt, const float* bias, void* y_nd,
-                       void* y_cm, int n, int d, int h, int w, int cin, int cout, float slope, void* stream) {
-  if (!x || !wt || !y_nd || !shape_ok(n, d, h, w)) return HDN_EINVAL;
+int hdn_conv3d_fwd_fused(const void* x, const void* x2, int src, const void* wt, const float* bias, const void* skip,
+                         const void* inp, int c_in, float* pred, void* y_nd, void* y_cm, int n, int d, int h, int w,
+                         int cin, int cout, float slope, void* stream) {
+  if (!x || !wt || !shape_ok(n, d, h, w)) return HDN_EINVAL;
+  if (pred ? (!inp || c_in < 1 || skip || src != kSrcPlain) : !y_nd) return HDN_EINVAL;
+  if (skip && src != kSrcPlain && src != kSrcUp) return HDN_EINVAL;
   const long long P = static_cast<long long>(n) * d * h * w;
   if (P % 64 != 0 || cin % 16 != 0 || cin < 16 || cout % 16 != 0 || cout < 16) return HDN_EINVAL;
   if (src == kSrcUp && (d % 2 || h % 2 || w % 2)) return HDN_EINVAL;
@@ -1141,12 +1326,28 @@ int hdn_conv3d_fwd_src(const void* x, const void* x2, int src, const void* wt, c
   const __bf16* xb = static_cast<const __bf16*>(x);
   const __bf16* x2b = static_cast<const __bf16*>(x2);
   const __bf16* wb = static_cast<const __bf16*>(wt);
-  __bf16* yb = static_cast<__bf16*>(y_nd);
-  __bf16* cb = static_cast<__bf16*>(y_cm);
-  if (src == kSrcUp) return conv_fwd<kSrcUp>(xb, nullptr, wb, bias, yb, cb, n, d, h, w, cin, cout, slope, as_stream(stream));
-  if (src == kSrcAdd) return conv_fwd<kSrcAdd>(xb, x2b, wb, bias, yb, cb, n, d, h, w, cin, cout, slope, as_stream(stream));
-  if (src == kSrcLow8) return conv_fwd<kSrcLow8>(xb, nullptr, wb, bias, yb, cb, n, d, h, w, cin, cout, slope, as_stream(stream));
-  return conv_fwd<kSrcPlain>(xb, nullptr, wb, bias, yb, cb, n, d, h, w, cin, cout, slope, as_stream(stream));
+  const Epilogue E{bias,
+                   slope,
+                   static_cast<const __bf16*>(skip),
+                   static_cast<__bf16*>(y_nd),
+                   static_cast<__bf16*>(y_cm),
+                   pred,
+                   static_cast<const __bf16*>(inp),
+                   c_in};
+  const hipStream_t s = as_stream(stream);
+  if (pred) return conv_fwd<kSrcPlain, kEpiPred>(xb, nullptr, wb, E, n, d, h, w, cin, cout, s);
+  if (skip && src == kSrcUp) return conv_fwd<kSrcUp, kEpiSkip>(xb, nullptr, wb, E, n, d, h, w, cin, cout, s);
+  if (skip) return conv_fwd<kSrcPlain, kEpiSkip>(xb, nullptr, wb, E, n, d, h, w, cin, cout, s);
+  if (src == kSrcUp) return conv_fwd<kSrcUp, kEpiPlain>(xb, nullptr, wb, E, n, d, h, w, cin, cout, s);
+  if (src == kSrcAdd) return conv_fwd<kSrcAdd, kEpiPlain>(xb, x2b, wb, E, n, d, h, w, cin, cout, s);
+  if (src == kSrcLow8) return conv_fwd<kSrcLow8, kEpiPlain>(xb, nullptr, wb, E, n, d, h, w, cin, cout, s);
+  return conv_fwd<kSrcPlain, kEpiPlain>(xb, nullptr, wb, E, n, d, h, w, cin, cout, s);
+}
+
+int hdn_conv3d_fwd_src(const void* x, const void* x2, int src, const void* wt, const float* bias, void* y_nd,
+                       void* y_cm, int n, int d, int h, int w, int cin, int cout, float slope, void* stream) {
+  return hdn_conv3d_fwd_fused(x, x2, src, wt, bias, nullptr, nullptr, 0, nullptr, y_nd, y_cm, n, d, h, w, cin, cout,
+                              slope, stream);
 }
 
 int hdn_conv3d_fwd(const void* x, const void* wt, const float* bias, void* y_nd, void* y_cm, int n,
@@ -1198,7 +1399,7 @@ int hdn_channel_sum(const void* cm, float* part, long long P, int C, int splits,
 int hdn_act_bwd(const void* y, const void* dy, void* dz_nd, void* dz_cm, long long P, int C,
                 float slope, void* stream) {
   if (!y || !dy || !dz_nd || P < 1 || C % 8 != 0) return HDN_EINVAL;
-  hipLaunchKernelGGL(k_act_bwd, dim3(blocks_for(P * (C / 8), 256)), dim3(256), 0, as_stream(stream),
+  hipLaunchKernelGGL(k_act_bwd, dim3(place_blocks(P, C)), dim3(256), 0, as_stream(stream),
                      static_cast<const __bf16*>(y), static_cast<const __bf16*>(dy),
                      static_cast<__bf16*>(dz_nd), static_cast<__bf16*>(dz_cm), P, C, slope);
   return launch_status();
@@ -1206,7 +1407,7 @@ int hdn_act_bwd(const void* y, const void* dy, void* dz_nd, void* dz_cm, long lo
 
 int hdn_add(const void* a, const void* b, void* y_nd, void* y_cm, long long P, int C, void* stream) {
   if (!a || !b || !y_nd || P < 1 || C % 8 != 0) return HDN_EINVAL;
-  hipLaunchKernelGGL(k_add, dim3(blocks_for(P * (C / 8), 256)), dim3(256), 0, as_stream(stream),
+  hipLaunchKernelGGL(k_add, dim3(place_blocks(P, C)), dim3(256), 0, as_stream(stream),
                      static_cast<const __bf16*>(a), static_cast<const __bf16*>(b),
                      static_cast<__bf16*>(y_nd), static_cast<__bf16*>(y_cm), P, C);
   return launch_status();
@@ -1216,7 +1417,7 @@ int hdn_pool_fwd(const void* x, void* y_nd, void* y_cm, int n, int d, int h, int
                  void* stream) {
   if (!x || !y_nd || !shape_ok(n, d, h, w) || C % 8 != 0) return HDN_EINVAL;
   const long long P = static_cast<long long>(n) * d * h * w;
-  hipLaunchKernelGGL(k_pool_fwd, dim3(blocks_for(P * (C / 8), 256)), dim3(256), 0, as_stream(stream),
+  hipLaunchKernelGGL(k_pool_fwd, dim3(place_blocks(P, C)), dim3(256), 0, as_stream(stream),
                      static_cast<const __bf16*>(x), static_cast<__bf16*>(y_nd),
                      static_cast<__bf16*>(y_cm), n, d, h, w, C);
   return launch_status();
@@ -1226,7 +1427,7 @@ int hdn_pool_bwd(const void* dy, void* dx, int n, int d2, int h2, int w2, int C,
   if (!dy || !dx || !shape_ok(n, d2, h2, w2) || C % 8 != 0 || d2 % 2 || h2 % 2 || w2 % 2)
     return HDN_EINVAL;
   const long long P = static_cast<long long>(n) * d2 * h2 * w2;
-  hipLaunchKernelGGL(k_pool_bwd, dim3(blocks_for(P * (C / 8), 256)), dim3(256), 0, as_stream(stream),
+  hipLaunchKernelGGL(k_pool_bwd, dim3(place_blocks(P, C)), dim3(256), 0, as_stream(stream),
                      static_cast<const __bf16*>(dy), static_cast<__bf16*>(dx), n, d2, h2, w2, C);
   return launch_status();
 }
@@ -1236,7 +1437,7 @@ int hdn_up_fwd(const void* x, void* y_nd, void* y_cm, int n, int d2, int h2, int
   if (!x || !y_nd || !shape_ok(n, d2, h2, w2) || C % 8 != 0 || d2 % 2 || h2 % 2 || w2 % 2)
     return HDN_EINVAL;
   const long long P = static_cast<long long>(n) * d2 * h2 * w2;
-  hipLaunchKernelGGL(k_up_fwd, dim3(blocks_for(P * (C / 8), 256)), dim3(256), 0, as_stream(stream),
+  hipLaunchKernelGGL(k_up_fwd, dim3(place_blocks(P, C)), dim3(256), 0, as_stream(stream),
                      static_cast<const __bf16*>(x), static_cast<__bf16*>(y_nd),
                      static_cast<__bf16*>(y_cm), n, d2, h2, w2, C);
   return launch_status();
@@ -1245,7 +1446,7 @@ int hdn_up_fwd(const void* x, void* y_nd, void* y_cm, int n, int d2, int h2, int
 int hdn_up_bwd(const void* dy, void* dx, int n, int d, int h, int w, int C, void* stream) {
   if (!dy || !dx || !shape_ok(n, d, h, w) || C % 8 != 0) return HDN_EINVAL;
   const long long P = static_cast<long long>(n) * d * h * w;
-  hipLaunchKernelGGL(k_up_bwd, dim3(blocks_for(P * (C / 8), 256)), dim3(256), 0, as_stream(stream),
+  hipLaunchKernelGGL(k_up_bwd, dim3(place_blocks(P, C)), dim3(256), 0, as_stream(stream),
                      static_cast<const __bf16*>(dy), static_cast<__bf16*>(dx), n, d, h, w, C);
   return launch_status();
 }

@@ -63,6 +63,8 @@ def _lib():
         "hdn_conv3d_fwd": [_c_void, _c_void, _c_void, _c_void, _c_void, i, i, i, i, i, i, f, _c_void],
         "hdn_conv3d_fwd_src": [_c_void, _c_void, i, _c_void, _c_void, _c_void, _c_void, i, i, i, i, i, i, f,
                                _c_void],
+        "hdn_conv3d_fwd_fused": [_c_void, _c_void, i, _c_void, _c_void, _c_void, _c_void, i, _c_void, _c_void, _c_void,
+                                 i, i, i, i, i, i, f, _c_void],
         "hdn_conv3d_wgrad": [_c_void, _c_void, _c_void, i, i, i, i, i, i, i, _c_void],
         "hdn_conv3d_wgrad_noalloc": [_c_void, _c_void, _c_void, i, i, i, i, i, i, i, _c_void],
         "hdn_reduce_splits": [_c_void, _c_void, _c_ll, i, _c_void],
@@ -302,24 +304,36 @@ class Conv3dDenoiser:
         out, _ = conv("head", *t, 0, activate=False)
         return out, cache
 
-    def _infer(self, x, dims):
+    def _infer(self, x, dims, predict: bool = False):
         """The forward pass without anything kept for the backward: no channel-major
-        copies, and each upsampling or skip addition read by the next convolution
-        instead of stored (identical values, so identical outputs)."""
+        copies, each upsampling read by the next convolution and each skip addition made in
+        the store of the convolution before it (identical values, so identical outputs).
+        Returns the head output, or with ``predict`` the prediction [N][D][H][W], which the
+        head's store then makes."""
+        torch = _torch()
         L = self.layers
         c0, c1, c2, _ = self.widths
 
-        def conv(name, inp, lvl, activate=True, x2=None, src=0):
-            return self._conv(L[name], inp, dims[lvl], activate, False, x2=x2, src=src)[0]
+        def conv(name, inp, lvl, src=0, skip=None):
+            n, d, h, w = dims[lvl]
+            lay = L[name]
+            head = name == "head"
+            pred = torch.empty((n, d, h, w), dtype=torch.float32, device=x.device) if head and predict else None
+            y = None if pred is not None else torch.empty((n, d, h, w, lay.cout), dtype=torch.bfloat16,
+                                                          device=x.device)
+            _call("hdn_conv3d_fwd_fused", _ptr(inp), None, src, _ptr(lay.wf), _ptr(lay.b), _ptr(skip), _ptr(x),
+                  CIN_PAD, _ptr(pred), _ptr(y), None, n, d, h, w, lay.cin, lay.cout, 1.0 if head else SLOPE,
+                  self._stream())
+            return y if pred is None else pred
 
         s0 = conv("e0b", conv("e0a", x, 0, src=3), 0)
         s1 = conv("e1b", conv("e1a", self._pool(s0, dims[0], c0, False)[0], 1), 1)
         s2 = conv("e2b", conv("e2a", self._pool(s1, dims[1], c1, False)[0], 2), 2)
         t = conv("e3b", conv("e3a", self._pool(s2, dims[2], c2, False)[0], 3), 3)
-        t = conv("d2b", conv("d2a", t, 2, src=1), 2, x2=s2, src=2)
-        t = conv("d1b", conv("d1a", t, 1, src=1), 1, x2=s1, src=2)
-        t = conv("d0b", conv("d0a", t, 0, src=1), 0, x2=s0, src=2)
-        return conv("head", t, 0, activate=False)
+        t = conv("d2b", conv("d2a", t, 2, src=1, skip=s2), 2)
+        t = conv("d1b", conv("d1a", t, 1, src=1, skip=s1), 1)
+        t = conv("d0b", conv("d0a", t, 0, src=1, skip=s0), 0)
+        return conv("head", t, 0)
 
     # ---------------------------------------------------------------- backward
 
@@ -426,13 +440,8 @@ class Conv3dDenoiser:
 
     def predict_tensor(self, x):
         """Prediction [N][D][H][W] (float32) for a packed input batch."""
-        torch = _torch()
-        out, _ = self.forward(x, None, keep=False)
-        P = out.numel() // HEAD_OUT
-        pred = torch.empty(P, dtype=torch.float32, device=x.device)
-        _call("hdn_loss", _ptr(out), _ptr(x), HEAD_OUT, CIN_PAD, None, None, None, None, _ptr(pred),
-              None, P, 1.0, self._stream())
-        return pred.reshape(x.shape[:4])
+        n, d, h, w, _ = x.shape
+        return self._infer(x, [(n, d >> k, h >> k, w >> k) for k in range(4)], predict=True)
 
 
 # ------------------------------------------------------------------------ data

@@ -61,6 +61,57 @@ def test_forward_split_and_whole(dn, shape, cin, cout):  # noqa: F811
     np.testing.assert_array_equal(_np(y_cm), _np(y).reshape(-1, cout).T)
 
 
+# Full-resolution rows: one slice, slices off the marching chunks (6 and 7), several chunks,
+# each channel pair; the other kernels' shapes for the fused steps.
+MARCHED = [((1, 1, 4, 64), 16, 16), ((2, 6, 4, 64), 16, 32), ((1, 7, 8, 64), 32, 16), ((1, 20, 4, 64), 16, 16)]
+
+
+@pytest.mark.parametrize("shape, cin, cout", MARCHED)
+def test_forward_marched(dn, shape, cin, cout):  # noqa: F811
+    test_forward_split_and_whole(dn, shape, cin, cout)
+
+
+@pytest.mark.parametrize("shape, cin, cout", MARCHED[1:] + [((1, 2, 8, 32), 32, 32), ((1, 2, 8, 32), 64, 32),
+                                                            ((1, 2, 4, 16), 64, 64), ((3, 16, 32, 32), 16, 16)])
+@pytest.mark.parametrize("upsampled", (False, True))
+def test_fused_steps_equal_separate_calls(dn, shape, cin, cout, upsampled):  # noqa: F811
+    """The skip addition and the prediction made in a convolution's store, against hdn_add
+    and hdn_loss on its stored output, bit for bit."""
+    import torch
+
+    n, d, h, w = shape
+    d -= d % 2 if upsampled else 0
+    shape = (n, d, h, w)
+    P = n * d * h * w
+    rng = np.random.default_rng(cin)
+    src = (n, d // 2, h // 2, w // 2) if upsampled else shape
+    x = _dev(_bf(rng.standard_normal(src + (cin,))))
+    wt = _dev(_bf(rng.standard_normal((27, cout, cin)) * 0.1))
+    bias = _dev(torch.from_numpy(rng.standard_normal(cout).astype(np.float32)))
+    skip = _dev(_bf(rng.standard_normal(shape + (cout,))))
+    y, want, got = (torch.zeros(shape + (cout,), dtype=torch.bfloat16, device="cuda:0") for _ in range(3))
+    args = (n, d, h, w, cin, cout, 0.1, None)
+
+    def fused(skip_ptr, inp, c_in, pred, out):
+        dn._call("hdn_conv3d_fwd_fused", x.data_ptr(), None, int(upsampled), wt.data_ptr(), bias.data_ptr(), skip_ptr,
+                 inp, c_in, pred, out, None, *args)
+
+    dn._call("hdn_conv3d_fwd_src", x.data_ptr(), None, int(upsampled), wt.data_ptr(), bias.data_ptr(), y.data_ptr(),
+             None, *args)
+    dn._call("hdn_add", y.data_ptr(), skip.data_ptr(), want.data_ptr(), None, P, cout, None)
+    fused(skip.data_ptr(), None, 0, None, got.data_ptr())
+    assert torch.equal(got, want)
+    pred, ref = (torch.zeros(P, device="cuda:0") for _ in range(2))
+    if upsampled:
+        with pytest.raises(ValueError):
+            fused(None, skip.data_ptr(), cout, pred.data_ptr(), None)
+        return
+    dn._call("hdn_loss", y.data_ptr(), skip.data_ptr(), cout, cout, None, None, None, None, ref.data_ptr(), None, P,
+             1.0, None)
+    fused(None, skip.data_ptr(), cout, pred.data_ptr(), None)
+    assert torch.equal(pred, ref)
+
+
 @pytest.mark.parametrize("splits, length", [(1, 5), (16, 64), (17, 65), (700, 6912)])
 def test_reduce_splits(dn, splits, length):  # noqa: F811
     import torch
