@@ -53,6 +53,11 @@ int hsp_apply(hsp_matrix *m, const double *weights, int n_w, long long row_begin
 int hsp_apply_device(hsp_matrix *m, const void *weights_device, int n_w, long long row_begin,
                      long long row_end, int precision, void *out_device, double *kernel_ms);
 
+/* hsp_apply into the internal product, copied to the host array out [row_end - row_begin]
+ * [n_w] (float64 or float32, as precision) before it returns: hsp_apply and hsp_fetch in one
+ * call, with one wait where weights and product are small (1 MiB each). */
+int hsp_apply_host(hsp_matrix* m, const double* weights, int n_w, long long row_begin, long long row_end,
+                   int precision, void* out, double* kernel_ms);
 /* Rows [row_begin, row_end) of the last product kept in the internal buffer, to host
  * memory [rows][n_w] of that product's element type. */
 int hsp_fetch(hsp_matrix *m, long long row_begin, long long row_end, void *host);

@@ -34,6 +34,7 @@ def _lib():
         "hsp_destroy": (None, [_c_void]),
         "hsp_last_error": (ctypes.c_char_p, [_c_void]),
         "hsp_apply": (ctypes.c_int, [_c_void, f64p, ctypes.c_int, ll, ll, ctypes.c_int, _c_void, f64p]),
+        "hsp_apply_host": (ctypes.c_int, [_c_void, f64p, ctypes.c_int, ll, ll, ctypes.c_int, _c_void, f64p]),
         "hsp_apply_device": (ctypes.c_int, [_c_void, _c_void, ctypes.c_int, ll, ll, ctypes.c_int, _c_void, f64p]),
         "hsp_fetch": (ctypes.c_int, [_c_void, ll, ll, _c_void]),
         "hsp_csr": (ctypes.c_int, [_c_void, i64p, ctypes.POINTER(ctypes.c_int32), _c_void]),
@@ -131,13 +132,16 @@ class DeviceDij:
             raise ValueError(f"weights shape {w.shape}: expected ({self.n_cols},) or ({self.n_cols}, n_w)")
         r0, r1 = (0, self.n_rows) if rows is None else (int(rows[0]), int(rows[1]))
         ms = ctypes.c_double()
-        self._check(_lib().hsp_apply(self._h, w2.ctypes.data_as(ctypes.POINTER(ctypes.c_double)),
-                                     int(w2.shape[1]), r0, r1, code, None, ctypes.byref(ms)), "hsp_apply")
-        self.last_kernel_ms = float(ms.value)
+        wp = w2.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+        n_w = int(w2.shape[1])
         if not fetch:
+            self._check(_lib().hsp_apply(self._h, wp, n_w, r0, r1, code, None, ctypes.byref(ms)), "hsp_apply")
+            self.last_kernel_ms = float(ms.value)
             return None
-        out = np.empty((r1 - r0, w2.shape[1]), dtype=dtype)
-        self._check(_lib().hsp_fetch(self._h, r0, r1, out.ctypes.data), "hsp_fetch")
+        out = np.empty((max(r1 - r0, 0), n_w), dtype=dtype)
+        self._check(_lib().hsp_apply_host(self._h, wp, n_w, r0, r1, code, out.ctypes.data, ctypes.byref(ms)),
+                    "hsp_apply")
+        self.last_kernel_ms = float(ms.value)
         return out[:, 0] if single else out
 
     def apply_device(self, weights, out, rows: tuple[int, int] | None = None) -> float:

@@ -89,14 +89,14 @@ class ToyPlanProblem:
 
     @cached_property
     def _roi(self):
-        """The region's rows on the device, and each region row's role."""
+        """The region's rows on the device, and the region rows of the PTV and the OAR."""
         from pyradmc_amd.spmm import DeviceDij
 
         indptr, indices, values, n_voxels, n_cols = self._csc
         oar = self.oar if self.oar.size else np.zeros(n_voxels, dtype=bool)
         keep = self.ptv | oar
         rows = _Rows(indptr, indices, values, keep, n_cols)
-        return DeviceDij(rows, device=self.device), self.ptv[keep], oar[keep]
+        return DeviceDij(rows, device=self.device), np.flatnonzero(self.ptv[keep]), np.flatnonzero(oar[keep])
 
 
 def objective_and_gradient(problem: ToyPlanProblem, weights) -> tuple[float, np.ndarray]:
@@ -111,7 +111,7 @@ def objective_and_gradient(problem: ToyPlanProblem, weights) -> tuple[float, np.
     f = float(r_ptv @ r_ptv) / n_ptv
     a = np.zeros(d.size)
     a[in_ptv] = 2.0 / n_ptv * r_ptv
-    if in_oar.any():
+    if in_oar.size:
         r_oar = np.maximum(0.0, d[in_oar] - problem.oar_max * problem.prescription)
         n_oar = r_oar.size
         f += problem.oar_penalty * float(r_oar @ r_oar) / n_oar
