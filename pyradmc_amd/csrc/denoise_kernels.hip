@@ -21,6 +21,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <limits>
 #include <mutex>
 
 #include "../../include/hipdn.h"
@@ -212,119 +213,113 @@ __global__ void __launch_bounds__(256) k_conv_fwd(const __bf16* __restrict__ x,
 }
 
 // The same convolution where 64-position waves are too few to fill the chip (the deep
-// levels of a small batch): the kNW waves of a workgroup take the k-steps of one 64-position
-// block in turn, each loading its next step's operands before this step's MFMAs, and
-// their sums add in a fixed tree through LDS. Four 8^3 volumes of 128 -> 128 channels:
-// 130 us as one wave per block (108 k-steps, each waiting for its loads), 22 us split;
-// 16^3, 64 -> 64: 67 and 28 us.
-constexpr int kSplitWaves = 8;
-
-template <int TM, int SRC>
-__global__ void __launch_bounds__(64 * kSplitWaves) k_conv_fwd_split(
-    const __bf16* __restrict__ x, const __bf16* __restrict__ x2, const __bf16* __restrict__ wt,
-    Epilogue E, int n, int d, int h, int w, int cin, int cout) {
-  __shared__ f32x4 sums[kSplitWaves / 2][TM * 4][64];
+// levels of a small batch). A wave's k-steps are a serial chain that waits for memory at
+// every step, so a wave takes M x M tiles of 16 positions and 16 output channels (4 tm / M^2
+// times as many waves as k_conv_fwd<tm> has) and loads its operands 8 (M = 1)
+// or 4 k-steps ahead of their MFMAs. Bound by the instructions of a step's addresses with
+// one wave per SIMD (37 us instead of 26 with the tap in vector registers), then by L2
+// reads, which M = 2 halves. The k-steps keep k_conv_fwd's order: identical sums.
+// (Splitting the k-steps over the waves of a workgroup took 22 and 28 us for the two below,
+// but its sums round differently, which moved the weight gradients of a training step by
+// 3 %.) Four 8^3 volumes of 128 -> 128 channels: 127 us as k_conv_fwd,
+// 26 us so; four 16^3, 64 -> 64: 67 and 28 us.
+template <int M, bool WIDE, int SRC>
+__global__ void __launch_bounds__(256) k_conv_fwd_deep(const __bf16* __restrict__ x, const __bf16* __restrict__ x2,
+                                                       const __bf16* __restrict__ wt, Epilogue E, int n, int d, int h,
+                                                       int w, int cin, int cout) {
+  constexpr int kDeep = M == 1 ? 8 : 4;
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const long long P = static_cast<long long>(n) * d * h * w;
-  const long long p0 = static_cast<long long>(blockIdx.x) * 64;
-  const int co0 = blockIdx.y * 16 * TM;
   const int col = lane & 15;
   const int kg = lane >> 4;
+  const int P = n * d * h * w;  // P * cin and 27 * cin * cout fit an int (conv_fwd)
+  const int co0 = blockIdx.y * 16 * M;
+  const int p0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 16 * M;
+  if (p0 >= P) return;  // P % 64 == 0: the other waves' positions are all inside
 
-  int pn[4], pz[4], py[4], px[4];
-#pragma unroll
-  for (int nb = 0; nb < 4; ++nb) {
-    long long t = p0 + 16 * nb + col;
-    px[nb] = static_cast<int>(t % w);
-    t /= w;
-    py[nb] = static_cast<int>(t % h);
-    t /= h;
-    pz[nb] = static_cast<int>(t % d);
-    pn[nb] = static_cast<int>(t / d);
-  }
-
-  f32x4 acc[TM][4];
-#pragma unroll
-  for (int m = 0; m < TM; ++m)
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb) acc[m][nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
+  // This lane's tap and first channel in the next k-step to load. Where the channels per tap
+  // are a multiple of 32 all lanes of a step share a tap and what depends on it is scalar.
   const int kc = SRC == kSrcLow8 ? 8 : cin;  // channels read per tap
-  const int K = 27 * kc;
-  // Operands of k-step k0 (zero past K). A position outside the volume reads the tensor's
-  // first element, always valid, and is replaced by zero.
-  auto load = [&](int k0, bf16x8 (&a)[TM], bf16x8 (&b)[4]) {
-    const int k = k0 + 8 * kg;
-    const bool in = k < K;
-    const int tap = in ? k / kc : 0;
-    const int c = in ? k - tap * kc : 0;
-    const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
+  const int steps = (27 * kc + 31) / 32;
+  int tap = WIDE ? 0 : 8 * kg / kc;
+  int c = WIDE ? 0 : 8 * kg - tap * kc;
+  const int lane_c = WIDE ? 8 * kg : 0;
+
+  int pn[M], pz[M], py[M], px[M], inside[M], at[M];  // inside: bit tap, the tap's voxel exists
 #pragma unroll
-    for (int m = 0; m < TM; ++m) {
-      a[m] = load8(wt + (static_cast<long long>(tap) * cout + co0 + 16 * m + col) * cin + c);
-      if (!in) a[m] = zero8();
-    }
+  for (int i = 0; i < M; ++i) {
+    const int p = p0 + 16 * i + col;
+    int t = p;
+    px[i] = t % w;
+    t /= w;
+    py[i] = t % h;
+    t /= h;
+    pz[i] = t % d;
+    pn[i] = t / d;
+    const int xs = (px[i] > 0) | 2 | (px[i] < w - 1) << 2;
+    const int ys = (py[i] > 0) | 1 << 3 | (py[i] < h - 1) << 6;
+    const int zs = (pz[i] > 0) | 1 << 9 | (pz[i] < d - 1) << 18;
+    inside[i] = xs * ys * zs;  // no two of the products share a bit
+    at[i] = p * cin + lane_c;
+  }
+
+  bf16x8 a[kDeep][M], b[kDeep][M];
+  bool in[kDeep], ok[kDeep][M];
+  // What lies past the last tap or outside the volume reads the tensor's first element,
+  // always valid, and is replaced by zero where it is used: a replacement here would wait
+  // for the load.
+  auto load = [&](int j) {
+    in[j] = tap < 27;
+    const int tp = in[j] ? tap : 0;
+    const int dz = tp / 9 - 1, dy = tp / 3 % 3 - 1, dx = tp % 3 - 1;
+    const int from = in[j] ? tp * cout * cin + c : 0;
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      const int zz = pz[nb] + dz, yy = py[nb] + dy, xx = px[nb] + dx;
-      const bool ok = in && zz >= 0 && zz < d && yy >= 0 && yy < h && xx >= 0 && xx < w;
-      long long q;
+    for (int m = 0; m < M; ++m) a[j][m] = load8(wt + (from + ((co0 + 16 * m + col) * cin + lane_c)));
+    const int shift = ((dz * h + dy) * w + dx) * cin + c;
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      ok[j][i] = in[j] && (inside[i] >> tp & 1);
+      int q = at[i] + shift;
       if constexpr (SRC == kSrcUp)
-        q = ((static_cast<long long>(pn[nb]) * (d >> 1) + (zz >> 1)) * (h >> 1) + (yy >> 1)) * (w >> 1) + (xx >> 1);
-      else
-        q = ((static_cast<long long>(pn[nb]) * d + zz) * h + yy) * w + xx;
-      q = ok ? q * cin + c : 0;
-      b[nb] = load8(x + q);
-      if constexpr (SRC == kSrcAdd) b[nb] = add8(b[nb], load8(x2 + q));
-      if (!ok) b[nb] = zero8();
+        q = (((pn[i] * (d >> 1) + (pz[i] + dz >> 1)) * (h >> 1) + (py[i] + dy >> 1)) * (w >> 1) + (px[i] + dx >> 1)) * cin +
+            lane_c + c;
+      q = ok[j][i] ? q : 0;
+      b[j][i] = load8(x + q);
+      if constexpr (SRC == kSrcAdd) b[j][i] = add8(b[j][i], load8(x2 + q));
     }
+    for (c += 32; c >= kc; c -= kc) ++tap;
   };
-  auto mfmas = [&](const bf16x8 (&a)[TM], const bf16x8 (&b)[4]) {
 #pragma unroll
-    for (int m = 0; m < TM; ++m)
+  for (int j = 0; j < kDeep; ++j) load(j);
+  f32x4 acc[M][M];
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb) acc[m][nb] = mfma16(a[m], b[nb], acc[m][nb]);
-  };
-  constexpr int kStep = 32 * kSplitWaves;
-  bf16x8 a0[TM], a1[TM], b0[4], b1[4];
-  int k0 = 32 * wave;
-  load(k0, a0, b0);
-  for (; k0 < K; k0 += 2 * kStep) {
-    load(k0 + kStep, a1, b1);
-    mfmas(a0, b0);
-    if (k0 + kStep >= K) break;
-    load(k0 + 2 * kStep, a0, b0);
-    mfmas(a1, b1);
-  }
-
-  for (int half = kSplitWaves / 2; half >= 1; half >>= 1) {
-    if (wave >= half && wave < 2 * half) {
+  for (int m = 0; m < M; ++m)
 #pragma unroll
-      for (int m = 0; m < TM; ++m)
+    for (int i = 0; i < M; ++i) acc[m][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s = 0; s < steps; s += kDeep) {
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) sums[wave - half][4 * m + nb][lane] = acc[m][nb];
-    }
-    __syncthreads();
-    if (wave < half) {
+    for (int j = 0; j < kDeep; ++j) {
+      if (s + j < steps) {
 #pragma unroll
-      for (int m = 0; m < TM; ++m)
+        for (int m = 0; m < M; ++m)
+          if (!WIDE && !in[j]) a[j][m] = zero8();
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) acc[m][nb] += sums[wave][4 * m + nb][lane];
-    }
-    __syncthreads();
-  }
-  if (wave != 0) return;
-
+        for (int i = 0; i < M; ++i) {
+          if (!ok[j][i]) b[j][i] = zero8();
 #pragma unroll
-  for (int m = 0; m < TM; ++m) {
-    const int cb = co0 + 16 * m + 4 * kg;
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      const long long p = p0 + 16 * nb + col;
-      conv_store<kEpiAny>(E, acc[m][nb], conv_other<kEpiAny>(E, cb, p, cout), cb, p, cout, P);
+          for (int m = 0; m < M; ++m) acc[m][i] = mfma16(a[j][m], b[j][i], acc[m][i]);
+        }
+      }
+      load(j);
     }
   }
+#pragma unroll
+  for (int m = 0; m < M; ++m)
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      const int cb = co0 + 16 * m + 4 * kg;
+      const long long p = p0 + 16 * i + col;
+      conv_store<kEpiAny>(E, acc[m][i], conv_other<kEpiAny>(E, cb, p, cout), cb, p, cout, P);
+    }
 }
 
 // The same convolution for rows of KW = 32 voxels (w == KW, h % (256 / KW) == 0,
@@ -1185,11 +1180,13 @@ extern "C" {
 
 namespace {
 
-// Below this many 64-position waves the k-steps are split over workgroups
-// (k_conv_fwd_split). Whole and split, us: 64 waves 125 and 22 (8^3 x 4, 128 -> 128),
-// 256 waves 66 and 27 (16^3 x 4, 64 -> 64), 768 waves 67 and 68 (12 x 8 x 8 x 32,
-// 64 -> 128), 1024 waves 37 and 52 (32^3 x 2, 32 -> 64).
-constexpr long long kFillWaves = 768;
+// Below kFillWaves 64-position waves a convolution runs as k_conv_fwd_deep, which reads more
+// per MFMA; below kPairWaves its waves take one tile instead of 2 x 2. Measured at 12 x 8 x 8
+// volumes of 128 -> 128 channels as k_conv_fwd, 2 x 2 tiles and single tiles: 576 waves 130,
+// 135 and 213 us, 384 waves 130, 93 and 143 us, 192 waves 128, 48 and 73 us; 8^3 volumes:
+// 128 waves 128, 48 and 50 us, 64 waves 128, 48 and 26 us.
+constexpr long long kFillWaves = 512;
+constexpr long long kPairWaves = 128;
 
 template <int SRC, int EPI>
 int conv_fwd(const __bf16* xb, const __bf16* x2b, const __bf16* wb, const Epilogue& E, int n, int d, int h, int w,
@@ -1221,14 +1218,17 @@ int conv_fwd(const __bf16* xb, const __bf16* x2b, const __bf16* wb, const Epilog
   }
   const long long P = static_cast<long long>(n) * d * h * w;
   const int tm = cout % 64 == 0 ? 4 : (cout % 32 == 0 ? 2 : 1);
-  // Fewer waves than kFillWaves leave SIMDs idle or waiting for loads: split the k-steps.
-  if (P / 64 * (cout / (16 * tm)) < kFillWaves) {
-    const int ts = cout % 32 == 0 ? 2 : 1;
-    const dim3 blocks(static_cast<unsigned int>(P / 64), static_cast<unsigned int>(cout / (16 * ts)));
-    if (ts == 2)
-      hipLaunchKernelGGL((k_conv_fwd_split<2, SRC>), blocks, dim3(64 * kSplitWaves), 0, stream, xb, x2b, wb, E, n, d, h, w, cin, cout);
-    else
-      hipLaunchKernelGGL((k_conv_fwd_split<1, SRC>), blocks, dim3(64 * kSplitWaves), 0, stream, xb, x2b, wb, E, n, d, h, w, cin, cout);
+  const long long waves = P / 64 * (cout / (16 * tm));
+  const long long most = std::numeric_limits<int>::max() / cin;
+  if (waves < kFillWaves && P <= most && 27LL * cout <= most) {
+    const int m = waves >= kPairWaves && cout % 32 == 0 ? 2 : 1;
+    const dim3 deep(static_cast<unsigned int>((P / 16 / m + 3) / 4), static_cast<unsigned int>(cout / 16 / m));
+    auto* kernel = &k_conv_fwd_deep<1, false, SRC>;
+    if (SRC != kSrcLow8 && cin % 32 == 0)
+      kernel = m == 2 ? &k_conv_fwd_deep<2, true, SRC> : &k_conv_fwd_deep<1, true, SRC>;
+    else if (m == 2)
+      kernel = &k_conv_fwd_deep<2, false, SRC>;
+    hipLaunchKernelGGL(kernel, deep, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, w, cin, cout);
     return launch_status();
   }
   const dim3 grid(static_cast<unsigned int>((P + 255) / 256), static_cast<unsigned int>(cout / (16 * tm)));

@@ -37,13 +37,15 @@ def test_weight_gradient_tiles(dn, shape, cin, cout, splits):  # noqa: F811
     np.testing.assert_allclose(_np(gw), ref, rtol=1e-4, atol=1e-4 * np.abs(ref).max())
 
 
-# Forward convolutions just below and at the wave count from which one wave takes a whole
-# 64-position block: the k-steps split over a workgroup, and not; few and many k-steps.
+# Forward convolutions by wave count: single tiles, 2 x 2 tiles (whole and partly filled last
+# workgroups) and, from 512 waves on, 64-position waves; taps shared by a k-step's lanes
+# (input channels in whole 32s) and not; an output channel count off the pairs.
 @pytest.mark.parametrize("shape, cin, cout", [
-    ((1, 1, 4, 16), 128, 128), ((3, 5, 8, 8), 128, 64), ((1, 8, 8, 8), 16, 48),
-    ((3, 15, 32, 32), 16, 16), ((3, 16, 32, 32), 16, 16),
+    ((1, 1, 4, 16), 128, 128), ((3, 5, 8, 8), 128, 64), ((1, 8, 8, 8), 16, 48), ((127, 1, 8, 8), 32, 32),
+    ((16, 8, 8, 8), 64, 64), ((43, 3, 8, 8), 16, 32), ((25, 3, 8, 8), 32, 48),
+    ((7, 73, 8, 8), 16, 16), ((8, 16, 16, 16), 16, 16),
 ])
-def test_forward_split_and_whole(dn, shape, cin, cout):  # noqa: F811
+def test_forward_by_wave_count(dn, shape, cin, cout):  # noqa: F811
     import torch
 
     rng = np.random.default_rng(cin + cout)
@@ -68,11 +70,12 @@ MARCHED = [((1, 1, 4, 64), 16, 16), ((2, 6, 4, 64), 16, 32), ((1, 7, 8, 64), 32,
 
 @pytest.mark.parametrize("shape, cin, cout", MARCHED)
 def test_forward_marched(dn, shape, cin, cout):  # noqa: F811
-    test_forward_split_and_whole(dn, shape, cin, cout)
+    test_forward_by_wave_count(dn, shape, cin, cout)
 
 
 @pytest.mark.parametrize("shape, cin, cout", MARCHED[1:] + [((1, 2, 8, 32), 32, 32), ((1, 2, 8, 32), 64, 32),
-                                                            ((1, 2, 4, 16), 64, 64), ((3, 16, 32, 32), 16, 16)])
+                                                            ((1, 2, 4, 16), 64, 64), ((2, 16, 16, 16), 64, 64),
+                                                            ((3, 16, 32, 32), 16, 16)])
 @pytest.mark.parametrize("upsampled", (False, True))
 def test_fused_steps_equal_separate_calls(dn, shape, cin, cout, upsampled):  # noqa: F811
     """The skip addition and the prediction made in a convolution's store, against hdn_add
