@@ -589,17 +589,18 @@ __global__ void __launch_bounds__(256, (CIN * TM == 16 ? 3 : 2) - (CIN == 16 && 
       for (int nb = 0; nb < 4; ++nb)
         other[m][nb] = conv_other<EPI>(E, 16 * m + 4 * kg, row + 16 * nb + col, cout);
     if (z + 1 < z1) load_plane(z + 2);
-    // Fragments of k-step s. Taps of the step's lane groups: kC8 groups share one.
+    // Fragments of k-step s (zero past K: a zero weight times an infinity is no zero). Taps
+    // of the step's lane groups: kC8 groups share one.
     auto load_b = [&](int s, bf16x8 (&b)[4]) {
+      constexpr int kTaps = 4 / kC8;  // taps of a step
       int at;
       if constexpr (kC8 == 4) {
         at = pb[s / 9] + ((s / 3 % 3) * kTW + s % 3) * kPosUnits;
       } else {
-        constexpr int kTaps = 4 / kC8;  // taps of a step
         at = 0;
 #pragma unroll
         for (int g = kTaps - 1; g >= 0; --g) {
-          const int tap = kTaps * s + g < 27 ? kTaps * s + g : 26;  // past K the weights are zero
+          const int tap = kTaps * s + g < 27 ? kTaps * s + g : 26;
           const int u = pb[tap / 9] + ((tap / 3 % 3) * kTW + tap % 3) * kPosUnits;
           at = kg / kC8 <= g ? u : at;
         }
@@ -608,6 +609,7 @@ __global__ void __launch_bounds__(256, (CIN * TM == 16 ? 3 : 2) - (CIN == 16 && 
       for (int nb = 0; nb < 4; ++nb) {
         const u32x4 f = ring[lane_units + at + 16 * nb * kPosUnits];
         std::memcpy(&b[nb], &f, 16);
+        if (kTaps * (s + 1) > 27 && kTaps * s + kg / kC8 >= 27) b[nb] = zero8();
       }
     };
     f32x4 acc[TM][4];

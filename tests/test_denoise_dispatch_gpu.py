@@ -73,6 +73,37 @@ def test_forward_marched(dn, shape, cin, cout):  # noqa: F811
     test_forward_by_wave_count(dn, shape, cin, cout)
 
 
+# An infinite activation gives the infinities that the oracle gives, in every build of the
+# marching kernel and in the others: what pads the last k-step past the 27 taps multiplies
+# zeros. (Positive weights: no sum meets infinities of both signs.)
+@pytest.mark.parametrize("src", (0, 1, 3))
+@pytest.mark.parametrize("shape, cin, cout", MARCHED + [((1, 2, 8, 32), 16, 32), ((1, 2, 4, 16), 16, 16),
+                                                        ((9, 16, 16, 16), 16, 16)])
+def test_an_infinity_stays_an_infinity(dn, shape, cin, cout, src):  # noqa: F811
+    import torch
+
+    n, d, h, w = shape
+    d += d % 2 if src == 1 else 0
+    rng = np.random.default_rng(cin + cout + src)
+    x = _rounded(rng.random((n, d, h, w, cin)))
+    if src == 1:
+        x = x[:, ::2, ::2, ::2].copy()
+    if src == 3:
+        x[..., 8:] = 0.0
+    x[0, 0, 0, 0, 3] = x[-1, -1, -1, -1, 5] = x[n // 2, x.shape[1] // 2, x.shape[2] // 2, x.shape[3] // 2, 0] = np.inf
+    wq = _rounded(rng.uniform(0.1, 1.0, (27, cout, cin)).astype(np.float32))
+    y = torch.empty((n, d, h, w, cout), dtype=torch.bfloat16, device="cuda:0")
+    xd, wd = _dev(_bf(x)), _dev(_bf(wq))
+    dn._call("hdn_conv3d_fwd_src", xd.data_ptr(), None, src, wd.data_ptr(), None, y.data_ptr(), None, n, d, h, w, cin,
+             cout, 0.1, None)
+    full = x.repeat(2, axis=1).repeat(2, axis=2).repeat(2, axis=3) if src == 1 else x
+    want, got = cr.conv_fwd(full, wq), _np(y)
+    assert np.isinf(want).any() and not np.isnan(want).any()
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(want))
+    finite = np.isfinite(want)
+    _close_bf16(got[finite], want[finite])
+
+
 @pytest.mark.parametrize("shape, cin, cout", MARCHED[1:] + [((1, 2, 8, 32), 32, 32), ((1, 2, 8, 32), 64, 32),
                                                             ((1, 2, 4, 16), 64, 64), ((2, 16, 16, 16), 64, 64),
                                                             ((3, 16, 32, 32), 16, 16)])
