@@ -3438,7 +3438,8 @@ static int enqueue_fold(hmc_ctx* ctx, int n_slots_used, const double* nhist, int
   HMC_HIP(ctx, hipGetLastError());
   ctx->sums_clear = false;
   if (n_slots_used >= ctx->dirty_slots) ctx->dirty_slots = 0;  // the fold zeroes what it reads
-  if (last) ctx->finalized = ctx->colmax_ready = true;
+  ctx->colmax_ready = last;  // any other fold changes what the maxima were taken over
+  if (last) ctx->finalized = true;
   return HMC_OK;
 }
 

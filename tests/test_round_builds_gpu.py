@@ -130,3 +130,34 @@ def test_folds_in_one_pass_equal_their_parts(columns, slots, blocks):
     expected = (want > 0.0) & (want >= 0.3 * want.max(axis=1, keepdims=True))
     np.testing.assert_array_equal(kept, expected.sum(axis=1))
     ctx.close()
+
+
+def test_a_fold_after_the_finalize_renews_the_column_maxima():
+    """hmc_truncate against the sums as they stand: a fold that follows the last one raises
+    one column's largest value, so the threshold moves with it."""
+    from pyradmc_amd import _native as nat
+
+    n_vox, columns = 300, 2
+    ctx = nat.Context(0)
+    zero, one, mass = np.zeros(3), np.ones(3), np.ones(n_vox)
+    ctx.call("hmc_set_scoring", n_vox, 1, 1, nat.ptr(zero, nat.c_double), nat.ptr(one, nat.c_double),
+             nat.ptr(mass, nat.c_double), columns, 1)
+    first = np.tile(np.arange(1, n_vox + 1, dtype=np.int64) * 10**9, (1, columns, 1))
+    later = np.zeros_like(first)
+    later[0, 1, 7] = 10**13
+    nhist = np.ones((1, columns))
+    kept, entries = np.zeros(columns, np.int64), nat.c_int64()
+
+    def truncated():
+        ctx.call("hmc_truncate", 0.5, nat.ptr(kept, nat.c_int64), nat.ctypes.byref(entries))
+        return kept.tolist()
+
+    ctx.call("hmc_set_quanta", nat.ptr(first, nat.c_int64))
+    ctx.call("hmc_fold_finalize", 1, nat.ptr(nhist, nat.c_double), 1, None, None)
+    assert truncated() == [n_vox // 2 + 1] * 2
+    for fold in (("hmc_fold", 1, nat.ptr(nhist, nat.c_double), None),
+                 ("hmc_fold_finalize", 1, nat.ptr(nhist, nat.c_double), 1, None, None)):
+        ctx.call("hmc_set_quanta", nat.ptr(later, nat.c_int64))
+        ctx.call(*fold)
+        assert truncated() == [n_vox // 2 + 1, 1]
+    ctx.close()
