@@ -53,6 +53,10 @@ int hsp_apply(hsp_matrix *m, const double *weights, int n_w, long long row_begin
 int hsp_apply_device(hsp_matrix *m, const void *weights_device, int n_w, long long row_begin,
                      long long row_end, int precision, void *out_device, double *kernel_ms);
 
+/* HSP_OK if hsp_apply and its forms take these arguments, else their error: for a caller that
+ * would allocate the result first. */
+int hsp_check_apply(hsp_matrix* m, int n_w, long long row_begin, long long row_end, int precision);
+
 /* hsp_apply into the internal product, copied to the host array out [row_end - row_begin]
  * [n_w] (float64 or float32, as precision) before it returns: hsp_apply and hsp_fetch in one
  * call, with one wait where weights and product are small (1 MiB each). */

@@ -1302,6 +1302,10 @@ int hsp_apply(hsp_matrix* m, const double* weights, int n_w, long long row_begin
   return apply_on_device(m, m->w, n_w, row_begin, row_end, precision, out_device, kernel_ms);
 }
 
+int hsp_check_apply(hsp_matrix* m, int n_w, long long row_begin, long long row_end, int precision) {
+  return m ? check_apply(m, n_w, row_begin, row_end, precision) : HSP_EINVAL;
+}
+
 int hsp_apply_host(hsp_matrix* m, const double* weights, int n_w, long long row_begin, long long row_end,
                    int precision, void* out, double* kernel_ms) {
   if (!m) return HSP_EINVAL;

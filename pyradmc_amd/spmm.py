@@ -36,6 +36,7 @@ def _lib():
         "hsp_apply": (ctypes.c_int, [_c_void, f64p, ctypes.c_int, ll, ll, ctypes.c_int, _c_void, f64p]),
         "hsp_apply_host": (ctypes.c_int, [_c_void, f64p, ctypes.c_int, ll, ll, ctypes.c_int, _c_void, f64p]),
         "hsp_apply_device": (ctypes.c_int, [_c_void, _c_void, ctypes.c_int, ll, ll, ctypes.c_int, _c_void, f64p]),
+        "hsp_check_apply": (ctypes.c_int, [_c_void, ctypes.c_int, ll, ll, ctypes.c_int]),
         "hsp_fetch": (ctypes.c_int, [_c_void, ll, ll, _c_void]),
         "hsp_csr": (ctypes.c_int, [_c_void, i64p, ctypes.POINTER(ctypes.c_int32), _c_void]),
         "hsp_block_entries": (ll, [_c_void]),
@@ -138,7 +139,9 @@ class DeviceDij:
             self._check(_lib().hsp_apply(self._h, wp, n_w, r0, r1, code, None, ctypes.byref(ms)), "hsp_apply")
             self.last_kernel_ms = float(ms.value)
             return None
-        out = np.empty((max(r1 - r0, 0), n_w), dtype=dtype)
+        # Refused before the result is allocated, which may be far beyond the host's memory.
+        self._check(_lib().hsp_check_apply(self._h, n_w, r0, r1, code), "hsp_apply")
+        out = np.empty((r1 - r0, n_w), dtype=dtype)
         self._check(_lib().hsp_apply_host(self._h, wp, n_w, r0, r1, code, out.ctypes.data, ctypes.byref(ms)),
                     "hsp_apply")
         self.last_kernel_ms = float(ms.value)

@@ -47,3 +47,21 @@ def test_few_vectors_match_the_reference_sum(n_w, n_rows, per_row):
     np.add.at(ref, cols, dij.dose * dij.indices)
     np.testing.assert_allclose(got, ref, rtol=1e-11, atol=1e-11 * max(np.abs(ref).max(), 1.0))
     dev.close()
+
+
+def test_refused_products_allocate_nothing():
+    """Row ranges outside the matrix and products beyond one launch are refused as such,
+    whatever memory their result would have taken."""
+    from pyradmc_amd.spmm import DeviceDij
+
+    dij, _ = _dij(21, (3, 0, 1), 40)
+    dev = DeviceDij(dij)
+    weights = np.ones(40)
+    for rows in ((0, 10**13), (-(10**13), 5), (5, 5), (6, 5), (0, 22)):
+        for fetch in (True, False):
+            with pytest.raises(ValueError, match="row range"):
+                dev.apply(weights, rows=rows, fetch=fetch)
+    with pytest.raises(ValueError):
+        dev.apply(np.ones((40, 0)))
+    assert dev.apply(weights).shape == (21,)
+    dev.close()
