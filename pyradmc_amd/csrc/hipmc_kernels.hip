@@ -1895,6 +1895,7 @@ int dev_alloc(hmc_ctx* ctx, T** ptr, size_t count) {
   hipError_t e = hipMalloc(reinterpret_cast<void**>(ptr), bytes);
   if (e != hipSuccess) {
     *ptr = nullptr;
+    (void)hipGetLastError();  // reported here, not by the next launch's check
     return fail(ctx, e == hipErrorOutOfMemory ? HMC_ENOMEM : HMC_EHIP,
                 std::string("hipMalloc: ") + hipGetErrorString(e));
   }
@@ -2250,6 +2251,7 @@ int hmc_set_gs(hmc_ctx* ctx, const float* values, int n_eta, int n_theta2, int n
   if (n_eta < 2 || n_theta2 < 2 || n_u < 1)
     return fail(ctx, HMC_EINVAL, "GS grid needs at least 2x2 nodes");
   HMC_HIP(ctx, hipSetDevice(ctx->device));
+  ctx->has_gs = false;  // a failure below can leave the cells freed
   const size_t count = static_cast<size_t>(n_eta) * n_theta2 * n_u;
   const long long cells = static_cast<long long>(n_eta - 1) * (n_theta2 - 1) * n_u;
   int rc = upload(ctx, &ctx->d_gs, values, count);

@@ -349,6 +349,7 @@ class HipEngine:
         key = (ecut, pcut, e_max, with_gs)
         if self._uploaded_tables == key:
             return
+        self._uploaded_tables = None  # until all of it is there
         keep = {}
 
         def f(name, arr=None):

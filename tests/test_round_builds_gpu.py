@@ -161,3 +161,23 @@ def test_a_fold_after_the_finalize_renews_the_column_maxima():
         ctx.call(*fold)
         assert truncated() == [n_vox // 2 + 1, 1]
     ctx.close()
+
+
+def test_a_grid_that_could_not_be_set_is_not_used():
+    """After hmc_set_gs has failed (here for want of memory), no transport reads what is
+    left of the cells before it; the next run uploads tables and grid again."""
+    from pyradmc_amd import AnalyticCrossSections, HipEngine, PencilBeamSource, VoxelGrid
+    from pyradmc_amd import _native as nat
+
+    grid = VoxelGrid.uniform_water((8, 8, 8), (1.0, 1.0, 1.0))
+    eng = HipEngine(grid, AnalyticCrossSections(geometry_densities=grid.max_density_by_material()))
+    source = PencilBeamSource(6.0, (4.0, 4.0, -1.0), (0.0, 0.0, 1.0))
+    before = eng.run(source, 1000, 2, seed=1)
+    nodes = np.zeros(8, np.float32)
+    with pytest.raises(MemoryError):
+        eng._ctx.call("hmc_set_gs", nat.ptr(nodes, nat.ctypes.c_float), 20_000, 20_000, 20_000, 0, 0)
+    with pytest.raises(RuntimeError, match="GS grid not set"):
+        eng.run(source, 1000, 2, seed=1)
+    eng._uploaded_tables = None
+    _same(before, eng.run(source, 1000, 2, seed=1))
+    eng.close()
