@@ -227,13 +227,17 @@ int hmc_set_profiling(hmc_ctx *ctx, int enabled);
  * of 256 in [256, 8192]), queue indices a wave claims at a time and output slots it
  * reserves at a time (each a multiple of 64 in [64, 1024]), and whether each group of
  * four rounds is replayed from a captured HIP graph (default 1; profiled transports
- * launch one by one, so that every kernel is timed). A context on which this was never
- * called sizes the first three itself, each round by its queue's length. None of them
- * changes a result. No reference counterpart beyond the
+ * launch one by one, so that every kernel is timed). 0 for any of the first three, the
+ * default, leaves it to the library: the width by the histories, the other two by each
+ * queue's length. None of them changes a result. No reference counterpart beyond the
  * chunk_size / queue_factor knobs of WarpEngine (engine.py:369-407): these are the
  * autotuner's knobs. */
 int hmc_set_launch(hmc_ctx *ctx, int round_lanes_per_cu, int refill_block, int push_chunk,
                    int use_graphs);
+/* The launch shape that a transport of this many histories (one chunk of them) takes on
+ * the context as it stands: workgroups of a round's grid, threads of each, refill block
+ * and push chunk (0: by the queue's length). No reference counterpart. */
+int hmc_round_grid(hmc_ctx *ctx, int64_t histories, int out[4]);
 
 /* Work ----------------------------------------------------------------------- */
 /* Generate and transport every primary of the work items into the dense tallies:

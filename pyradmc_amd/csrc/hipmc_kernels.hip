@@ -2926,12 +2926,13 @@ int hmc_set_profiling(hmc_ctx* ctx, int enabled) {
 
 int hmc_set_launch(hmc_ctx* ctx, int round_lanes_per_cu, int refill_block, int push_chunk, int use_graphs) {
   if (!ctx) return HMC_EINVAL;
-  if (round_lanes_per_cu < 256 || round_lanes_per_cu > 8192 || round_lanes_per_cu % 256 != 0)
-    return fail(ctx, HMC_EINVAL, "round lanes per CU must be a multiple of 256 in [256, 8192]");
-  if (refill_block < 64 || refill_block > 1024 || refill_block % 64 != 0)
-    return fail(ctx, HMC_EINVAL, "refill block must be a multiple of 64 in [64, 1024]");
-  if (push_chunk < 64 || push_chunk > 1024 || push_chunk % 64 != 0)
-    return fail(ctx, HMC_EINVAL, "push chunk must be a multiple of 64 in [64, 1024]");
+  // 0: sized by the work, as on a new context
+  if (round_lanes_per_cu < 0 || round_lanes_per_cu > 8192 || round_lanes_per_cu % 256 != 0)
+    return fail(ctx, HMC_EINVAL, "round lanes per CU must be 0 or a multiple of 256 up to 8192");
+  if (refill_block < 0 || refill_block > 1024 || refill_block % 64 != 0)
+    return fail(ctx, HMC_EINVAL, "refill block must be 0 or a multiple of 64 up to 1024");
+  if (push_chunk < 0 || push_chunk > 1024 || push_chunk % 64 != 0)
+    return fail(ctx, HMC_EINVAL, "push chunk must be 0 or a multiple of 64 up to 1024");
   ctx->round_lanes_per_cu = round_lanes_per_cu;
   ctx->refill_block = refill_block;
   ctx->push_chunk = push_chunk;
@@ -2953,6 +2954,21 @@ constexpr int kRoundsPerSync = 4;
 // 2048 with refill blocks and push chunks of 64); 100-beamlet Dij 30.8, 30.9, 31.7 ms
 // (38.3).
 constexpr int kAutoLanesPerCu = 768;
+
+// Whether the rounds take the build for one material (kOne).
+static bool one_material_rounds(const hmc_ctx* ctx) {
+  return ctx->t.n_mat == 1 && ctx->t.n_points <= kTablePoints && small_grid(ctx->g.nx, ctx->g.ny, ctx->g.nz) &&
+         small_grid(ctx->s.nx, ctx->s.ny, ctx->s.nz);
+}
+
+// Workgroups of a round's grid for a transport of n histories (a chunk of them).
+static unsigned int round_workgroups(const hmc_ctx* ctx, long long n) {
+  const long long cus = std::max(ctx->cu_count, 1);
+  const long long lanes = ctx->round_lanes_per_cu ? cus * ctx->round_lanes_per_cu
+                                                  : std::min(cus * kAutoLanesPerCu, std::max(cus * 256, n));
+  const unsigned int blocks = static_cast<unsigned int>(blocks_for(lanes));
+  return one_material_rounds(ctx) ? std::max(1u, blocks * 256u / kElectronThreads<true>) : blocks;
+}
 
 // ------------------------------------------------------------- electron energy sort
 //
@@ -3104,10 +3120,9 @@ static bool fast_rounds(const TransportParams& P) {
 static int enqueue_round_group(hmc_ctx* ctx, const TransportParams& P, unsigned int round_blocks,
                                unsigned int cap, hipEvent_t* events) {
   const bool fast = fast_rounds(P);
-  const bool one = P.t.n_mat == 1 && P.t.n_points <= kTablePoints && small_grid(P.g.nx, P.g.ny, P.g.nz) &&
-                   small_grid(P.s.nx, P.s.ny, P.s.nz);
-  const unsigned int one_blocks = std::max(1u, round_blocks * 256u / kElectronThreads<true>);
-  static_assert(kPhotonThreads<true> == kElectronThreads<true>, "both rounds launch one_blocks");
+  const bool one = one_material_rounds(ctx);
+  static_assert(kPhotonThreads<true> == kElectronThreads<true> && kPhotonThreads<false> == kElectronThreads<false>,
+                "both rounds launch round_blocks");
   unsigned int* counts = ctx->d_counts;
   unsigned int* heads = ctx->d_counts + 4;
   int pa = 0, ea = 1, pb = 2, eb = 3;
@@ -3120,10 +3135,10 @@ static int enqueue_round_group(hmc_ctx* ctx, const TransportParams& P, unsigned 
     // Photon round: consume pa; electrons append to ea, photons to pb.
     if (ev) HMC_HIP(ctx, hipEventRecord(ev[0], ctx->stream));
     if (one && fast)
-      hipLaunchKernelGGL((k_photon_round<true, true>), dim3(one_blocks), dim3(kPhotonThreads<true>), 0, ctx->stream, P,
+      hipLaunchKernelGGL((k_photon_round<true, true>), dim3(round_blocks), dim3(kPhotonThreads<true>), 0, ctx->stream, P,
                          qa_p, heads + pa, qa_e, qb_p);
     else if (one)
-      hipLaunchKernelGGL((k_photon_round<false, true>), dim3(one_blocks), dim3(kPhotonThreads<true>), 0, ctx->stream,
+      hipLaunchKernelGGL((k_photon_round<false, true>), dim3(round_blocks), dim3(kPhotonThreads<true>), 0, ctx->stream,
                          P, qa_p, heads + pa, qa_e, qb_p);
     else if (fast)
       hipLaunchKernelGGL((k_photon_round<true, false>), dim3(round_blocks), dim3(kPhotonThreads<false>), 0,
@@ -3154,10 +3169,10 @@ static int enqueue_round_group(hmc_ctx* ctx, const TransportParams& P, unsigned 
     }
     if (ev) HMC_HIP(ctx, hipEventRecord(ev[2], ctx->stream));
     if (one && fast)
-      hipLaunchKernelGGL((k_electron_round<true, true>), dim3(one_blocks), dim3(kElectronThreads<true>), 0,
+      hipLaunchKernelGGL((k_electron_round<true, true>), dim3(round_blocks), dim3(kElectronThreads<true>), 0,
                          ctx->stream, P, qin_e, head_e, qb_p, qb_e);
     else if (one)
-      hipLaunchKernelGGL((k_electron_round<false, true>), dim3(one_blocks), dim3(kElectronThreads<true>), 0,
+      hipLaunchKernelGGL((k_electron_round<false, true>), dim3(round_blocks), dim3(kElectronThreads<true>), 0,
                          ctx->stream, P, qin_e, head_e, qb_p, qb_e);
     else if (fast)
       hipLaunchKernelGGL((k_electron_round<true, false>), dim3(round_blocks), dim3(kElectronThreads<false>), 0,
@@ -3219,6 +3234,17 @@ static int launch_round_group(hmc_ctx* ctx, const TransportParams& P, unsigned i
   }
   HMC_HIP(ctx, hipGraphLaunch(ctx->round_graph, ctx->stream));
   *replayed = true;
+  return HMC_OK;
+}
+
+int hmc_round_grid(hmc_ctx* ctx, int64_t histories, int out[4]) {
+  if (!ctx || !out || histories < 1) return fail(ctx, HMC_EINVAL, "bad round grid arguments");
+  if (!ctx->has_grid || !ctx->has_scoring || !ctx->has_tables)
+    return fail(ctx, HMC_ESTATE, "grid, scoring and tables must be set");
+  out[0] = static_cast<int>(round_workgroups(ctx, histories));
+  out[1] = one_material_rounds(ctx) ? kElectronThreads<true> : kElectronThreads<false>;
+  out[2] = ctx->refill_block;
+  out[3] = ctx->push_chunk;
   return HMC_OK;
 }
 
@@ -3302,14 +3328,8 @@ int hmc_transport(hmc_ctx* ctx, uint64_t seed, const hmc_work_item* items, int n
   // Rounds launch at full width: lanes of an exhausted queue exit at once, so the host
   // never needs a queue's size to launch it, and it enqueues kRoundsPerSync photon /
   // electron rounds between count reads.
-  // Where the caller set no width: kAutoLanesPerCu, or fewer lanes when a chunk's
-  // histories need fewer (at least one workgroup per CU).
-  const long long cus = std::max(ctx->cu_count, 1);
-  const long long lanes = ctx->round_lanes_per_cu
-                              ? cus * ctx->round_lanes_per_cu
-                              : std::min(cus * kAutoLanesPerCu, std::max(cus * 256, chunk_n));
-  const unsigned int round_blocks = static_cast<unsigned int>(blocks_for(lanes));
-  if (static_cast<long long>(round_blocks) * 4 * ctx->refill_block > (1ll << 30))
+  const unsigned int round_blocks = round_workgroups(ctx, chunk_n);
+  if (static_cast<long long>(round_blocks) * kMaxBlockWaves * ctx->refill_block > (1ll << 30))
     return fail(ctx, HMC_EINVAL, "round width times refill block too large");
   long long overflow = 0, rounds = 0, launches[2] = {0, 0}, graph_launches = 0;
   double kernel_ms[2] = {0.0, 0.0};

@@ -281,8 +281,7 @@ class HipEngine:
         self._index = _device_index(self.device)
         self._ctx = nat.Context(self._index)
         self._info = nat.device_info(self._index)
-        # set_launch's defaults; until it is called the library sizes the rounds by their queues
-        self.launch = {"round_lanes_per_cu": 2048, "refill_block": 64, "push_chunk": 64, "use_graphs": True}
+        self.launch = {"round_lanes_per_cu": 0, "refill_block": 0, "push_chunk": 0, "use_graphs": True}
         self._population_token = None
         self._ray_model = None
 
@@ -627,13 +626,14 @@ class HipEngine:
         the result's ``counters``); a measurement hook, off by default."""
         self._ctx.call("hmc_set_profiling", 1 if enabled else 0)
 
-    def set_launch(self, round_lanes_per_cu: int = 2048, refill_block: int = 64, push_chunk: int = 64,
+    def set_launch(self, round_lanes_per_cu: int = 0, refill_block: int = 0, push_chunk: int = 0,
                    use_graphs: bool = True) -> None:
         """Launch shape of the transport rounds: lanes per CU of each round's grid,
-        queue indices a wave claims at a time, output slots it reserves at a time, and
-        whether groups of rounds replay a captured HIP graph. Results do not depend on
-        them (each particle carries its own random stream; tallies are integers);
-        ``pyradmc_amd.autotune`` picks them."""
+        queue indices a wave claims at a time, output slots it reserves at a time (0, as
+        on a new engine: sized by the library, by the histories and each queue's length),
+        and whether groups of rounds replay a captured HIP graph. ``launch`` holds what is
+        set. Results do not depend on them (each particle carries its own random stream;
+        tallies are integers); ``pyradmc_amd.autotune`` picks them."""
         self._ctx.call("hmc_set_launch", int(round_lanes_per_cu), int(refill_block), int(push_chunk),
                        1 if use_graphs else 0)
         self.launch = {"round_lanes_per_cu": int(round_lanes_per_cu), "refill_block": int(refill_block),

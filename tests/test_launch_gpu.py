@@ -57,6 +57,35 @@ def test_rounds_sized_by_their_queue_match_a_fixed_shape(slab, histories):
           sized)
 
 
+def _round_grid(engine, histories):
+    from pyradmc_amd import _native as nat
+
+    got = (nat.c_int * 4)()
+    engine._ctx.call("hmc_round_grid", int(histories), got)
+    return dict(zip(("workgroups", "threads", "refill_block", "push_chunk"), got))
+
+
+def test_knobs_left_out_stay_automatic(slab):
+    """Setting one knob leaves the others to the queue's length, and set_launch() with
+    nothing set gives back an engine on which it was never called."""
+    grid, xs, src = slab
+    eng = _engine(grid, xs)
+    ref = eng.run(src, 300_000, 4, seed=11)
+    fresh = eng.launch
+    assert fresh == {"round_lanes_per_cu": 0, "refill_block": 0, "push_chunk": 0, "use_graphs": True}
+    sized = _round_grid(eng, 300_000)
+    eng.set_launch(use_graphs=False)
+    assert eng.launch == {**fresh, "use_graphs": False} and _round_grid(eng, 300_000) == sized
+    _same(ref, eng.run(src, 300_000, 4, seed=11))
+    eng.set_launch(refill_block=128)
+    assert eng.launch == {**fresh, "refill_block": 128}
+    assert _round_grid(eng, 300_000) == {**sized, "refill_block": 128}
+    _same(ref, eng.run(src, 300_000, 4, seed=11))
+    eng.set_launch()
+    assert eng.launch == fresh and _round_grid(eng, 300_000) == sized
+    _same(ref, eng.run(src, 300_000, 4, seed=11))
+
+
 def test_graph_replays_match_eager_runs(slab):
     grid, xs, src = slab
     eng = _engine(grid, xs)
