@@ -12,6 +12,10 @@ the tallies are integer sums, so dose and Dij are bit-identical under any of the
 * ``push_chunk`` - output queue slots a wave reserves with one atomic;
 * ``use_graphs`` - replay each group of four rounds from a captured HIP graph.
 
+Zero lanes, refill block or push chunk leave that knob to the library, which sizes it by
+the work; the search starts at what the engine runs (on a new engine, all of them so) and
+has it among its candidates, so it never settles on a shape that it measured as slower.
+
 ``tune`` runs a coordinate descent over candidate values, timing a caller-supplied
 piece of work (the median of ``repeats`` runs per candidate), applies the best and
 stores it in a JSON cache keyed by device and workload, so later engines on the same
@@ -30,9 +34,9 @@ from dataclasses import asdict, dataclass
 from pathlib import Path
 
 DEFAULT_CANDIDATES = {
-    "round_lanes_per_cu": (512, 768, 1024, 1536, 2048, 3072),
-    "refill_block": (64, 128, 256, 512, 1024),
-    "push_chunk": (64, 128, 256),
+    "round_lanes_per_cu": (0, 512, 768, 1024, 1536, 2048, 3072),
+    "refill_block": (0, 64, 128, 256, 512, 1024),
+    "push_chunk": (0, 64, 128, 256),
     "chunk_size": (None, 4 << 20, 2 << 20),
     "use_graphs": (True, False),
 }
@@ -41,7 +45,7 @@ DEFAULT_CANDIDATES = {
 @dataclass
 class LaunchConfig:
     chunk_size: int | None = None  # None: the engine sizes chunks from free memory
-    round_lanes_per_cu: int = 2048
+    round_lanes_per_cu: int = 2048  # 0 here and in the next two: sized by the library
     refill_block: int = 64
     push_chunk: int = 64
     use_graphs: bool = True
@@ -66,6 +70,11 @@ def workload_key(engine, source, n_histories: int, n_batches: int, transport_ele
              type(source).__name__, f"{float(source.max_energy):.4g}", f"e{int(bool(transport_electrons))}",
              f"n2^{scale}", f"b{int(n_batches)}"]
     return "|".join(parts)
+
+
+def current(engine) -> LaunchConfig:
+    """What the engine runs now."""
+    return LaunchConfig(chunk_size=engine.chunk_size, **engine.launch)
 
 
 def _read_cache(path: Path) -> dict:
@@ -101,10 +110,10 @@ def tune(engine, work, candidates: dict | None = None, repeats: int = 3, start: 
     each knob in turn takes the value with the lowest median time of ``work()`` over
     ``repeats`` runs, the other knobs held at their best so far; up to ``passes``
     sweeps over the knobs (stopping early when a sweep changes nothing, since the
-    knobs interact). Applies the best configuration to ``engine`` and returns
-    (config, seconds, trials)."""
+    knobs interact), from ``start`` (None: what the engine runs now). Applies the best
+    configuration to ``engine`` and returns (config, seconds, trials)."""
     candidates = DEFAULT_CANDIDATES if candidates is None else candidates
-    best = LaunchConfig(**asdict(start)) if start else LaunchConfig()
+    best = LaunchConfig(**asdict(start)) if start else current(engine)
     measured: dict = {}
     trials = []
 

@@ -133,3 +133,22 @@ def test_dij_tuning_times_run_dij_and_caches_under_its_own_key(tmp_path, monkeyp
                               truncation=1e-4)
     assert again == config and len(seen) == calls  # from the cache, nothing timed
     assert eng.launch["round_lanes_per_cu"] == 1024
+
+
+def test_the_search_starts_at_the_automatic_sizing_and_can_return_to_it():
+    """On an engine as it is built every knob is automatic: that is timed first, kept where
+    no candidate is faster, and among the candidates once another knob has moved."""
+    automatic = {"round_lanes_per_cu": 0, "refill_block": 0, "push_chunk": 0, "use_graphs": True}
+    eng = _FakeEngine()
+    eng.launch = dict(automatic)
+    clock = [0.0]
+
+    def work():
+        clock[0] += 1.0 + sum(eng.launch[k] != v for k, v in automatic.items())
+
+    config, seconds, trials = autotune.tune(eng, work, repeats=1, timer=lambda: clock[0])
+    assert trials[0] == ({"chunk_size": None, **automatic}, 1.0)
+    assert (config, seconds) == (autotune.LaunchConfig(None, 0, 0, 0, True), 1.0)
+    assert eng.launch == automatic
+    eng.launch = {"round_lanes_per_cu": 2048, "refill_block": 64, "push_chunk": 64, "use_graphs": True}
+    assert autotune.tune(eng, work, repeats=1, timer=lambda: clock[0])[0] == config
