@@ -18,20 +18,24 @@ has it among its candidates, so it never settles on a shape that it measured as 
 
 ``tune`` runs a coordinate descent over candidate values, timing a caller-supplied
 piece of work (the median of ``repeats`` runs per candidate), applies the best and
-stores it in a JSON cache keyed by device and workload, so later engines on the same
-workload pick it up with ``load``. ``tune_run`` times an open-field ``run``,
-``tune_dij`` a whole ``run_dij``.
+stores it in a JSON cache keyed by device, library build and workload, so later
+engines on the same workload pick it up with ``load``. ``tune_run`` times an open-field
+``run``, ``tune_dij`` a whole ``run_dij``.
 """
 
 from __future__ import annotations
 
+import hashlib
 import json
 import math
 import os
 import statistics
 import time
 from dataclasses import asdict, dataclass
+from functools import lru_cache
 from pathlib import Path
+
+from pyradmc_amd import build
 
 DEFAULT_CANDIDATES = {
     "round_lanes_per_cu": (0, 512, 768, 1024, 1536, 2048, 3072),
@@ -61,14 +65,24 @@ def apply(engine, config: LaunchConfig) -> None:
     engine.set_launch(config.round_lanes_per_cu, config.refill_block, config.push_chunk, config.use_graphs)
 
 
+@lru_cache(maxsize=4)
+def _library_id(path: Path) -> str:
+    """The kernels' build, by the library's bytes: a shape that was best for other kernels
+    need not be for these."""
+    try:
+        return hashlib.sha256(path.read_bytes()).hexdigest()[:12]
+    except OSError:
+        return "none"
+
+
 def workload_key(engine, source, n_histories: int, n_batches: int, transport_electrons: bool = True) -> str:
-    """Device, grid, source type and energy, history count (to a power of two) and
-    batches: the things the best launch shape depends on."""
+    """Device, library build, grid, source type and energy, history count (to a power of
+    two) and batches: the things the best launch shape depends on."""
     grid = engine.grid
     scale = max(int(n_histories), 1).bit_length()
     parts = [engine.device_name, str(engine._info.get("cu_count")), "x".join(str(int(v)) for v in grid.shape),
              type(source).__name__, f"{float(source.max_energy):.4g}", f"e{int(bool(transport_electrons))}",
-             f"n2^{scale}", f"b{int(n_batches)}"]
+             f"n2^{scale}", f"b{int(n_batches)}", f"lib{_library_id(build.LIB_PATH)}"]
     return "|".join(parts)
 
 

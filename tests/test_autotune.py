@@ -152,3 +152,13 @@ def test_the_search_starts_at_the_automatic_sizing_and_can_return_to_it():
     assert eng.launch == automatic
     eng.launch = {"round_lanes_per_cu": 2048, "refill_block": 64, "push_chunk": 64, "use_graphs": True}
     assert autotune.tune(eng, work, repeats=1, timer=lambda: clock[0])[0] == config
+
+
+def test_a_shape_chosen_for_other_kernels_is_not_applied(tmp_path, monkeypatch):
+    eng, src = _FakeEngine(), SimpleNamespace(max_energy=6.0)
+    keys = []
+    for name, content in (("a.so", b"kernels"), ("b.so", b"other kernels"), ("c.so", b"kernels")):
+        (tmp_path / name).write_bytes(content)
+        monkeypatch.setattr(autotune.build, "LIB_PATH", tmp_path / name)
+        keys.append(autotune.workload_key(eng, src, 10_000_000, 20))
+    assert keys[0] == keys[2] != keys[1]
