@@ -229,7 +229,8 @@ int hmc_set_profiling(hmc_ctx *ctx, int enabled);
  * four rounds is replayed from a captured HIP graph (default 1; profiled transports
  * launch one by one, so that every kernel is timed). 0 for any of the first three, the
  * default, leaves it to the library: the width by the histories, the other two by each
- * queue's length. None of them changes a result. No reference counterpart beyond the
+ * queue's length. The width is the general build's: with one material a round has one
+ * workgroup of 768 to a CU. None of them changes a result. No reference counterpart beyond the
  * chunk_size / queue_factor knobs of WarpEngine (engine.py:369-407): these are the
  * autotuner's knobs. */
 int hmc_set_launch(hmc_ctx *ctx, int round_lanes_per_cu, int refill_block, int push_chunk,

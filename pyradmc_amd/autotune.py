@@ -7,7 +7,8 @@ the tallies are integer sums, so dose and Dij are bit-identical under any of the
   ``chunk_size * queue_factor`` particles); the reference's own knob
   (pyradmc/backends/warp/engine.py:175-186 records its chunk sweep);
 * ``round_lanes_per_cu`` - lanes per CU in each round's grid (persistent lanes; the
-  resident share runs first, the rest as earlier lanes retire);
+  resident share runs first, the rest as earlier lanes retire; with one material a CU
+  takes one workgroup of 768 at any width);
 * ``refill_block`` - queue indices a wave claims with one atomic;
 * ``push_chunk`` - output queue slots a wave reserves with one atomic;
 * ``use_graphs`` - replay each group of four rounds from a captured HIP graph.

@@ -2949,7 +2949,8 @@ constexpr int kRoundsPerSync = 4;
 
 // Lanes per CU of a round's grid where the caller set none: three waves per SIMD. A
 // wave's steps are gathers of 64 scattered addresses, and the CU's one L1 serves about
-// one line per cycle: more waves thrash it sooner than they hide its latency. Slab
+// one line per cycle: more waves thrash it sooner than they hide its latency. Measured on
+// the general build, before the build for one material had its own workgroup: slab
 // phantom, 1e7 histories, whole run: 6.54 ms at 768, 6.61 at 1024, 6.84 at 1280 (9.2 at
 // 2048 with refill blocks and push chunks of 64); 100-beamlet Dij 30.8, 30.9, 31.7 ms
 // (38.3).
@@ -2961,13 +2962,20 @@ static bool one_material_rounds(const hmc_ctx* ctx) {
          small_grid(ctx->s.nx, ctx->s.ny, ctx->s.nz);
 }
 
-// Workgroups of a round's grid for a transport of n histories (a chunk of them).
+// Workgroups of a round's grid for a transport of n histories (a chunk of them). The build
+// for one material takes one to a CU at any width and length: its 12 waves and 94 KB of
+// LDS (electrons) leave no room for a second, so more would only queue behind the first,
+// and fewer would leave CUs idle (a claim is 64 particles or more, so a short queue
+// spreads over all of them; a workgroup without particles ends at once). Counted in 256-lane
+// units and cut to 768-lane workgroups, as before, 80 000 histories had 104 of 256 CUs and
+// a width of 2048 lanes 682 workgroups: 1e6 histories on the slab phantom took 2.50 ms with
+// refill blocks of 256 at that width, 1.66 ms so; a quick-start pencil 0.56 and 0.55 ms.
 static unsigned int round_workgroups(const hmc_ctx* ctx, long long n) {
   const long long cus = std::max(ctx->cu_count, 1);
+  if (one_material_rounds(ctx)) return static_cast<unsigned int>(cus);
   const long long lanes = ctx->round_lanes_per_cu ? cus * ctx->round_lanes_per_cu
                                                   : std::min(cus * kAutoLanesPerCu, std::max(cus * 256, n));
-  const unsigned int blocks = static_cast<unsigned int>(blocks_for(lanes));
-  return one_material_rounds(ctx) ? std::max(1u, blocks * 256u / kElectronThreads<true>) : blocks;
+  return static_cast<unsigned int>(blocks_for(lanes));
 }
 
 // ------------------------------------------------------------- electron energy sort

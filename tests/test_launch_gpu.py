@@ -86,6 +86,27 @@ def test_knobs_left_out_stay_automatic(slab):
     _same(ref, eng.run(src, 300_000, 4, seed=11))
 
 
+@pytest.mark.parametrize("lanes", (0, 256, 512, 2048, 8192))
+def test_round_grids_fill_the_cus_and_no_more(slab, lanes):
+    """One material: a workgroup fills its CU, so a round has one to a CU at any width and
+    number of histories. Two: 256-lane workgroups, as many as the width says, and by the
+    histories (at least one to a CU) where none is set."""
+    from tests.test_round_builds_gpu import TwoEqualRows
+
+    grid, xs, src = slab
+    one, two = _engine(grid, xs), _engine(grid, TwoEqualRows(xs))
+    cus = one._info["cu_count"]
+    for eng in (one, two):
+        eng.set_launch(round_lanes_per_cu=lanes)
+        eng.run(src, 1000, 1, seed=1)  # uploads the tables
+    for histories in (1, 1000, 80_000, 10_000_000):
+        got = _round_grid(one, histories)
+        assert (got["workgroups"], got["threads"]) == (cus, 768)
+        auto = min(3 * cus, max(cus, -(-histories // 256)))
+        got = _round_grid(two, histories)
+        assert (got["workgroups"], got["threads"]) == (lanes // 256 * cus if lanes else auto, 256)
+
+
 def test_graph_replays_match_eager_runs(slab):
     grid, xs, src = slab
     eng = _engine(grid, xs)
