@@ -235,6 +235,12 @@ int hmc_set_profiling(hmc_ctx *ctx, int enabled);
  * autotuner's knobs. */
 int hmc_set_launch(hmc_ctx *ctx, int round_lanes_per_cu, int refill_block, int push_chunk,
                    int use_graphs);
+/* Slots (0 to 32, default 32 each) of the electron rounds' two stacks per wave: particles
+ * that wait for their Moller interaction, and delta electrons the wave transports itself.
+ * What finds no slot interacts in place, or goes to the next round's queue: with 0 and 0
+ * nothing passes through a stack. No effect on a result, which is what this is for: a
+ * check of the stacks against a schedule without them. No reference counterpart. */
+int hmc_set_round_stacks(hmc_ctx *ctx, int moller_slots, int delta_slots);
 /* The launch shape that a transport of this many histories (one chunk of them) takes on
  * the context as it stands: workgroups of a round's grid, threads of each, refill block
  * and push chunk (0: by the queue's length). No reference counterpart. */

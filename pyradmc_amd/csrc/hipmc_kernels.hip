@@ -216,6 +216,7 @@ struct TransportParams {
   float log_pcut;  // logf(pcut), for the bremsstrahlung spectrum
   int transport_electrons, msc_gs, dose_to_water, max_steps;
   unsigned int refill_block;  // queue indices a wave claims at a time (multiple of 64; 0: by the queue's length)
+  unsigned int moller_slots, fresh_slots;  // slots in use of a wave's stacks (hmc_set_round_stacks)
 };
 
 // Per-lane books kept in registers and flushed once per lane at the end of a round;
@@ -848,7 +849,7 @@ k_electron_round(TransportParams P, Queue qin, unsigned int* head, Queue qp, Que
         const unsigned long long born = __ballot(1);
         const unsigned int slot =
             n_fresh + static_cast<unsigned int>(__popcll(born & ((1ull << __lane_id()) - 1ull)));
-        if (slot < static_cast<unsigned int>(kFreshSlots)) {
+        if (slot < P.fresh_slots) {
           fresh[0][slot] = __float_as_uint(x);
           fresh[1][slot] = __float_as_uint(y);
           fresh[2][slot] = __float_as_uint(z);
@@ -867,7 +868,7 @@ k_electron_round(TransportParams P, Queue qin, unsigned int* head, Queue qp, Que
         rotate(ux, uy, uz, cp, mphi + kPi);
         e -= delta;
       }
-      n_fresh = min(n_fresh + made, static_cast<unsigned int>(kFreshSlots));
+      n_fresh = min(n_fresh + made, P.fresh_slots);
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     } else if (refill_now) {
       const bool took = n_fresh != 0u;
@@ -1095,7 +1096,7 @@ k_electron_round(TransportParams P, Queue qin, unsigned int* head, Queue qp, Que
       const unsigned int slot =
           waiting + static_cast<unsigned int>(__popcll(met & ((1ull << __lane_id()) - 1ull)));
       if (moller) {
-        if (slot < static_cast<unsigned int>(kMollerSlots)) {
+        if (slot < P.moller_slots) {
           stack[0][slot] = __float_as_uint(x);
           stack[1][slot] = __float_as_uint(y);
           stack[2][slot] = __float_as_uint(z);
@@ -1113,7 +1114,7 @@ k_electron_round(TransportParams P, Queue qin, unsigned int* head, Queue qp, Que
           parked = true;
         }
       }
-      waiting = min(waiting + static_cast<unsigned int>(__popcll(met)), static_cast<unsigned int>(kMollerSlots));
+      waiting = min(waiting + static_cast<unsigned int>(__popcll(met)), P.moller_slots);
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     }
   }
@@ -1839,6 +1840,7 @@ struct hmc_ctx {
   int round_lanes_per_cu = 0;
   int refill_block = 0;
   int push_chunk = 0;
+  int moller_slots = kMollerSlots, fresh_slots = kFreshSlots;  // hmc_set_round_stacks
   bool use_graphs = true;
   // the captured group of rounds and what it was captured with
   hipGraphExec_t round_graph = nullptr;
@@ -2940,6 +2942,15 @@ int hmc_set_launch(hmc_ctx* ctx, int round_lanes_per_cu, int refill_block, int p
   return HMC_OK;
 }
 
+int hmc_set_round_stacks(hmc_ctx* ctx, int moller_slots, int delta_slots) {
+  if (!ctx) return HMC_EINVAL;
+  if (moller_slots < 0 || moller_slots > kMollerSlots || delta_slots < 0 || delta_slots > kFreshSlots)
+    return fail(ctx, HMC_EINVAL, "stack slots outside the stacks");
+  ctx->moller_slots = moller_slots;
+  ctx->fresh_slots = delta_slots;
+  return HMC_OK;
+}
+
 // Enqueue one group of kRoundsPerSync photon / electron rounds on the context's stream,
 // starting from queue roles (0, 1 | 2, 3): photons and electrons in queues 0 and 1,
 // outputs to 2 and 3, roles swapped after each round. The group has an even number of
@@ -2949,11 +2960,10 @@ constexpr int kRoundsPerSync = 4;
 
 // Lanes per CU of a round's grid where the caller set none: three waves per SIMD. A
 // wave's steps are gathers of 64 scattered addresses, and the CU's one L1 serves about
-// one line per cycle: more waves thrash it sooner than they hide its latency. Measured on
-// the general build, before the build for one material had its own workgroup: slab
-// phantom, 1e7 histories, whole run: 6.54 ms at 768, 6.61 at 1024, 6.84 at 1280 (9.2 at
-// 2048 with refill blocks and push chunks of 64); 100-beamlet Dij 30.8, 30.9, 31.7 ms
-// (38.3).
+// one line per cycle: more waves thrash it sooner than they hide its latency. The general
+// build on three materials, whole runs at 512, 768, 1024, 1280 and 2048: 1e7 histories on
+// the slab phantom 6.12, 5.57, 5.60, 5.95 and 7.01 ms; 100-beamlet Dij 24.5, 22.8, 22.7,
+// 23.6 and 25.3 ms.
 constexpr int kAutoLanesPerCu = 768;
 
 // Whether the rounds take the build for one material (kOne).
@@ -3328,6 +3338,8 @@ int hmc_transport(hmc_ctx* ctx, uint64_t seed, const hmc_work_item* items, int n
   P.dose_to_water = ctx->phys.dose_to_water;
   P.max_steps = 1 << 20;
   P.refill_block = static_cast<unsigned int>(ctx->refill_block);
+  P.moller_slots = static_cast<unsigned int>(ctx->moller_slots);
+  P.fresh_slots = static_cast<unsigned int>(ctx->fresh_slots);
 
   hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, ctx->stream, ctx->d_ledger,
                      static_cast<long long>(L_COUNT), 0ull);
