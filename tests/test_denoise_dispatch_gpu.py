@@ -146,6 +146,35 @@ def test_fused_steps_equal_separate_calls(dn, shape, cin, cout, upsampled):  # n
     assert torch.equal(pred, ref)
 
 
+@pytest.mark.parametrize("shape, cin, cout", MARCHED + [
+    ((1, 2, 8, 32), 32, 32), ((1, 2, 8, 32), 64, 32),  # staged tiles
+    ((1, 2, 4, 16), 64, 64), ((1, 8, 8, 8), 16, 48), ((16, 8, 8, 8), 64, 64), ((48, 8, 8, 8), 16, 32),  # small waves
+    ((9, 16, 16, 16), 16, 16),  # 64-position waves
+])
+def test_added_input_equals_a_separate_addition(dn, shape, cin, cout):  # noqa: F811
+    """src 2 (x + x2 read as the input) against hdn_add and src 0, bit for bit, in every
+    forward kernel; no part of the network reads its input so any more."""
+    import torch
+
+    n, d, h, w = shape
+    P = n * d * h * w
+    rng = np.random.default_rng(cin + cout)
+    x, x2 = (_dev(_bf(rng.standard_normal(shape + (cin,)))) for _ in range(2))
+    wt = _dev(_bf(rng.standard_normal((27, cout, cin)) * 0.1))
+    bias = _dev(torch.from_numpy(rng.standard_normal(cout).astype(np.float32)))
+    added = torch.empty_like(x)
+    want, got = (torch.zeros(shape + (cout,), dtype=torch.bfloat16, device="cuda:0") for _ in range(2))
+    want_cm, got_cm = (torch.zeros((cout, P), dtype=torch.bfloat16, device="cuda:0") for _ in range(2))
+    args = (n, d, h, w, cin, cout, 0.1, None)
+    dn._call("hdn_add", x.data_ptr(), x2.data_ptr(), added.data_ptr(), None, P, cin, None)
+    dn._call("hdn_conv3d_fwd", added.data_ptr(), wt.data_ptr(), bias.data_ptr(), want.data_ptr(), want_cm.data_ptr(),
+             *args)
+    dn._call("hdn_conv3d_fwd_src", x.data_ptr(), x2.data_ptr(), 2, wt.data_ptr(), bias.data_ptr(), got.data_ptr(),
+             got_cm.data_ptr(), *args)
+    assert torch.equal(got, want) and torch.equal(got_cm, want_cm)
+    assert torch.count_nonzero(want.float()) > 0
+
+
 @pytest.mark.parametrize("splits, length", [(1, 5), (16, 64), (17, 65), (700, 6912)])
 def test_reduce_splits(dn, splits, length):  # noqa: F811
     import torch
