@@ -322,11 +322,11 @@ __global__ void __launch_bounds__(256) k_conv_fwd_deep(const __bf16* __restrict_
     }
 }
 
-// The same convolution for rows of KW = 32 voxels (w == KW, h % (256 / KW) == 0,
+// The same convolution for rows of KW = 32 voxels, or 64 (w == KW, h % (256 / KW) == 0,
 // cout 16 x TM): a workgroup computes 256 / KW consecutive h-rows of one z-slice (256
 // positions; each wave 64 of them) and first stages the input those rows read - 3 z x
 // (rows + 2) h x (KW + 2) w positions with their one-voxel halo, zero outside the
-// volume - in LDS (33, 65 or 130 KB for cin 16, 32 or 64). Every tap's operand then comes
+// volume - in LDS (KW 32: 33, 65 or 130 KB for cin 16, 32 or 64; KW 64: 38 or 76 KB). Every tap's operand then comes
 // from LDS instead of a gathered global load. The k-loop, MFMA operands and output are
 // those of k_conv_fwd, so the two kernels give identical sums.
 template <int TM, int CIN, int SRC, int EPI, int KW>
@@ -475,6 +475,12 @@ __global__ void __launch_bounds__(256) k_conv_fwd_tile(const __bf16* __restrict_
   }
 }
 
+// Workgroups of k_conv_fwd_march to a CU that its registers are budgeted for: three of
+// 16 -> 16 channels, else two; one less with the second input or skip that 16 channels
+// prefetch.
+template <int TM, int CIN, int SRC, int EPI>
+constexpr int kMarchPerCu = (CIN * TM == 16 ? 3 : 2) - (CIN == 16 && (SRC == kSrcAdd || EPI == kEpiSkip) ? 1 : 0);
+
 // The same convolution for rows of 64 voxels (w == 64, h % 4 == 0, cin 16 or 32, cout
 // 16 x TM): the full-resolution layers, bound by the LDS reads of their input fragments
 // (one 1 KiB fragment per MFMA and 16 output channels). A workgroup takes four h-rows and
@@ -488,8 +494,7 @@ __global__ void __launch_bounds__(256) k_conv_fwd_tile(const __bf16* __restrict_
 // channels 445 and 260 (the copy rate's floor is 170), the 2-channel input 382 and 190,
 // 32 -> 16 upsampled 870 and 400 (450 with the skip addition in its store).
 template <int TM, int CIN, int SRC, int EPI>
-__global__ void __launch_bounds__(256, (CIN * TM == 16 ? 3 : 2) - (CIN == 16 && (SRC == kSrcAdd || EPI == kEpiSkip) ? 1 : 0))
-    k_conv_fwd_march(
+__global__ void __launch_bounds__(256, (kMarchPerCu<TM, CIN, SRC, EPI>)) k_conv_fwd_march(
     const __bf16* __restrict__ x, const __bf16* __restrict__ x2, const __bf16* __restrict__ wt,
     Epilogue E, int n, int d, int h, int cout, int zc) {
   constexpr int kW = 64, kRows = 4, kTW = kW + 2, kTH = kRows + 2, kPos = kTH * kTW;
@@ -1190,22 +1195,64 @@ namespace {
 constexpr long long kFillWaves = 512;
 constexpr long long kPairWaves = 128;
 
+// Slices of a marching workgroup: those for which the rounds that the workgroups take on the
+// card, each as long as its slices and about two more for the first planes and the weights,
+// are the shortest; where two are alike the longer (fewer planes loaded twice). A fixed
+// length of six and up left small volumes on few CUs, and counts off a whole round left the
+// last one nearly empty. 16 -> 16 channels over 1 x 8, 1 x 64, 2 x 96 and 16 x 96 slices of
+// 64 x 64, us: a 3-plane tile per slice 7.8, 13.1, 29.4 and 225, marching with six slices or
+// more 17.7, 18.5, 22.1 and 145, with this rule 7.8, 11.1, 20.3 and 134; 16 -> 32: 8.7, 18.7,
+// 41.4 and 322; 25.6, 27.2, 33.3 and 256; 8.2, 17.2, 33.3 and 248.
+constexpr int kCus = 256;
+
+int march_slices(long long columns, int d, int per_cu) {
+  const long long resident = static_cast<long long>(kCus) * per_cu;
+  int best = 1;
+  long long least = std::numeric_limits<long long>::max();
+  for (int zc = 1; zc <= std::min(d, 128); ++zc) {
+    const long long groups = columns * ((d + zc - 1) / zc);
+    const long long cost = (groups + resident - 1) / resident * (zc + 2);
+    if (cost <= least) {
+      least = cost;
+      best = zc;
+    }
+  }
+  return best;
+}
+
+template <int TM, int CIN, int SRC, int EPI>
+int launch_march(const __bf16* xb, const __bf16* x2b, const __bf16* wb, const Epilogue& E, int n, int d, int h,
+                 int cout, hipStream_t stream) {
+  const long long columns = static_cast<long long>(n) * (h / 4);
+  // With 32 channels on either side, a tile per slice where a CU has fewer than three slices
+  // (32 -> 16 over 24 slices 10.4 us and 11.7 marching, 16 -> 32 over 40 13.4 and 14.8, over 64
+  // 18.7 and 17.2). 16 -> 32 of two added inputs hold one marching workgroup to a CU and are
+  // faster so at any size (over 64 slices 21 and 31 us, over 32 x 96 763 and 917).
+  constexpr bool kAlways = SRC == kSrcAdd && TM == 2;
+  if constexpr (TM * CIN == 32) {
+    if (kAlways || columns * d < 3 * kCus) {
+      hipLaunchKernelGGL((k_conv_fwd_tile<TM, CIN, SRC, EPI, 64>), dim3(static_cast<unsigned int>(columns * d)),
+                         dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, cout);
+      return launch_status();
+    }
+  }
+  // The 2-channel input's planes and weights are half as large: four fit.
+  const int zc = march_slices(columns, d, SRC == kSrcLow8 && TM * CIN == 16 ? 4 : kMarchPerCu<TM, CIN, SRC, EPI>);
+  const dim3 blocks(static_cast<unsigned int>(columns * ((d + zc - 1) / zc)));
+  if constexpr (!kAlways)
+    hipLaunchKernelGGL((k_conv_fwd_march<TM, CIN, SRC, EPI>), blocks, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h,
+                       cout, zc);
+  return launch_status();
+}
+
 template <int SRC, int EPI>
 int conv_fwd(const __bf16* xb, const __bf16* x2b, const __bf16* wb, const Epilogue& E, int n, int d, int h, int w,
              int cin, int cout, hipStream_t stream) {
   if (w == 64 && h % 4 == 0 && (cin == 16 || cin == 32) && (cout == 16 || (cout == 32 && cin == 16))) {
-    // Full-resolution layers: about 2048 workgroups, each over enough slices (6 or more)
-    // to spread the two extra planes it loads.
-    const long long columns = static_cast<long long>(n) * (h / 4);
-    const int zc = static_cast<int>(std::min<long long>(d, std::max<long long>(6, columns * d / 2048)));
-    const dim3 blocks(static_cast<unsigned int>(columns * ((d + zc - 1) / zc)));
-    if (cin == 16 && cout == 32)
-      hipLaunchKernelGGL((k_conv_fwd_march<2, 16, SRC, EPI>), blocks, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, cout, zc);
-    else if (cin == 16)
-      hipLaunchKernelGGL((k_conv_fwd_march<1, 16, SRC, EPI>), blocks, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, cout, zc);
-    else
-      hipLaunchKernelGGL((k_conv_fwd_march<1, 32, SRC, EPI>), blocks, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, cout, zc);
-    return launch_status();
+    // Full-resolution layers.
+    if (cin == 16 && cout == 32) return launch_march<2, 16, SRC, EPI>(xb, x2b, wb, E, n, d, h, cout, stream);
+    if (cin == 16) return launch_march<1, 16, SRC, EPI>(xb, x2b, wb, E, n, d, h, cout, stream);
+    return launch_march<1, 32, SRC, EPI>(xb, x2b, wb, E, n, d, h, cout, stream);
   }
   if (w == 32 && h % 8 == 0 && (cin == 16 || cin == 32 || cin == 64) && cout == 32) {
     // Half-resolution layers: the same staging, 8 rows of 32 per workgroup.

@@ -63,9 +63,11 @@ def test_forward_by_wave_count(dn, shape, cin, cout):  # noqa: F811
     np.testing.assert_array_equal(_np(y_cm), _np(y).reshape(-1, cout).T)
 
 
-# Full-resolution rows: one slice, slices off the marching chunks (6 and 7), several chunks,
-# each channel pair; the other kernels' shapes for the fused steps.
-MARCHED = [((1, 1, 4, 64), 16, 16), ((2, 6, 4, 64), 16, 32), ((1, 7, 8, 64), 32, 16), ((1, 20, 4, 64), 16, 16)]
+# Full-resolution rows of each channel pair: one slice to a workgroup (16 -> 16) or a tile
+# (with 32), and from 3 slices a CU on two slices to a workgroup with a last one of one; the
+# other kernels' shapes for the fused steps.
+MARCHED = [((1, 1, 4, 64), 16, 16), ((2, 6, 4, 64), 16, 32), ((1, 7, 8, 64), 32, 16), ((1, 20, 4, 64), 16, 16),
+           ((11, 7, 44, 64), 16, 16), ((6, 17, 32, 64), 16, 32), ((6, 17, 32, 64), 32, 16)]
 
 
 @pytest.mark.parametrize("shape, cin, cout", MARCHED)
@@ -173,6 +175,36 @@ def test_added_input_equals_a_separate_addition(dn, shape, cin, cout):  # noqa: 
              got_cm.data_ptr(), *args)
     assert torch.equal(got, want) and torch.equal(got_cm, want_cm)
     assert torch.count_nonzero(want.float()) > 0
+
+
+@pytest.mark.parametrize("cin, cout", [(16, 16), (16, 32), (32, 16)])
+@pytest.mark.parametrize("src", (0, 1, 2, 3))
+def test_volumes_of_a_batch_equal_volumes_alone(dn, cin, cout, src):  # noqa: F811
+    """Sixteen volumes of 21 (20 upsampled) slices march 6 to 11 slices to a workgroup, one
+    alone takes a workgroup or tile per slice: the same bits, with and without a skip."""
+    import torch
+
+    n, d, h, w = 16, 20 if src == 1 else 21, 64, 64
+    rng = np.random.default_rng(cin + src)
+    dims = (d // 2, h // 2, w // 2) if src == 1 else (d, h, w)
+    x, x2 = (_dev(_bf(rng.standard_normal((n,) + dims + (cin,), dtype=np.float32))) for _ in range(2))
+    if src == 3:
+        x[..., 8:] = 0
+    wt, bias = _dev(_bf(rng.standard_normal((27, cout, cin)) * 0.1)), _dev(torch.zeros(cout))
+    skip = _dev(_bf(rng.standard_normal((n, d, h, w, cout), dtype=np.float32)))
+    for with_skip in (False, True) if src < 2 else (False,):
+        batch, alone = (torch.zeros_like(skip) for _ in range(2))
+
+        def call(y, first, count):
+            dn._call("hdn_conv3d_fwd_fused", x[first].data_ptr(), x2[first].data_ptr() if src == 2 else None, src,
+                     wt.data_ptr(), bias.data_ptr(), skip[first].data_ptr() if with_skip else None, None, 0, None,
+                     y[first].data_ptr(), None, count, d, h, w, cin, cout, 0.1, None)
+
+        call(batch, 0, n)
+        for i in range(n):
+            call(alone, i, 1)
+        assert torch.equal(batch, alone)
+        assert torch.count_nonzero(batch.float()) > 0
 
 
 @pytest.mark.parametrize("splits, length", [(1, 5), (16, 64), (17, 65), (700, 6912)])
