@@ -881,16 +881,13 @@ __global__ void __launch_bounds__(256, 2) k_conv_wgrad_tile(const __bf16* __rest
               ci0, co0, cin, cout);
 }
 
-// out[i] = sum_s part[s][i] in a fixed order: wave g of a workgroup adds splits g,
-// g + 16, ... of 64 outputs, eight loads in flight, and the 16 waves' sums add in wave
-// order. One thread per output, as before, left 27 waves to walk 2048 splits one load at a
-// time: 470 us for 56 MB; 9 us now for the 21 MB that k_conv_wgrad_tile's splits leave.
-constexpr int kReduceWaves = 16;
-
-__global__ void __launch_bounds__(64 * kReduceWaves) k_reduce_splits(const float* __restrict__ part,
-                                                                     float* __restrict__ out, long long len,
-                                                                     int splits) {
-  __shared__ float sums[kReduceWaves][64];
+// out[i] = sum_s part[s][i] in a fixed order: wave g of the kWaves that share 64 outputs adds
+// splits g, g + kWaves, ..., eight loads in flight, and the waves' sums add in wave order
+// (launch_reduce has the choice of kWaves).
+template <int kWaves>
+__global__ void __launch_bounds__(64 * kWaves) k_reduce_splits(const float* __restrict__ part,
+                                                               float* __restrict__ out, long long len, int splits) {
+  __shared__ float sums[kWaves][64];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   for (long long i0 = static_cast<long long>(blockIdx.x) * 64; i0 < len; i0 += static_cast<long long>(gridDim.x) * 64) {
@@ -898,15 +895,19 @@ __global__ void __launch_bounds__(64 * kReduceWaves) k_reduce_splits(const float
     float s = 0.0f;
     if (i < len) {
 #pragma unroll 8
-      for (int k = wave; k < splits; k += kReduceWaves) s += part[static_cast<long long>(k) * len + i];
+      for (int k = wave; k < splits; k += kWaves) s += part[static_cast<long long>(k) * len + i];
     }
-    sums[wave][lane] = s;
-    __syncthreads();
-    if (wave == 0 && i < len) {
-      for (int g = 1; g < kReduceWaves; ++g) s += sums[g][lane];
-      out[i] = s;
+    if constexpr (kWaves == 1) {
+      if (i < len) out[i] = s;
+    } else {
+      sums[wave][lane] = s;
+      __syncthreads();
+      if (wave == 0 && i < len) {
+        for (int g = 1; g < kWaves; ++g) s += sums[g][lane];
+        out[i] = s;
+      }
+      __syncthreads();
     }
-    __syncthreads();
   }
 }
 
@@ -1328,7 +1329,14 @@ void launch_wgrad(const void* x_cm, const void* dz_cm, float* part, int splits, 
 
 void launch_reduce(const float* part, float* out, long long len, int splits, hipStream_t stream) {
   const unsigned int blocks = static_cast<unsigned int>(std::min<long long>(blocks_for(len, 64), 65535));
-  hipLaunchKernelGGL(k_reduce_splits, dim3(blocks), dim3(64 * kReduceWaves), 0, stream, part, out, len, splits);
+  // Sixteen waves to 64 outputs where there are many splits to walk or too few outputs to fill
+  // the CUs; else one, where sixteen would mostly wait for each other. us with 16 waves and
+  // with one: 13 824 outputs of 768 splits 7.9 and 34.9, 55 296 of 256 9.8 and 14.1; 110 592 of
+  // 96 11.7 and 8.0, 442 368 of 4 11.2 and 7.2, of 48 24.4 and 14.1.
+  if (splits >= 256 || len < 16384)
+    hipLaunchKernelGGL(k_reduce_splits<16>, dim3(blocks), dim3(64 * 16), 0, stream, part, out, len, splits);
+  else
+    hipLaunchKernelGGL(k_reduce_splits<1>, dim3(blocks), dim3(64), 0, stream, part, out, len, splits);
 }
 
 // Device address of `scratch` on each GPU, looked up once per device with that device

@@ -207,7 +207,8 @@ def test_volumes_of_a_batch_equal_volumes_alone(dn, cin, cout, src):  # noqa: F8
         assert torch.count_nonzero(batch.float()) > 0
 
 
-@pytest.mark.parametrize("splits, length", [(1, 5), (16, 64), (17, 65), (700, 6912)])
+@pytest.mark.parametrize("splits, length", [(1, 5), (16, 64), (17, 65), (700, 6912), (1, 16383), (3, 16384), (5, 16385),
+                                            (255, 20_000), (256, 20_000)])
 def test_reduce_splits(dn, splits, length):  # noqa: F811
     import torch
 
