@@ -77,8 +77,9 @@ struct Epilogue {
   int c_in;  // channels of inp
 };
 
-// Kinds of epilogue. The tiled kernels are built per kind and load what it needs (conv_other)
-// before their k-steps, so that the loads run under the MFMAs; kEpiAny decides at run time.
+// Kinds of epilogue. All but k_conv_fwd_deep are built per kind, and the tiled kernels load what
+// it needs (conv_other) before their k-steps, so that the loads run under the MFMAs; kEpiAny
+// decides at run time (in k_conv_fwd that cost 1 to 5 %).
 constexpr int kEpiPlain = 0, kEpiSkip = 1, kEpiPred = 2, kEpiAny = 3;
 
 // What a lane's four sums of channels cb .. cb + 3 at position p are combined with.
@@ -128,7 +129,7 @@ __device__ inline void conv_store(const Epilogue& E, const f32x4& sum, uint2 oth
 // zero padding. One wave computes 16*TM output channels x 64 positions (4 blocks of
 // 16); a workgroup of 4 waves covers 256 consecutive positions (P % 64 == 0). K = 27*cin runs in
 // chunks of 32; each lane's 8 k values lie inside one tap since cin % 8 == 0.
-template <int TM, int SRC>
+template <int TM, int SRC, int EPI>
 __global__ void __launch_bounds__(256) k_conv_fwd(const __bf16* __restrict__ x,
                                                   const __bf16* __restrict__ x2,
                                                   const __bf16* __restrict__ wt, Epilogue E, int n, int d, int h,
@@ -207,7 +208,7 @@ __global__ void __launch_bounds__(256) k_conv_fwd(const __bf16* __restrict__ x,
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
       const long long p = p0 + 16 * nb + col;
-      conv_store<kEpiAny>(E, acc[m][nb], conv_other<kEpiAny>(E, cb, p, cout), cb, p, cout, P);
+      conv_store<EPI>(E, acc[m][nb], conv_other<EPI>(E, cb, p, cout), cb, p, cout, P);
     }
   }
 }
@@ -1283,11 +1284,11 @@ int conv_fwd(const __bf16* xb, const __bf16* x2b, const __bf16* wb, const Epilog
   }
   const dim3 grid(static_cast<unsigned int>((P + 255) / 256), static_cast<unsigned int>(cout / (16 * tm)));
   if (tm == 4)
-    hipLaunchKernelGGL((k_conv_fwd<4, SRC>), grid, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, w, cin, cout);
+    hipLaunchKernelGGL((k_conv_fwd<4, SRC, EPI>), grid, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, w, cin, cout);
   else if (tm == 2)
-    hipLaunchKernelGGL((k_conv_fwd<2, SRC>), grid, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, w, cin, cout);
+    hipLaunchKernelGGL((k_conv_fwd<2, SRC, EPI>), grid, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, w, cin, cout);
   else
-    hipLaunchKernelGGL((k_conv_fwd<1, SRC>), grid, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, w, cin, cout);
+    hipLaunchKernelGGL((k_conv_fwd<1, SRC, EPI>), grid, dim3(256), 0, stream, xb, x2b, wb, E, n, d, h, w, cin, cout);
   return launch_status();
 }
 
