@@ -34,9 +34,9 @@ extern "C" {
  * this is the data gradient of a convolution. */
 int hdn_conv3d_fwd(const void* x, const void* w, const float* bias, void* y_nd, void* y_cm, int n,
                    int d, int h, int w_, int cin, int cout, float slope, void* stream);
-/* The same convolution reading its input through the preceding element-wise step, for
- * inference (the values equal those of the separate calls, so the outputs are
- * identical): src 0 reads x; src 1 (HDN_SRC_UP) reads hdn_up_fwd(x), x having half
+/* The same convolution reading its input through the preceding element-wise step (the
+ * values equal those of the separate calls, so the outputs are identical; the network's
+ * inference uses 1 and 3): src 0 reads x; src 1 (HDN_SRC_UP) reads hdn_up_fwd(x), x having half
  * the output dims d, h, w (all even); src 2 (HDN_SRC_ADD) reads hdn_add(x, x2); src 3
  * (HDN_SRC_LOW8) reads x whose channels beyond the first 8 are zero (the padded network
  * input), skipping them in the reduction. */

@@ -715,7 +715,7 @@ __device__ inline void store_wgrad(const f32x4 (&acc)[27], float4 (*sums)[9][64]
 // Weight-gradient partials: part[s][tap][co][ci] = sum over split s's positions of
 // dz[p][co] x[p + off(tap)][ci]. A workgroup owns one 16x16 (ci, co) block for all 27
 // taps (108 accumulators a lane) and a contiguous range of positions, which its four waves
-// take in chunks of 32; their sums add in wave order (add_waves). For rows that
+// take in chunks of 32; their sums add in wave order (store_wgrad). For rows that
 // k_conv_wgrad_tile does not take.
 __global__ void __launch_bounds__(256) k_conv_wgrad(const __bf16* __restrict__ x_cm,
                                                    const __bf16* __restrict__ dz_cm,
@@ -1182,10 +1182,6 @@ int launch_status() { return hipGetLastError() == hipSuccess ? HDN_OK : HDN_EHIP
 bool shape_ok(int n, int d, int h, int w) { return n > 0 && d > 0 && h > 0 && w > 0; }
 
 }  // namespace
-
-extern "C" {
-
-}  // extern "C"
 
 namespace {
 

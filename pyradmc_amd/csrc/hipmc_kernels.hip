@@ -6,7 +6,7 @@
 //   tables          float4 rows per material: photon (compton, photo, pair, rayleigh),
 //                   electron A (csda, moller, restricted range, radiative),
 //                   electron B (scattering power, log eta, restricted stopping, 0)
-//   GS grid         f32 [n_eta][n_theta2][512]
+//   GS grid         float4 [n_eta - 1][n_theta2 - 1][512]: a cell's four nodes at one u
 //   particles       48-byte records (3 x 16 B) in four ping-pong queues
 //   tallies         int64 quanta [column][scoring voxel]; f64 sums s1, s2 alike
 //
@@ -488,15 +488,16 @@ __device__ inline bool enter_grid(const DevGrid& g, float& x, float& y, float& z
 #endif
 
 // Idle lanes of a wave in the electron round that make a refill worth its pass (of 64;
-// measured on the bench's slab step: 8 and 32 were slower than 16, and the photon
-// round gained nothing from the same rule).
+// measured on the bench's slab step: 8 and 32 were slower than 16).
 constexpr int kRefillIdleLanes = 16;
 
 // Largest table of the kOne builds (tables of one material in LDS).
 constexpr int kTablePoints = 2048;
 
 // Lanes of a wave in the photon round that make a refill, or a pass over the real
-// interactions, worth its instructions.
+// interactions, worth its instructions (1e7 histories on the slab phantom, whole run at 8, 16
+// and 24: 4.94, 4.90 and 4.85 ms; refills deferred without batched interactions gained
+// nothing).
 constexpr int kPhotonBatch = 24;
 
 // Energy bins of the electron queue's sort (a quarter octave each above the cutoff),
@@ -732,8 +733,10 @@ k_photon_round(TransportParams P, Queue qin, unsigned int* head, Queue qe, Queue
 // with what photons make, and its serial tail is shorter (4.86 -> 4.58 ms of a slab run).
 // Slab phantom, 1e7 histories, whole run: 6.54 ms with tables in L2 and Moller
 // interactions in place, 5.46 with both changes, 5.28 with 24-bit voxel indices and
-// unscaled quotients, 4.98 with the GS nodes of a cell in one 16-byte gather. Blocks of
-// 12 waves, one to a CU: 5.0 ms; two to a CU 5.3 (the L1 holds fewer waves' lines).
+// unscaled quotients, 4.98 with the GS nodes of a cell in one 16-byte gather (which moves
+// more memory, the cells are four times the nodes, but waits once). One block of 12 waves to
+// a CU: with the two stacks' 35 KB beside the tables a second has no room, and without the
+// second stack, when two fitted, two took 5.3 ms.
 // More materials or longer tables than fit take the general build.
 constexpr int kMollerSlots = 32;     // stack slots of a wave
 constexpr int kMollerBatch = 16;     // waiting particles that make a batch

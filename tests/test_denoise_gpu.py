@@ -353,9 +353,9 @@ def test_denoised_builder_float32_values_are_the_float64_values_rounded(dn):
 
 @pytest.mark.parametrize("widths", [(16, 32, 64, 128), (16, 16, 32, 32)])
 def test_inference_with_fused_inputs_equals_the_stored_forward(dn, widths):
-    # Inference reads each upsampling and skip addition inside the next convolution
-    # (full-resolution tiled and general kernels alike); the values are those the
-    # separate kernels store, so the head output is the same bit for bit.
+    # Inference reads each upsampling inside the next convolution and makes each skip addition
+    # in the store of the one before it (full-resolution and general kernels alike); the values
+    # are those the separate kernels store, so the head output is the same bit for bit.
     import torch
 
     model = dn.Conv3dDenoiser(widths=widths, seed=11)
