@@ -759,7 +759,8 @@ struct ElectronShared<true> {
   uint32_t fresh[kElectronThreads<true> / 64][kParticleWords - 1][kFreshSlots];
 };
 
-template <bool kFast, bool kOne>
+// kSet: the stacks' slots in use are the caller's (hmc_set_round_stacks).
+template <bool kFast, bool kOne, bool kSet>
 __global__ void __launch_bounds__(kElectronThreads<kOne>) __attribute__((amdgpu_waves_per_eu(kOne ? 3 : HMC_ROUND_WAVES, 8)))
 k_electron_round(TransportParams P, Queue qin, unsigned int* head, Queue qp, Queue qe) {
   __shared__ ElectronShared<kOne> sh;
@@ -801,6 +802,8 @@ k_electron_round(TransportParams P, Queue qin, unsigned int* head, Queue qp, Que
   };
   auto& stack = sh.stack[wave_in_block];
   auto& fresh = sh.fresh[wave_in_block];
+  const unsigned int moller_slots = kSet ? P.moller_slots : static_cast<unsigned int>(kMollerSlots);
+  const unsigned int fresh_slots = kSet ? P.fresh_slots : static_cast<unsigned int>(kFreshSlots);
   unsigned int waiting = 0;  // stack entries of this wave
   unsigned int n_fresh = 0;  // and delta electrons
   bool parked = false;       // this lane's Moller interaction found the stack full
@@ -852,7 +855,7 @@ k_electron_round(TransportParams P, Queue qin, unsigned int* head, Queue qp, Que
         const unsigned long long born = __ballot(1);
         const unsigned int slot =
             n_fresh + static_cast<unsigned int>(__popcll(born & ((1ull << __lane_id()) - 1ull)));
-        if (slot < P.fresh_slots) {
+        if (slot < fresh_slots) {
           fresh[0][slot] = __float_as_uint(x);
           fresh[1][slot] = __float_as_uint(y);
           fresh[2][slot] = __float_as_uint(z);
@@ -871,7 +874,7 @@ k_electron_round(TransportParams P, Queue qin, unsigned int* head, Queue qp, Que
         rotate(ux, uy, uz, cp, mphi + kPi);
         e -= delta;
       }
-      n_fresh = min(n_fresh + made, P.fresh_slots);
+      n_fresh = min(n_fresh + made, fresh_slots);
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     } else if (refill_now) {
       const bool took = n_fresh != 0u;
@@ -1099,7 +1102,7 @@ k_electron_round(TransportParams P, Queue qin, unsigned int* head, Queue qp, Que
       const unsigned int slot =
           waiting + static_cast<unsigned int>(__popcll(met & ((1ull << __lane_id()) - 1ull)));
       if (moller) {
-        if (slot < P.moller_slots) {
+        if (slot < moller_slots) {
           stack[0][slot] = __float_as_uint(x);
           stack[1][slot] = __float_as_uint(y);
           stack[2][slot] = __float_as_uint(z);
@@ -1117,7 +1120,7 @@ k_electron_round(TransportParams P, Queue qin, unsigned int* head, Queue qp, Que
           parked = true;
         }
       }
-      waiting = min(waiting + static_cast<unsigned int>(__popcll(met)), P.moller_slots);
+      waiting = min(waiting + static_cast<unsigned int>(__popcll(met)), moller_slots);
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     }
   }
@@ -3189,18 +3192,17 @@ static int enqueue_round_group(hmc_ctx* ctx, const TransportParams& P, unsigned 
       head_e = heads + pa;
     }
     if (ev) HMC_HIP(ctx, hipEventRecord(ev[2], ctx->stream));
-    if (one && fast)
-      hipLaunchKernelGGL((k_electron_round<true, true>), dim3(round_blocks), dim3(kElectronThreads<true>), 0,
-                         ctx->stream, P, qin_e, head_e, qb_p, qb_e);
+    const bool set = P.moller_slots != kMollerSlots || P.fresh_slots != kFreshSlots;
+    auto* electrons = &k_electron_round<false, false, false>;
+    if (set)
+      electrons = one ? (fast ? &k_electron_round<true, true, true> : &k_electron_round<false, true, true>)
+                      : (fast ? &k_electron_round<true, false, true> : &k_electron_round<false, false, true>);
     else if (one)
-      hipLaunchKernelGGL((k_electron_round<false, true>), dim3(round_blocks), dim3(kElectronThreads<true>), 0,
-                         ctx->stream, P, qin_e, head_e, qb_p, qb_e);
+      electrons = fast ? &k_electron_round<true, true, false> : &k_electron_round<false, true, false>;
     else if (fast)
-      hipLaunchKernelGGL((k_electron_round<true, false>), dim3(round_blocks), dim3(kElectronThreads<false>), 0,
-                         ctx->stream, P, qin_e, head_e, qb_p, qb_e);
-    else
-      hipLaunchKernelGGL((k_electron_round<false, false>), dim3(round_blocks), dim3(kElectronThreads<false>), 0,
-                         ctx->stream, P, qin_e, head_e, qb_p, qb_e);
+      electrons = &k_electron_round<true, false, false>;
+    hipLaunchKernelGGL(electrons, dim3(round_blocks), dim3(one ? kElectronThreads<true> : kElectronThreads<false>), 0,
+                       ctx->stream, P, qin_e, head_e, qb_p, qb_e);
     HMC_HIP(ctx, hipGetLastError());
     if (ev) HMC_HIP(ctx, hipEventRecord(ev[3], ctx->stream));
     hipLaunchKernelGGL(k_reset_consumed, dim3(1), dim3(64), 0, ctx->stream, counts, heads, pa, ea, cap,
