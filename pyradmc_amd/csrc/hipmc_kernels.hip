@@ -1801,8 +1801,7 @@ struct hmc_ctx {
   DevTables t{};
   std::vector<void*> table_buffers;
   bool has_tables = false;
-  float* d_gs = nullptr;         // nodes as given
-  float4* d_gs_cells = nullptr;  // DevTables::gs
+  float4* d_gs_cells = nullptr;  // DevTables::gs, then the nodes as given
   bool has_gs = false;
 
   // source
@@ -2040,7 +2039,7 @@ void hmc_destroy(hmc_ctx* ctx) {
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
   void* ptrs[] = {ctx->d_density,      ctx->d_material,    ctx->d_mass,       ctx->d_edep,
-                  ctx->d_s1,           ctx->d_s2,          ctx->d_nhist,      ctx->d_gs,
+                  ctx->d_s1,           ctx->d_s2,          ctx->d_nhist,
                   ctx->d_gs_cells,
                   ctx->d_edges,        ctx->d_cdf,         ctx->d_beamlet,    ctx->d_up_particle,
                   ctx->d_up,           ctx->d_q[0],        ctx->d_q[1],       ctx->d_q[2],
@@ -2262,10 +2261,10 @@ int hmc_set_gs(hmc_ctx* ctx, const float* values, int n_eta, int n_theta2, int n
   ctx->has_gs = false;  // a failure below can leave the cells freed
   const size_t count = static_cast<size_t>(n_eta) * n_theta2 * n_u;
   const long long cells = static_cast<long long>(n_eta - 1) * (n_theta2 - 1) * n_u;
-  int rc = upload(ctx, &ctx->d_gs, values, count);
-  if (rc == HMC_OK) rc = dev_alloc(ctx, &ctx->d_gs_cells, static_cast<size_t>(cells));
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_gs_cells, dim3(blocks_for(cells, 256, 8192)), dim3(256), 0, ctx->stream, ctx->d_gs, n_theta2,
+  if (int rc = dev_alloc(ctx, &ctx->d_gs_cells, static_cast<size_t>(cells) + (count + 3) / 4)) return rc;
+  float* nodes = reinterpret_cast<float*>(ctx->d_gs_cells + cells);
+  HMC_HIP(ctx, hipMemcpy(nodes, values, count * sizeof(float), hipMemcpyHostToDevice));
+  hipLaunchKernelGGL(k_gs_cells, dim3(blocks_for(cells, 256, 8192)), dim3(256), 0, ctx->stream, nodes, n_theta2,
                      n_u, cells, ctx->d_gs_cells);
   HMC_HIP(ctx, hipGetLastError());
   ctx->t.gs = ctx->d_gs_cells;
